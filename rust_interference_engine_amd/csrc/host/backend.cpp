@@ -790,12 +790,11 @@ bool HipBackend::ffn_moe(const DevLayer &L, int n, bool direct) {
 }
 
 // The device-grouped prompt path needs the int8 MFMA GEMMs for the experts' matrices:
-// a gated pair (Q4_0, Q8_0 or Q4_K) and a down projection with a GEMM.
+// a gated pair and a down projection of types with a GEMM.
 bool HipBackend::moe_grouped_ok(const DevLayer &L) const {
     const size_t E = m_.cfg.n_embd, ff = L.ff;
     const int gt = L.gate.ty;
-    return L.gate.ty == L.up.ty && (gt == T_Q4_0 || gt == T_Q8_0 || gt == T_Q4_K) && gemm_supported(gt, E) &&
-           gemm_supported(L.down.ty, ff) && d_moe_off_ != nullptr;
+    return L.gate.ty == L.up.ty && gemm_supported(gt, E) && gemm_supported(L.down.ty, ff) && d_moe_off_ != nullptr;
 }
 
 void HipBackend::forward(const uint32_t *tokens, size_t n, size_t pos, bool all_logits, float *logits, size_t logits_len) {

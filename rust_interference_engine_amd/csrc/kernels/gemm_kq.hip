@@ -1,5 +1,6 @@
-// gemm_kq.hip — prompt-batch matmul of Q4_K weights × Q8_K activations on CDNA4
-// int8 MFMA, the batched counterpart of the Q4_K block dot (the x86 prefill tiles
+// gemm_kq.hip — prompt-batch matmul of K-quant weights × Q8_K activations on CDNA4
+// int8 MFMA: Q4_K and Q5_K (one kernel) and Q6_K.  Q4_K is described first:
+// the batched counterpart of the Q4_K block dot (the x86 prefill tiles
 // of kernels/mod.rs:238-296 cover Q4_K; kernels/avx2.rs dot_q4_k 78-107).
 //
 // Per 256-value superblock b, for activation row t and weight row r:
@@ -20,12 +21,22 @@
 // 16·(l/32)..+16; tokens are permuted onto the A rows so that lane l's 16
 // results are the 16 consecutive tokens 16·(l/32) + v.
 //
+// Q5_K weights (quant/reference.rs:321-350) differ in the code alone: the fifth bits
+// come from the superblock's 32 qh bytes.  The stage store joins nibble and bit into
+// one byte per code (two ALU operations per four codes, once per workgroup), so the
+// multiply loop reads its B operand without the nibble shifts of Q4_K, for 64 more LDS
+// bytes per row.  Bound like Q4_K by the int32 scale multiply-adds between the MFMAs.
+// A 421-token prompt through two layers of hidden 3072 (Q5_K, V and one down
+// projection Q6_K) takes 905 µs, against 7439 µs with its Q5_K weights in the batched
+// GEMV, which reads and unpacks every weight once per 4 tokens.
+//
 // Q6_K weights × Q8_K activations (kernels/avx2.rs dot_q6_k 109-151): per
 // superblock y += (f16(d_r)·d_t)·Σ_k sc_k·Σ_{16} (q6−32)·q8.  The codes are
 // unpacked once per stage into int8 q6−32 in LDS (four at a time); each
 // 16-value sub-block dot is one v_mfma_i32_32x32x16_i8 (exact), Σ_k sc_k·D_k
 // accumulates in int32 with 24-bit multiply-adds (|.| < 2^27), and the
-// superblock's float product is the rank-1 f32 MFMA of d_t and d_r.
+// superblock's float product is the rank-1 f32 MFMA of d_t and d_r.  The gated form
+// stages gate and up rows beside each other (two weight tiles per activation tile).
 #include "../common.hpp"
 #include "../device.hpp"
 #include "../kernels.hpp"
@@ -91,11 +102,15 @@ __device__ __forceinline__ TileRows tile_rows(const KqP &p, int tg) {
 __device__ __forceinline__ int act_row(const KqP &p, int r) { return p.grouped && p.grp.amap ? p.grp.amap[r] : r; }
 __device__ __forceinline__ int out_row(const KqP &p, int r) { return p.grouped && p.grp.omap ? p.grp.omap[r] : r; }
 constexpr int KA_ST = 128 + 16;  // activation bytes per token in LDS (one half superblock, padded)
-constexpr int KW_ST = 64 + 16;   // weight nibble bytes per row in LDS (one half superblock, padded)
+// weight code bytes per row in LDS (one half superblock, padded): Q4_K keeps its nibble
+// pairs, Q5_K one byte per code
+template <int TY> constexpr int kw_st() { return (TY == T_Q5_K ? 128 : 64) + 16; }
+template <int TY> constexpr int kq_block() { return TY == T_Q5_K ? 176 : 144; }  // superblock bytes
+template <int TY> constexpr int kq_qs() { return TY == T_Q5_K ? 48 : 16; }       // offset of its nibbles
 
 // BN = 32 keeps the 6-bit scales and mins as bytes, so that two 128-row stages of
 // the gated pair fit two workgroups in a CU's LDS.
-template <bool GLU, int BN = KQ_BN>
+template <int TY, bool GLU, int BN = KQ_BN>
 struct __align__(16) KqStage {
     static constexpr int NW = GLU ? 2 : 1, BM = kq_bm<BN>();
     using ScT = std::conditional_t<BN == 64, int, uint8_t>;
@@ -103,28 +118,30 @@ struct __align__(16) KqStage {
     int8_t a[BN * KA_ST];
     float da[BN];
     float bs[BN * 8];              // the superblock's 32-value activation sums (both halves hold all 8)
-    uint8_t wq[NW][BM * KW_ST];
+    uint8_t wq[NW][BM * kw_st<TY>()];
     float wd[NW][BM], wdm[NW][BM];
     ScT wsc[NW][BM * 8];           // 6-bit scales of the 8 sub-blocks
     MnT wm[NW][BM * 8];            // 6-bit mins
 };
 
-template <bool GLU, int BN = KQ_BN>
+template <int TY, bool GLU, int BN = KQ_BN>
 struct KqRegs {
     static constexpr int NA = BN == 64 ? 2 : 1, NQ = (BN == 32 && GLU) ? 4 : 2;
     v4i a[NA];        // 32 (BN 64) or 16 (BN 32) activation bytes of the thread's token
     float da;
     v4i bs[2];        // the token's 16 bsums (int16)
     v4i wq[NQ];       // 32 nibble bytes of the thread's row (64, both units, in the 32-token gated form)
+    v4i qh[TY == T_Q5_K ? 2 : 1];  // Q5_K: the superblock's 32 bytes of fifth bits
     v4i hdr;          // d, dmin, scales[12]
 };
 
 // stage loads for half hs of superblock sb
 // tokA: the activation row of the thread's token (tid/4, or tid/8 for BN 32); tokD: of
 // token tid (tid < BN); woff: the expert's byte offset in a grouped launch
-template <bool GLU, int BN = KQ_BN>
+template <int TY, bool GLU, int BN = KQ_BN>
 __device__ __forceinline__ void kq_load(const KqP &p, int sg, int row0, int tokA, int tokD, size_t woff, int sb, int hs, int tid,
-                                        KqRegs<GLU, BN> &R) {
+                                        KqRegs<TY, GLU, BN> &R) {
+    static_assert(TY == T_Q4_K || BN == 64, "32-token tiles serve Q4_K");
     const int K = p.K, nsb = K >> 8;
     if constexpr (BN == 64) {
         const v4i *src = (const v4i *)(p.qs + (size_t)tokA * K + 256 * sb + 128 * hs + 32 * (tid & 3));
@@ -151,16 +168,21 @@ __device__ __forceinline__ void kq_load(const KqP &p, int sg, int row0, int tokA
         const int nw = (GLU && BN == 64) ? (tid >> 7) : 0, idx = BN == 64 ? (tid & 127) : tid, u = idx & 1;
         const int s = GLU ? nw : sg;
         const int row = min(row0 + (idx >> 1), p.rows[GLU ? 0 : sg] - 1);
-        const uint8_t *blk = p.w[s] + woff + (size_t)row * p.rb[s] + 144 * (size_t)sb;
-        const v4i *q = (const v4i *)(blk + 16 + 64 * hs + 32 * u);
+        const uint8_t *blk = p.w[s] + woff + (size_t)row * p.rb[s] + kq_block<TY>() * (size_t)sb;
+        const v4i *q = (const v4i *)(blk + kq_qs<TY>() + 64 * hs + 32 * u);
         R.wq[0] = wload(q);
         R.wq[1] = wload(q + 1);
+        if constexpr (TY == T_Q5_K) {
+            R.qh[0] = wload((const v4i *)(blk + 16));
+            R.qh[1] = wload((const v4i *)(blk + 32));
+        }
         R.hdr = wload((const v4i *)blk);
     }
 }
 
-template <bool GLU, int BN = KQ_BN>
-__device__ __forceinline__ void kq_store(KqStage<GLU, BN> &S, int tid, const KqRegs<GLU, BN> &R) {
+// hs: the half that R holds (Q5_K: which of its fifth-bit planes)
+template <int TY, bool GLU, int BN = KQ_BN>
+__device__ __forceinline__ void kq_store(KqStage<TY, GLU, BN> &S, int tid, int hs, const KqRegs<TY, GLU, BN> &R) {
     if constexpr (BN == 64) {
         v4i *dst = (v4i *)(S.a + (tid >> 2) * KA_ST + 32 * (tid & 3));
         dst[0] = R.a[0];
@@ -182,7 +204,7 @@ __device__ __forceinline__ void kq_store(KqStage<GLU, BN> &S, int tid, const KqR
             nw = tid >> 7;
             row = tid & 127;
             u = 0;
-            v4i *dst = (v4i *)(S.wq[nw] + row * KW_ST);
+            v4i *dst = (v4i *)(S.wq[nw] + row * kw_st<TY>());
 #pragma unroll
             for (int i = 0; i < 4; i++) dst[i] = R.wq[i];
         } else {
@@ -190,9 +212,29 @@ __device__ __forceinline__ void kq_store(KqStage<GLU, BN> &S, int tid, const KqR
             const int idx = BN == 64 ? (tid & 127) : tid;
             row = idx >> 1;
             u = idx & 1;
-            v4i *dst = (v4i *)(S.wq[nw] + row * KW_ST + 32 * u);
-            dst[0] = R.wq[0];
-            dst[1] = R.wq[1];
+            if constexpr (TY == T_Q5_K) {
+                // the unit's two sub-blocks as bytes: nibble + 16·(bit 2(2hs + u) of qh, and
+                // the next bit for the high nibbles): quant/reference.rs:321-350
+                const int b0 = 4 * hs + 2 * u;
+                v4i lo[2], hi[2];
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int c = 0; c < 4; c++) {
+                        const uint32_t q = (uint32_t)R.wq[i][c], b = (uint32_t)R.qh[i][c] >> b0;
+                        lo[i][c] = (int)((q & 0x0F0F0F0Fu) | ((b & 0x01010101u) << 4));
+                        hi[i][c] = (int)(((q >> 4) & 0x0F0F0F0Fu) | ((b & 0x02020202u) << 3));
+                    }
+                v4i *dst = (v4i *)(S.wq[nw] + row * kw_st<TY>() + 64 * u);
+                dst[0] = lo[0];
+                dst[1] = lo[1];
+                dst[2] = hi[0];
+                dst[3] = hi[1];
+            } else {
+                v4i *dst = (v4i *)(S.wq[nw] + row * kw_st<TY>() + 32 * u);
+                dst[0] = R.wq[0];
+                dst[1] = R.wq[1];
+            }
         }
         if (u == 0) {
             const uint32_t h0 = (uint32_t)R.hdr[0], h1 = (uint32_t)R.hdr[1], h2 = (uint32_t)R.hdr[2], h3 = (uint32_t)R.hdr[3];
@@ -202,8 +244,8 @@ __device__ __forceinline__ void kq_store(KqStage<GLU, BN> &S, int tid, const KqR
             for (int j = 0; j < 8; j++) {
                 int sc, mn;
                 q4k_scale_min(h1, h2, h3, j, sc, mn);  // get_scale_min_k4 (quant/reference.rs:8-16)
-                S.wsc[nw][row * 8 + j] = (typename KqStage<GLU, BN>::ScT)sc;
-                S.wm[nw][row * 8 + j] = (typename KqStage<GLU, BN>::MnT)mn;
+                S.wsc[nw][row * 8 + j] = (typename KqStage<TY, GLU, BN>::ScT)sc;
+                S.wm[nw][row * 8 + j] = (typename KqStage<TY, GLU, BN>::MnT)mn;
             }
         }
     }
@@ -216,10 +258,10 @@ __device__ __forceinline__ void kq_store(KqStage<GLU, BN> &S, int tid, const KqR
 // result only for instructions it generates itself.
 __device__ __forceinline__ int mad24(int a, int b, int c) { return c + __mul24(a, b); }
 
-template <bool GLU, int BN = KQ_BN>
-__global__ __launch_bounds__(256) void gemm_q4k_kernel(KqP p) {
+template <int TY, bool GLU, int BN = KQ_BN>
+__global__ __launch_bounds__(256) void gemm_q45k_kernel(KqP p) {
     constexpr int NW = GLU ? 2 : 1, BM = kq_bm<BN>(), WC = BN / 32;  // waves along the tokens
-    __shared__ KqStage<GLU, BN> st[2];
+    __shared__ KqStage<TY, GLU, BN> st[2];
     const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
     const int wr = wv / WC, wc = wv % WC;
     // workgroups of one row group share an XCD (id mod 8); the K splits of one tile
@@ -259,25 +301,30 @@ __global__ __launch_bounds__(256) void gemm_q4k_kernel(KqP p) {
     const int nsb = p.K >> 8;
     const int sb0 = KSPLIT ? ksi * nsb / p.ks : 0;
     const int n_stages = KSPLIT ? ((ksi + 1) * nsb / p.ks - sb0) * 2 : nsb * 2;
-    KqRegs<GLU, BN> R;
-    kq_load<GLU, BN>(p, sg, row0, tokA, tokD, woff, sb0, 0, tid, R);
-    kq_store<GLU, BN>(st[0], tid, R);
+    KqRegs<TY, GLU, BN> R;
+    kq_load<TY, GLU, BN>(p, sg, row0, tokA, tokD, woff, sb0, 0, tid, R);
+    kq_store<TY, GLU, BN>(st[0], tid, 0, R);
     __syncthreads();
     for (int s = 0; s < n_stages; s++) {
         const int hs = s & 1;
-        if (s + 1 < n_stages) kq_load<GLU, BN>(p, sg, row0, tokA, tokD, woff, sb0 + ((s + 1) >> 1), (s + 1) & 1, tid, R);
-        const KqStage<GLU, BN> &S = st[s & 1];
+        if (s + 1 < n_stages) kq_load<TY, GLU, BN>(p, sg, row0, tokA, tokD, woff, sb0 + ((s + 1) >> 1), (s + 1) & 1, tid, R);
+        const KqStage<TY, GLU, BN> &S = st[s & 1];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const v4i av = *(const v4i *)(S.a + arow * KA_ST + 32 * j + 16 * h);
 #pragma unroll
             for (int a = 0; a < NW; a++) {
-                const uint4 q = *(const uint4 *)(S.wq[a] + wrow * KW_ST + 32 * (j >> 1) + 16 * h);
-                const uint32_t sh = 4u * (uint32_t)(j & 1);
-                const v4i bw = {(int)((q.x >> sh) & 0x0F0F0F0Fu), (int)((q.y >> sh) & 0x0F0F0F0Fu), (int)((q.z >> sh) & 0x0F0F0F0Fu),
-                                (int)((q.w >> sh) & 0x0F0F0F0Fu)};
+                v4i bw;
+                if constexpr (TY == T_Q5_K) {
+                    bw = *(const v4i *)(S.wq[a] + wrow * kw_st<TY>() + 32 * j + 16 * h);
+                } else {
+                    const uint4 q = *(const uint4 *)(S.wq[a] + wrow * kw_st<TY>() + 32 * (j >> 1) + 16 * h);
+                    const uint32_t sh = 4u * (uint32_t)(j & 1);
+                    bw = v4i{(int)((q.x >> sh) & 0x0F0F0F0Fu), (int)((q.y >> sh) & 0x0F0F0F0Fu), (int)((q.z >> sh) & 0x0F0F0F0Fu),
+                             (int)((q.w >> sh) & 0x0F0F0F0Fu)};
+                }
                 const v16i I = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, bw, zi, 0, 0, 0);
-                const int sc = (int)S.wsc[a][wrow * 8 + 4 * hs + j];  // |sc| < 64, |I| < 2^16
+                const int sc = (int)S.wsc[a][wrow * 8 + 4 * hs + j];  // |sc| < 64, |I| < 2^17
 #pragma unroll
                 for (int v = 0; v < 16; v++) s1[a][v] = mad24(sc, I[v], s1[a][v]);
             }
@@ -311,7 +358,7 @@ __global__ __launch_bounds__(256) void gemm_q4k_kernel(KqP p) {
                 }
             }
         }
-        if (s + 1 < n_stages) kq_store<GLU, BN>(st[(s + 1) & 1], tid, R);
+        if (s + 1 < n_stages) kq_store<TY, GLU, BN>(st[(s + 1) & 1], tid, (s + 1) & 1, R);
         __syncthreads();
     }
     // ---- epilogue: lane holds weight row row0 + wrow for tokens t0 + wc·32 + 16h + v ----
@@ -337,21 +384,28 @@ __global__ __launch_bounds__(256) void gemm_q4k_kernel(KqP p) {
 // ---- Q6_K ----------------------------------------------------------------
 constexpr int K6_ST = 128 + 16;  // weight code bytes per row in LDS (one half superblock, padded)
 
+template <bool GLU>
 struct __align__(16) K6Stage {
+    static constexpr int NW = GLU ? 2 : 1;
     int8_t a[KQ_BN * KA_ST];
     float da[KQ_BN];
-    int8_t wq[KQ_BM * K6_ST];  // q6 − 32 of the half, in value order
-    float wd[KQ_BM];
-    int wsc[KQ_BM * 8];        // the half's 8 signed sub-block scales
+    int8_t wq[NW][KQ_BM * K6_ST];  // q6 − 32 of the half, in value order
+    float wd[NW][KQ_BM];
+    int wsc[NW][KQ_BM * 8];        // the half's 8 signed sub-block scales
 };
 
-struct K6Regs {
-    v4i a[2];
-    float da;
+struct K6W {  // one weight row's part of a half superblock
     uint32_t lo[3], hi[3], qh[3];  // 8 bytes each from a 2-byte aligned address (+1 dword)
     uint32_t sc[3];                // the half's 8 scale bytes
     uint32_t d;
     uint32_t sh_l, sh_h, sh_q, sh_s;
+};
+
+template <bool GLU>
+struct K6Regs {
+    v4i a[2];
+    float da;
+    K6W w[GLU ? 2 : 1];
 };
 
 // 3 dwords from the dword-aligned address at or below p; sh = p's offset in the first
@@ -364,8 +418,9 @@ __device__ __forceinline__ void ld3_a2(const uint8_t *p, uint32_t (&w)[3], uint3
 }
 
 // thread → (row tid/4, part tid%4): values l + 32i of the half, l in 8·part..+8, i = 0..3
+template <bool GLU>
 __device__ __forceinline__ void k6_load(const KqP &p, int sg, int row0, int tokA, int tokD, size_t woff, int sb, int hs, int tid,
-                                        K6Regs &R) {
+                                        K6Regs<GLU> &R) {
     const int K = p.K, nsb = K >> 8;
     {
         const v4i *src = (const v4i *)(p.qs + (size_t)tokA * K + 256 * sb + 128 * hs + 32 * (tid & 3));
@@ -373,18 +428,24 @@ __device__ __forceinline__ void k6_load(const KqP &p, int sg, int row0, int tokA
         R.a[1] = src[1];
     }
     if (tid < KQ_BN) R.da = p.d[(size_t)tokD * nsb + sb];
-    const int row = min(row0 + (tid >> 2), p.rows[sg] - 1), part = tid & 3;
-    const uint8_t *blk = p.w[sg] + woff + (size_t)row * p.rb[sg] + 210 * (size_t)sb;
-    ld3_a2(blk + 64 * hs + 8 * part, R.lo, R.sh_l);
-    ld3_a2(blk + 64 * hs + 32 + 8 * part, R.hi, R.sh_h);
-    ld3_a2(blk + 128 + 32 * hs + 8 * part, R.qh, R.sh_q);
-    if (part == 0) {
-        ld3_a2(blk + 192 + 8 * hs, R.sc, R.sh_s);
-        R.d = wload((const uint16_t *)(blk + 208));
+    const int row = min(row0 + (tid >> 2), p.rows[GLU ? 0 : sg] - 1), part = tid & 3;
+#pragma unroll
+    for (int a = 0; a < (GLU ? 2 : 1); a++) {
+        const int s = GLU ? a : sg;
+        K6W &w = R.w[a];
+        const uint8_t *blk = p.w[s] + woff + (size_t)row * p.rb[s] + 210 * (size_t)sb;
+        ld3_a2(blk + 64 * hs + 8 * part, w.lo, w.sh_l);
+        ld3_a2(blk + 64 * hs + 32 + 8 * part, w.hi, w.sh_h);
+        ld3_a2(blk + 128 + 32 * hs + 8 * part, w.qh, w.sh_q);
+        if (part == 0) {
+            ld3_a2(blk + 192 + 8 * hs, w.sc, w.sh_s);
+            w.d = wload((const uint16_t *)(blk + 208));
+        }
     }
 }
 
-__device__ __forceinline__ void k6_store(K6Stage &S, int tid, const K6Regs &R) {
+template <bool GLU>
+__device__ __forceinline__ void k6_store(K6Stage<GLU> &S, int tid, const K6Regs<GLU> &R) {
     {
         v4i *dst = (v4i *)(S.a + (tid >> 2) * KA_ST + 32 * (tid & 3));
         dst[0] = R.a[0];
@@ -392,37 +453,43 @@ __device__ __forceinline__ void k6_store(K6Stage &S, int tid, const K6Regs &R) {
     }
     if (tid < KQ_BN) S.da[tid] = R.da;
     const int row = tid >> 2, part = tid & 3;
-    const uint32_t lo[2] = {__builtin_amdgcn_alignbyte(R.lo[1], R.lo[0], R.sh_l), __builtin_amdgcn_alignbyte(R.lo[2], R.lo[1], R.sh_l)};
-    const uint32_t hi[2] = {__builtin_amdgcn_alignbyte(R.hi[1], R.hi[0], R.sh_h), __builtin_amdgcn_alignbyte(R.hi[2], R.hi[1], R.sh_h)};
-    const uint32_t qh[2] = {__builtin_amdgcn_alignbyte(R.qh[1], R.qh[0], R.sh_q), __builtin_amdgcn_alignbyte(R.qh[2], R.qh[1], R.sh_q)};
-    // value l + 32i: low nibble of ql[l] (i = 0), ql[l + 32] (i = 1), high nibbles (i = 2, 3);
-    // bits 2i, 2i+1 of qh[l] on top (quant/reference.rs:190-212).  Four codes per dword:
-    // (q | 0x80) − 32, then bit 7 flipped back, is the int8 q − 32 without cross-byte borrows.
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint32_t *src = (i & 1) ? hi : lo;
-        const int sl = 4 * (i >> 1), sq = 2 * i;
-        uint32_t w[2];
+    for (int a = 0; a < (GLU ? 2 : 1); a++) {
+        const K6W &R6 = R.w[a];
+        const uint32_t lo[2] = {__builtin_amdgcn_alignbyte(R6.lo[1], R6.lo[0], R6.sh_l), __builtin_amdgcn_alignbyte(R6.lo[2], R6.lo[1], R6.sh_l)};
+        const uint32_t hi[2] = {__builtin_amdgcn_alignbyte(R6.hi[1], R6.hi[0], R6.sh_h), __builtin_amdgcn_alignbyte(R6.hi[2], R6.hi[1], R6.sh_h)};
+        const uint32_t qh[2] = {__builtin_amdgcn_alignbyte(R6.qh[1], R6.qh[0], R6.sh_q), __builtin_amdgcn_alignbyte(R6.qh[2], R6.qh[1], R6.sh_q)};
+        // value l + 32i: low nibble of ql[l] (i = 0), ql[l + 32] (i = 1), high nibbles (i = 2, 3);
+        // bits 2i, 2i+1 of qh[l] on top (quant/reference.rs:190-212).  Four codes per dword:
+        // (q | 0x80) − 32, then bit 7 flipped back, is the int8 q − 32 without cross-byte borrows.
 #pragma unroll
-        for (int k = 0; k < 2; k++) {
-            const uint32_t q = ((src[k] >> sl) & 0x0F0F0F0Fu) | (((qh[k] >> sq) & 0x03030303u) << 4);
-            w[k] = ((q | 0x80808080u) - 0x20202020u) ^ 0x80808080u;
+        for (int i = 0; i < 4; i++) {
+            const uint32_t *src = (i & 1) ? hi : lo;
+            const int sl = 4 * (i >> 1), sq = 2 * i;
+            uint32_t w[2];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const uint32_t q = ((src[k] >> sl) & 0x0F0F0F0Fu) | (((qh[k] >> sq) & 0x03030303u) << 4);
+                w[k] = ((q | 0x80808080u) - 0x20202020u) ^ 0x80808080u;
+            }
+            *(uint2 *)(S.wq[a] + row * K6_ST + 32 * i + 8 * part) = make_uint2(w[0], w[1]);
         }
-        *(uint2 *)(S.wq + row * K6_ST + 32 * i + 8 * part) = make_uint2(w[0], w[1]);
-    }
-    if (part == 0) {
-        const uint32_t s0 = __builtin_amdgcn_alignbyte(R.sc[1], R.sc[0], R.sh_s), s1 = __builtin_amdgcn_alignbyte(R.sc[2], R.sc[1], R.sh_s);
+        if (part == 0) {
+            const uint32_t s0 = __builtin_amdgcn_alignbyte(R6.sc[1], R6.sc[0], R6.sh_s), s1 = __builtin_amdgcn_alignbyte(R6.sc[2], R6.sc[1], R6.sh_s);
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            S.wsc[row * 8 + k] = (int)(int8_t)(s0 >> (8 * k));
-            S.wsc[row * 8 + 4 + k] = (int)(int8_t)(s1 >> (8 * k));
+            for (int k = 0; k < 4; k++) {
+                S.wsc[a][row * 8 + k] = (int)(int8_t)(s0 >> (8 * k));
+                S.wsc[a][row * 8 + 4 + k] = (int)(int8_t)(s1 >> (8 * k));
+            }
+            S.wd[a][row] = h2f(R6.d);
         }
-        S.wd[row] = h2f(R.d);
     }
 }
 
+template <bool GLU>
 __global__ __launch_bounds__(256) void gemm_q6k_kernel(KqP p) {
-    __shared__ K6Stage st[2];
+    constexpr int NW = GLU ? 2 : 1;
+    __shared__ K6Stage<GLU> st[2];
     const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
     const int wr = wv >> 1, wc = wv & 1;
     // workgroups of one row group share an XCD (id mod 8); the K splits of one tile
@@ -433,7 +500,7 @@ __global__ __launch_bounds__(256) void gemm_q6k_kernel(KqP p) {
     const int tg = u % p.n_tg;
     const int rg = (u / p.n_tg) * 8 + xcd;
     if (rg >= p.n_rg) return;  // whole workgroup: uniform
-    const int sg = (p.nseg > 1 && rg >= p.rg_end[0]) ? ((p.nseg > 2 && rg >= p.rg_end[1]) ? 2 : 1) : 0;
+    const int sg = (!GLU && p.nseg > 1 && rg >= p.rg_end[0]) ? ((p.nseg > 2 && rg >= p.rg_end[1]) ? 2 : 1) : 0;
     const int row0 = (rg - (sg ? p.rg_end[sg - 1] : 0)) * KQ_BM;
     const TileRows tr = tile_rows(p, tg);
     if (tr.e < 0) return;  // whole workgroup: uniform
@@ -446,43 +513,51 @@ __global__ __launch_bounds__(256) void gemm_q6k_kernel(KqP p) {
     const int arow = wc * 32 + tok_m;
     const v16i zi = {0};
     const v16f zf = {0};
-    float acc[16];
-    int s1[16];
+    float acc[NW][16];
+    int s1[NW][16];
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-        acc[v] = 0.0f;
-        s1[v] = 0;
-    }
+    for (int a = 0; a < NW; a++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            acc[a][v] = 0.0f;
+            s1[a][v] = 0;
+        }
     // this workgroup's superblocks [sb0, sb0 + n_stages / 2) (its K split)
     const int nsb = p.K >> 8;
     const int sb0 = ksi * nsb / p.ks;
     const int n_stages = ((ksi + 1) * nsb / p.ks - sb0) * 2;
-    K6Regs R;
-    k6_load(p, sg, row0, tokA, tokD, woff, sb0, 0, tid, R);
-    k6_store(st[0], tid, R);
+    K6Regs<GLU> R;
+    k6_load<GLU>(p, sg, row0, tokA, tokD, woff, sb0, 0, tid, R);
+    k6_store<GLU>(st[0], tid, R);
     __syncthreads();
     for (int s = 0; s < n_stages; s++) {
         const int hs = s & 1;
-        if (s + 1 < n_stages) k6_load(p, sg, row0, tokA, tokD, woff, sb0 + ((s + 1) >> 1), (s + 1) & 1, tid, R);
-        const K6Stage &S = st[s & 1];
+        if (s + 1 < n_stages) k6_load<GLU>(p, sg, row0, tokA, tokD, woff, sb0 + ((s + 1) >> 1), (s + 1) & 1, tid, R);
+        const K6Stage<GLU> &S = st[s & 1];
 #pragma unroll
         for (int k = 0; k < 8; k++) {  // 16-value sub-blocks of the half
             const long av = *(const long *)(S.a + arow * KA_ST + 16 * k + 8 * h);
-            const long bw = *(const long *)(S.wq + wrow * K6_ST + 16 * k + 8 * h);
-            const v16i D = __builtin_amdgcn_mfma_i32_32x32x16_i8(av, bw, zi, 0, 0, 0);
-            const int sc = S.wsc[wrow * 8 + k];
 #pragma unroll
-            for (int v = 0; v < 16; v++) s1[v] = mad24(sc, D[v], s1[v]);
-        }
-        if (hs == 1) {  // end of the superblock: (d_r·d_t)·Σ sc·D
-            const v16f p1 = __builtin_amdgcn_mfma_f32_32x32x2f32(h == 0 ? S.da[arow] : 0.0f, h == 0 ? S.wd[wrow] : 0.0f, zf, 0, 0, 0);
+            for (int a = 0; a < NW; a++) {
+                const long bw = *(const long *)(S.wq[a] + wrow * K6_ST + 16 * k + 8 * h);
+                const v16i D = __builtin_amdgcn_mfma_i32_32x32x16_i8(av, bw, zi, 0, 0, 0);
+                const int sc = S.wsc[a][wrow * 8 + k];
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                acc[v] = fmaf(p1[v], (float)s1[v], acc[v]);
-                s1[v] = 0;
+                for (int v = 0; v < 16; v++) s1[a][v] = mad24(sc, D[v], s1[a][v]);
             }
         }
-        if (s + 1 < n_stages) k6_store(st[(s + 1) & 1], tid, R);
+        if (hs == 1) {  // end of the superblock: (d_r·d_t)·Σ sc·D
+#pragma unroll
+            for (int a = 0; a < NW; a++) {
+                const v16f p1 = __builtin_amdgcn_mfma_f32_32x32x2f32(h == 0 ? S.da[arow] : 0.0f, h == 0 ? S.wd[a][wrow] : 0.0f, zf, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    acc[a][v] = fmaf(p1[v], (float)s1[a][v], acc[a][v]);
+                    s1[a][v] = 0;
+                }
+            }
+        }
+        if (s + 1 < n_stages) k6_store<GLU>(st[(s + 1) & 1], tid, R);
         __syncthreads();
     }
     const int rows = p.rows[sg];
@@ -495,9 +570,11 @@ __global__ __launch_bounds__(256) void gemm_q6k_kernel(KqP p) {
     for (int v = 0; v < 16; v++) {
         const int r = tr.r0 + wc * 32 + 16 * h + v;
         if (r < tr.r_end) {
+            float y = acc[0][v];
+            if constexpr (GLU) y = (p.glu == 2 ? gelu_tanh_f(acc[0][v]) : silu_f(acc[0][v])) * acc[NW - 1][v];
             float *o = out + (size_t)out_row(p, r) * ld + row;
-            if (epi == EPI_ADD) *o += acc[v];
-            else *o = acc[v];
+            if (epi == EPI_ADD) *o += y;
+            else *o = y;
         }
     }
 }
@@ -518,7 +595,7 @@ void kq_groups(KqP &p, int nseg, const GroupTiles *grp, int bm = KQ_BM) {
 }
 
 // The non-gated 64-token form splits K as k6_launch does (below).
-template <bool GLU, int BN = KQ_BN>
+template <int TY, bool GLU, int BN = KQ_BN>
 void kq_launch(KqP p, hipStream_t st, float *part = nullptr, size_t part_cap = 0) {
     const int slots = (p.n_rg + 7) / 8;
     const int tiles = slots * 8 * p.n_tg, nsb = p.K >> 8;
@@ -529,36 +606,37 @@ void kq_launch(KqP p, hipStream_t st, float *part = nullptr, size_t part_cap = 0
         p.part = part;
         p.part_stride = plane;
     }
-    hipLaunchKernelGGL((gemm_q4k_kernel<GLU, BN>), dim3(tiles * p.ks), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((gemm_q45k_kernel<TY, GLU, BN>), dim3(tiles * p.ks), dim3(256), 0, st, p);
     if (p.ks > 1) launch_gemm_add_parts(p.out[0], p.part, p.part_stride, p.ks - 1, p.rows[0], p.ld[0], p.n_tok, st);
 }
 
 // A single ungrouped segment whose tiles number under 512 splits K in 2 or 4
 // (each split ≥ 4 superblocks) while part holds the extra splits' partial sums
 // (part_cap floats); the partials are added by a second launch.
-void k6_launch(KqP p, hipStream_t st, float *part, size_t part_cap) {
+template <bool GLU>
+void k6_launch(KqP p, hipStream_t st, float *part = nullptr, size_t part_cap = 0) {
     const int slots = (p.n_rg + 7) / 8;
     const int tiles = slots * 8 * p.n_tg, nsb = p.K >> 8;
     p.ks = 1;
-    if (!p.grouped && p.nseg == 1 && part && p.n_tok > 64) {
+    if (!GLU && !p.grouped && p.nseg == 1 && part && p.n_tok > 64) {
         const size_t plane = (size_t)p.n_tok * p.ld[0];
         while (p.ks < 4 && tiles * p.ks < 512 && nsb / (2 * p.ks) >= 4 && (size_t)(2 * p.ks - 1) * plane <= part_cap) p.ks *= 2;
         p.part = part;
         p.part_stride = plane;
     }
-    hipLaunchKernelGGL(gemm_q6k_kernel, dim3(tiles * p.ks), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((gemm_q6k_kernel<GLU>), dim3(tiles * p.ks), dim3(256), 0, st, p);
     if (p.ks > 1) launch_gemm_add_parts(p.out[0], p.part, p.part_stride, p.ks - 1, p.rows[0], p.ld[0], p.n_tok, st);
 }
 
 }  // namespace
 
-bool gemm_kq_supported(int ty, size_t K) { return (ty == T_Q4_K || ty == T_Q6_K) && K % 256 == 0 && K > 0; }
+bool gemm_kq_supported(int ty, size_t K) { return (ty == T_Q4_K || ty == T_Q5_K || ty == T_Q6_K) && K % 256 == 0 && K > 0; }
 
 bool launch_gemm_kq(const GemvSeg *segs, int nseg, const ActQ8 &act, int n_tok, int K, hipStream_t st, const GroupTiles *grp, float *part,
                     size_t part_cap) {
     if (nseg < 1 || nseg > 3 || n_tok < 1 || !act.qs || !act.d || (grp && (nseg != 1 || grp->max_tiles < 1))) return false;
     const int ty = segs[0].w.ty;
-    if (ty == T_Q4_K && !act.bsums) return false;
+    if (ty != T_Q6_K && !act.bsums) return false;
     KqP p{};
     for (int i = 0; i < nseg; i++) {
         const GemvSeg &s = segs[i];
@@ -579,16 +657,17 @@ bool launch_gemm_kq(const GemvSeg *segs, int nseg, const ActQ8 &act, int n_tok, 
     if (grp && grp->bn != KQ_BN && (grp->bn != 32 || ty != T_Q4_K)) return false;
     const bool t32 = grp && grp->bn == 32;  // 32-token tiles of a Q4_K expert grouping
     kq_groups(p, nseg, grp, t32 ? kq_bm<32>() : KQ_BM);
-    if (ty == T_Q6_K) k6_launch(p, st, part, part_cap);
-    else if (t32) kq_launch<false, 32>(p, st);
-    else kq_launch<false>(p, st, part, part_cap);
+    if (ty == T_Q6_K) k6_launch<false>(p, st, part, part_cap);
+    else if (ty == T_Q5_K) kq_launch<T_Q5_K, false>(p, st, part, part_cap);
+    else if (t32) kq_launch<T_Q4_K, false, 32>(p, st);
+    else kq_launch<T_Q4_K, false>(p, st, part, part_cap);
     return true;
 }
 
 bool launch_gemm_kq_glu(const DevWeight &gate, const DevWeight &up, const ActQ8 &act, int n_tok, int K, float *h, int ld, int gelu,
                         hipStream_t st, const GroupTiles *grp) {
     if (grp && grp->max_tiles < 1) return false;
-    if (n_tok < 1 || !act.qs || !act.d || !act.bsums || gate.ty != up.ty || gate.ty != T_Q4_K || !gemm_kq_supported(gate.ty, K) ||
+    if (n_tok < 1 || !act.qs || !act.d || (gate.ty != T_Q6_K && !act.bsums) || gate.ty != up.ty || !gemm_kq_supported(gate.ty, K) ||
         gate.cols != (size_t)K || up.cols != (size_t)K || gate.rows != up.rows || !gate.data || !up.data || !h)
         return false;
     KqP p{};
@@ -607,11 +686,13 @@ bool launch_gemm_kq_glu(const DevWeight &gate, const DevWeight &up, const ActQ8 
     p.qs = act.qs;
     p.d = act.d;
     p.bsums = act.bsums;
-    if (grp && grp->bn != KQ_BN && grp->bn != 32) return false;
+    if (grp && grp->bn != KQ_BN && (grp->bn != 32 || gate.ty != T_Q4_K)) return false;
     const bool t32 = grp && grp->bn == 32;  // 32-token tiles of a Q4_K expert grouping
     kq_groups(p, 1, grp, t32 ? kq_bm<32>() : KQ_BM);
-    if (t32) kq_launch<true, 32>(p, st);
-    else kq_launch<true>(p, st);
+    if (gate.ty == T_Q6_K) k6_launch<true>(p, st);
+    else if (gate.ty == T_Q5_K) kq_launch<T_Q5_K, true>(p, st);
+    else if (t32) kq_launch<T_Q4_K, true, 32>(p, st);
+    else kq_launch<T_Q4_K, true>(p, st);
     return true;
 }
 

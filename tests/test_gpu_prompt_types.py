@@ -1,0 +1,45 @@
+"""Prompt matmuls of the weight types beyond Q4_0 / Q8_0 / Q4_K on the matrix cores,
+against the oracle: kernels through rie_hip_k_gemm, gated and grouped forms
+through small models."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+from test_gpu_parity import Q5_K, Q6_K, _gemv, _pair, _quant_on_gpu, act_fmt, cuda  # noqa: E402,F401
+
+
+def _check_rows(oracle, cuda, ty, k, rows, n_tok):
+    """k_gemm rows within 1e-5·Σ|w·x| + 1e-6 of the oracle's block dots (the f32 sums'
+    rounding over K ≤ 2^14 terms in any order stays under 1e-5 of the magnitudes)"""
+    import ggml_np as G
+    w = oracle.Rng(31 + ty).random_weight(ty, rows, k)
+    x = (np.random.default_rng(k + n_tok).uniform(-1, 1, (n_tok, k)) * 2).astype(np.float32)
+    got = _gemv(ty, w, rows, k, _quant_on_gpu(x, act_fmt(ty), cuda)["dev"], None, n_tok, cuda, gemm=True)
+    wf = G.dequantize(ty, w, rows * k).reshape(rows, k).astype(np.float64)
+    rb = G.row_bytes(ty, k)
+    for t in range(n_tok):
+        a = oracle.quantize_act(ty, x[t])
+        want = np.array([oracle.vec_dot(ty, w[i * rb:(i + 1) * rb], a, k) for i in range(rows)])
+        mag = np.abs(wf * x[t].astype(np.float64)).sum(axis=1)
+        assert np.all(np.abs(got[t] - want) <= 1e-5 * mag + 1e-6), (ty, k, rows, n_tok, t)
+
+
+# one superblock, row and token remainders, a K split in two uneven parts (13 superblocks)
+@pytest.mark.parametrize("k,rows,n_tok", [(256, 40, 9), (512, 200, 33), (1024, 300, 130), (3328, 96, 70)])
+def test_q5_k_gemm_matches_oracle_rows(oracle, cuda, k, rows, n_tok):
+    _check_rows(oracle, cuda, Q5_K, k, rows, n_tok)
+
+
+@pytest.mark.parametrize("arch,ty", [("llama", Q5_K), ("gemma2", Q5_K), ("gemma2", Q6_K), ("qwen3moe", Q5_K), ("qwen3moe", Q6_K)])
+def test_gated_and_grouped_k_quant_prompts_match_oracle(oracle, cuda, arch, ty):
+    """Gate/up with SwiGLU or GELU in one launch, and experts grouped on the device."""
+    from naive_model import max_rel_err
+    spec, g, o = _pair(oracle, arch, ty, 0, n_ctx=96, max_batch=70)
+    nv = spec.n_vocab
+    toks = [(i * 29 + 3) % nv for i in range(70)]
+    lg, lo = g.forward(toks, 0, True), o.forward(toks, 0, True)
+    for t in range(70):
+        err = max_rel_err(lg[t * nv:(t + 1) * nv], lo[t * nv:(t + 1) * nv])
+        assert err < 0.03, f"{arch} {ty}: token {t}: {err}"
