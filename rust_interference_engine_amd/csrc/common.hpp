@@ -94,6 +94,13 @@ struct ActQ8 {
     int16_t *bsums = nullptr;
 };
 
+// f32 rows as sums of 16-bit parts, for matmuls with unquantized weights on the 16-bit
+// matrix cores: [n][k] bf16 ×3, or f16 ×3 of the row times 1/scale[row] (a power of two)
+struct ActSplit {
+    uint16_t *p[3] = {nullptr, nullptr, nullptr};
+    float *scale = nullptr;
+};
+
 // A weight matrix resident in HBM in its native ggml block layout.
 struct DevWeight {
     int ty = -1;

@@ -204,6 +204,17 @@ HipBackend::HipBackend(const uint8_t *gguf, size_t len, const BackendConfig &cfg
     // partial sums of K-split prompt GEMMs (up to three planes of a batch's E-wide
     // outputs, at most 64 MiB): only batches above 64 tokens split
     gemm_ws_cap_ = mb > 64 ? std::min<size_t>(3 * mb * E, (size_t)1 << 24) : 0;
+    // BF16 / F16 matrices: the parts of a prompt's rows, and the partial sums of up to
+    // four splits of Q/K/V (at most 64 MiB)
+    bool halves = act_format(out_w_.ty) == ACT_F32 && out_w_.ty != T_F32;
+    for (auto &L : layers_)
+        for (const DevWeight *w : {&L.wq, &L.wk, &L.wv, &L.wo, &L.gate, &L.up, &L.down, &L.router, &L.sh_gate, &L.sh_up, &L.sh_down})
+            halves = halves || w->ty == T_BF16 || w->ty == T_F16;
+    if (halves && mb > 8) {
+        for (auto &p : split_.p) p = dalloc<uint16_t>(allocs_, mb * kmax_);
+        split_.scale = dalloc<float>(allocs_, mb);
+        gemm_ws_cap_ = std::max(gemm_ws_cap_, std::min<size_t>(4 * mb * std::max(E, qd + 2 * kvd), (size_t)1 << 24));
+    }
     if (gemm_ws_cap_) d_gemm_ws_ = dalloc<float>(allocs_, gemm_ws_cap_);
     // routed experts per token as the layers run them (clamped to [1, n_expert], model/mod.rs:176)
     const size_t nu = std::max<size_t>(n_used_max_, 1);
@@ -303,6 +314,7 @@ void HipBackend::prepare(const float *x, const float *norm, int n, int K, const 
         if (ws[i] && ws[i]->ty >= 0) need[act_format(ws[i]->ty)] = true;
     const float eps = m_.cfg.rms_eps;
     bool wrote_f32 = false;
+    split_ty_ = -1;
     if (need[ACT_Q8_0]) {
         launch_rmsnorm_quant(x, K, norm, eps, n, K, need[ACT_F32] ? d_xn_ : nullptr, ACT_Q8_0, act0_, st_, ref_order);
         wrote_f32 = need[ACT_F32];
@@ -312,10 +324,23 @@ void HipBackend::prepare(const float *x, const float *norm, int n, int K, const 
         wrote_f32 = wrote_f32 || need[ACT_F32];
     }
     if (need[ACT_F32] && !wrote_f32) {
-        if (norm) launch_rmsnorm(x, K, norm, eps, n, K, d_xn_, K, 0, st_, ref_order);
-        else RIE_HIP_CHECK(hipMemcpyAsync(d_xn_, x, (size_t)n * K * 4, hipMemcpyDeviceToDevice, st_));
+        int fty = -1;
+        for (int i = 0; i < nw && fty < 0; i++)
+            if (ws[i] && gemm_float_supported(ws[i]->ty, K)) fty = ws[i]->ty;
+        float_rows(x, norm, n, K, fty, ref_order);
     }
     check_launch("prepare");
+}
+
+void HipBackend::float_rows(const float *x, const float *norm, int n, int K, int ty, bool ref_order) {
+    if (n > 8 && split_.p[0] && gemm_float_supported(ty, K)) {
+        launch_split_rows(x, K, norm, m_.cfg.rms_eps, n, K, d_xn_, ty, split_, st_, ref_order);
+        split_ty_ = ty;
+        return;
+    }
+    split_ty_ = -1;
+    if (norm) launch_rmsnorm(x, K, norm, m_.cfg.rms_eps, n, K, d_xn_, K, 0, st_, ref_order);
+    else RIE_HIP_CHECK(hipMemcpyAsync(d_xn_, x, (size_t)n * K * 4, hipMemcpyDeviceToDevice, st_));
 }
 
 // matmul_multi (matmul.rs:136-176): decode-sized batches stream the weights
@@ -334,6 +359,16 @@ void HipBackend::matmul(const GemvSeg *segs, int nseg, int n, int K, const ActQ8
             int e = s + 1;
             while (e < j && e - s < 3 && segs[e].w.ty == segs[s].w.ty) e++;
             if (!launch_gemm(&segs[s], e - s, a, n, K, st_, nullptr, d_gemm_ws_, gemm_ws_cap_)) break;
+            s = e;
+        }
+        while (n > 8 && s < j && split_.p[0] && gemm_float_supported(segs[s].w.ty, K)) {
+            int e = s + 1;
+            while (e < j && e - s < 3 && segs[e].w.ty == segs[s].w.ty) e++;
+            if (split_ty_ != segs[s].w.ty) {
+                launch_split_rows(d_xn_, K, nullptr, 0.0f, n, K, nullptr, segs[s].w.ty, split_, st_);
+                split_ty_ = segs[s].w.ty;
+            }
+            if (!launch_gemm_float(&segs[s], e - s, split_, n, K, st_, d_gemm_ws_, gemm_ws_cap_)) break;
             s = e;
         }
         if (s < j && !launch_gemv(&segs[s], j - s, a, d_xn_, n, K, st_))
@@ -357,6 +392,7 @@ void HipBackend::ffn_dense(const DevLayer &L, int n, float *out, int epi) {
     const ActQ8 &a = act_format(L.gate.ty) == ACT_Q8K ? actk_ : act0_;
     bool done = false;
     if (n > 8 && gemm_supported(L.gate.ty, E)) done = launch_gemm_glu(L.gate, L.up, a, n, E, d_h_, ff, c.gelu, nullptr, st_);
+    if (n > 8 && L.gate.ty == split_ty_) done = launch_gemm_float_glu(L.gate, L.up, split_, n, E, d_h_, ff, c.gelu, st_);
     const int fmt = act_format(L.down.ty);
     // single-token Q8_0 down projection: the gate/up kernel quantizes h itself
     bool h_quantized = false;
@@ -371,7 +407,7 @@ void HipBackend::ffn_dense(const DevLayer &L, int n, float *out, int epi) {
     // over the 8192-value hidden of the Llama-3.2-3B shape measured 670 against 690
     // tok/s, its 32 KB of x per workgroup on every workgroup's critical path)
     if (!h_quantized) {
-        if (fmt == ACT_F32) RIE_HIP_CHECK(hipMemcpyAsync(d_xn_, d_h_, (size_t)n * ff * 4, hipMemcpyDeviceToDevice, st_));
+        if (fmt == ACT_F32) float_rows(d_h_, nullptr, n, ff, L.down.ty);
         else launch_quant_only(d_h_, ff, n, ff, fmt, fmt == ACT_Q8K ? actk_ : act0_, st_);
         mark("quant");
     }
@@ -498,7 +534,7 @@ void HipBackend::run_layers(int n, size_t pos0, const int *d_pos0, bool all_logi
         // one token, K-quant wo: its GEMV quantizes the attention output itself (Q8_K prologue without a norm)
         const bool wo_self_q = n == 1 && !capture_ && wo_fmt == ACT_Q8K && gemv_quant_ok(L.wo.ty, qd);
         if (wo_fmt == ACT_Q8K && !wo_self_q) launch_quant_only(d_att_, qd, n, qd, ACT_Q8K, actk_, st_);
-        if (wo_fmt == ACT_F32) RIE_HIP_CHECK(hipMemcpyAsync(d_xn_, d_att_, (size_t)n * qd * 4, hipMemcpyDeviceToDevice, st_));
+        if (wo_fmt == ACT_F32) float_rows(d_att_, nullptr, n, qd, L.wo.ty);
         const bool direct = !L.post_attn_norm && c.residual_scale == 1.0f;
         GemvSeg so{L.wo, direct ? d_x_ : d_o_, E, direct ? EPI_ADD : EPI_STORE};
         if (wo_self_q) {
@@ -567,7 +603,7 @@ void HipBackend::head(int first, int m) {
                      launch_gemv(&s, 1, fmt == ACT_Q8K ? actk_ : act0_, d_xn_, 1, E, st_, &nin));
     if (head_normed_) {  // the normalized rows are kept in d_xn_ for Backend::hidden
         if (fmt == ACT_F32) {
-            launch_rmsnorm(xr, E, out_norm_, c.rms_eps, m, E, d_xn_, E, 0, st_);
+            float_rows(xr, out_norm_, m, E, out_w_.ty);
         } else {
             launch_rmsnorm_quant(xr, E, out_norm_, c.rms_eps, m, E, d_xn_, fmt, fmt == ACT_Q8K ? actk_ : act0_, st_);
         }
@@ -599,10 +635,11 @@ void HipBackend::expert_ffn(const DevWeight &g, const DevWeight &u, const DevWei
     const ActQ8 &a = act_format(g.ty) == ACT_Q8K ? actk_ : act0_;
     bool done = false;
     if (m > 8 && gemm_supported(g.ty, E)) done = launch_gemm_glu(g, u, a, m, E, d_h_, ff, c.gelu, nullptr, st_);
+    if (m > 8 && g.ty == split_ty_) done = launch_gemm_float_glu(g, u, split_, m, E, d_h_, ff, c.gelu, st_);
     if (!done && !launch_gemv_glu(g, u, a, d_xn_, m, E, d_h_, ff, c.gelu, nullptr, st_))
         throw Error{E_UNSUPPORTED, "unsupported: expert FFN weights"};
     const int fmt = act_format(dn.ty);
-    if (fmt == ACT_F32) RIE_HIP_CHECK(hipMemcpyAsync(d_xn_, d_h_, (size_t)m * ff * 4, hipMemcpyDeviceToDevice, st_));
+    if (fmt == ACT_F32) float_rows(d_h_, nullptr, m, ff, dn.ty);
     else launch_quant_only(d_h_, ff, m, ff, fmt, fmt == ACT_Q8K ? actk_ : act0_, st_);
     GemvSeg s{dn, y, E, EPI_STORE};
     matmul(&s, 1, m, ff);

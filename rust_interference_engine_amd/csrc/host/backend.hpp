@@ -133,6 +133,10 @@ class HipBackend {
     int *d_route_cnt_ = nullptr;  // arrival counter of the router GEMV that routes one token
     ActQ8 act0_, actk_;  // Q8_0 and Q8_K batches
     ActQ8 act_h_;        // Q8_0 of the single-token FFN hidden
+    ActSplit split_;     // 16-bit parts of d_xn_'s rows (models with BF16 / F16 matrices)
+    int split_ty_ = -1;  // the weight type split_ was made for, -1: not d_xn_'s present rows
+    // d_xn_ = RMSNorm(x)·norm (x itself without norm) in f32, with its parts where n rows go to the GEMM of ty
+    void float_rows(const float *x, const float *norm, int n, int K, int ty, bool ref_order = false);
     size_t kmax_ = 0, ff_max_ = 0, part_floats_ = 0;
     size_t n_used_max_ = 0;  // largest clamped routed-expert count of any MoE layer
     // MoE scratch

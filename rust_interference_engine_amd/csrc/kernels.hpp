@@ -194,6 +194,18 @@ void launch_gemm_add_parts(float *out, const float *part, size_t stride, int n_p
 bool launch_gemm_kq_glu(const DevWeight &gate, const DevWeight &up, const ActQ8 &act, int n_tok, int K, float *h, int ld, int gelu,
                         hipStream_t st, const GroupTiles *grp = nullptr);
 
+// ---- gemm_float.hip (prefill, BF16 / F16 × f32 on 16-bit MFMA) ----
+bool gemm_float_supported(int ty, size_t K);
+// the parts of n_rows rows of RMSNorm(x)·w (x itself without w) for weights of type ty,
+// and the rows themselves to xn when given; ref_order as in launch_rmsnorm
+void launch_split_rows(const float *x, int ldx, const float *w, float eps, int n_rows, int E, float *xn, int ty, const ActSplit &act,
+                       hipStream_t st, bool ref_order = false);
+// act: the rows' parts for the segments' (one) type; part (part_cap floats): room for a K
+// split.  False (nothing launched) for weights that the kernel does not take.
+bool launch_gemm_float(const GemvSeg *segs, int nseg, const ActSplit &act, int n_tok, int K, hipStream_t st, float *part, size_t part_cap);
+bool launch_gemm_float_glu(const DevWeight &gate, const DevWeight &up, const ActSplit &act, int n_tok, int K, float *h, int ld, int gelu,
+                           hipStream_t st);
+
 // ---- gemm.hip (prefill, int8 MFMA) ----
 bool gemm_supported(int ty, size_t K);
 // grp: one segment per expert group (the segment's rows are one expert's; see GroupTiles)
