@@ -1626,6 +1626,83 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a) {
     }
 }
 
+// The same for head sizes 64, 128 and 256 and up to 64 ranges: one wave per (token,
+// head), lane l holding dims V·l .. V·l + V − 1 and, first, range l's maximum and sum.
+// No barriers, and a quarter of the workgroups (512 tokens × 32 heads, 4 ranges:
+// 26 us in the kernel above).
+template <int HD>
+__global__ __launch_bounds__(256) void attn_combine_rows_kernel(AttnArgs a) {
+    constexpr int V = HD / 64;
+    const int lane = threadIdx.x & 63, i0 = V * lane;
+    const int row = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));  // t·n_head + h
+    if (row >= a.n_tok * a.n_head) return;
+    const float *part = a.part + (size_t)row * a.n_split * (HD + 2);
+    float m = -INFINITY, l = 0.0f;
+    if (lane < a.n_split) {
+        m = part[(size_t)lane * (HD + 2) + HD];
+        l = part[(size_t)lane * (HD + 2) + HD + 1];
+    }
+    const float M = xmax_f<64>(m);
+    const float w = l > 0.0f ? expf(m - M) : 0.0f;
+    const float inv = 1.0f / xsum_f<64>(l * w);
+    float o[V] = {};
+#pragma unroll 4
+    for (int s = 0; s < a.n_split; s++) {
+        const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s));
+#pragma unroll
+        for (int i = 0; i < V; i++) o[i] = fmaf(part[(size_t)s * (HD + 2) + i0 + i], ws, o[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < V; i++) o[i] *= inv;
+    if (a.kv_type == 2) {  // o ← Rᵀ o: the FWHT's stages of distance 1, 2, …, HD/2, then signs (turbo.rs:114-117)
+#pragma unroll
+        for (int st = 1; st < V; st *= 2)
+#pragma unroll
+            for (int i = 0; i < V; i++)
+                if (!(i & st)) {
+                    const float p = o[i], q = o[i + st];
+                    o[i] = p + q;
+                    o[i + st] = p - q;
+                }
+        xor_up<1, 32>([&](auto oc) {
+            constexpr int O = decltype(oc)::value;
+#pragma unroll
+            for (int i = 0; i < V; i++) {
+                const float p = xor_f<O>(o[i]);
+                o[i] = (lane & O) == 0 ? o[i] + p : p - o[i];
+            }
+        });
+        const float sc = 1.0f / sqrtf((float)HD);
+#pragma unroll
+        for (int i = 0; i < V; i++) o[i] = o[i] * sc * a.turbo_signs[i0 + i];
+    }
+    const size_t e0 = (size_t)row * HD + i0;
+#pragma unroll
+    for (int i = 0; i < V; i++) a.att[e0 + i] = o[i];
+    if (a.att_fmt == ACT_Q8_0) {  // 32/V lanes per block
+        float amax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < V; i++) amax = fmaxf(amax, fabsf(o[i]));
+        amax = xmax_f<32 / V>(amax);
+        const float d = amax / 127.0f, id = d != 0.0f ? 1.0f / d : 0.0f;
+        int su = 0, scl = 0;
+#pragma unroll
+        for (int i = 0; i < V; i++) {
+            const int q = (int)rintf(o[i] * id), qc = q < -127 ? -127 : (q > 127 ? 127 : q);
+            su += q;
+            scl += qc;
+            a.att_q.qs[e0 + i] = (int8_t)qc;
+        }
+        su = xsum_i<32 / V>(su);
+        scl = xsum_i<32 / V>(scl);
+        if (lane % (32 / V) == 0) {
+            a.att_q.d[e0 / 32] = d;
+            if (a.att_q.s) a.att_q.s[e0 / 32] = d * (float)su;
+            if (a.att_q.isum) a.att_q.isum[e0 / 32] = scl;
+        }
+    }
+}
+
 template <int KVT, int SUB>
 static void launch_split_g(const AttnArgs &a, int G, dim3 grid, hipStream_t st) {
     if (G <= 2) hipLaunchKernelGGL((attn_split_kernel<KVT, SUB, 2>), grid, dim3(256), 0, st, a);
@@ -1710,11 +1787,15 @@ void launch_attention(const AttnArgs &a, hipStream_t st) {
     case 1: launch_kvt<1>(a, grid, st); break;
     default: launch_kvt<2>(a, grid, st); break;
     }
-    hipLaunchKernelGGL(attn_combine_kernel, dim3(a.n_head, a.n_tok), dim3(256), 0, st, a);
+    launch_attention_combine(a, st);
 }
 
 void launch_attention_combine(const AttnArgs &a, hipStream_t st) {
-    hipLaunchKernelGGL(attn_combine_kernel, dim3(a.n_head, a.n_tok), dim3(256), 0, st, a);
+    const dim3 rows((a.n_tok * a.n_head + 3) / 4);
+    if (a.n_split <= 64 && a.hd == 64) hipLaunchKernelGGL(attn_combine_rows_kernel<64>, rows, dim3(256), 0, st, a);
+    else if (a.n_split <= 64 && a.hd == 128) hipLaunchKernelGGL(attn_combine_rows_kernel<128>, rows, dim3(256), 0, st, a);
+    else if (a.n_split <= 64 && a.hd == 256) hipLaunchKernelGGL(attn_combine_rows_kernel<256>, rows, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(attn_combine_kernel, dim3(a.n_head, a.n_tok), dim3(256), 0, st, a);
 }
 
 bool attention_fused_ok(const AttnArgs &a) {

@@ -19,6 +19,16 @@
 // probabilities before the P·V product (axpy_rotated_4's factor), and the output
 // goes back through the inverse rotation (FWHT, 1/√128, signs) in the epilogue.
 //
+// Q8_0 caches (KVT = 1, cpu.rs:564-582): the query is quantized to Q8_0 as it is
+// loaded, the 32-value block dots are the reference's exact integer dots, on
+// v_mfma_i32_32x32x32_i8, and a score is Σ_b (d_k·isum)·d_q over its blocks.  A value
+// row's d·code has at most 18 significant bits, so it is staged as two f16 halves
+// without rounding and P·V takes the four products of its halves and the probability's.
+// A block of 32 dims whose values leave the f16 range (|d| > 512 somewhere) is found
+// at its staging; the workgroup then runs its tiles once more with that block's values
+// times 2^-8.  (512 tokens at 7680, 32 heads of 128: 2360 us per layer in
+// attn_split_kernel, a workgroup per token and KV head on the vector units.)
+//
 // Work split: a workgroup (4 waves) owns one KV head and a block of query rows;
 // each wave owns 32 tokens of one query head.  Scores are computed transposed,
 // Sᵀ = K·Qᵀ (v_mfma_f32_32x32x16_f16: lane l holds token l mod 32 and 16 cache
@@ -38,6 +48,8 @@ namespace rie {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x16 __attribute__((ext_vector_type(16)));
 
 namespace {
 
@@ -85,10 +97,21 @@ __device__ __forceinline__ half8 split_hi(const float (&x)[8], half8 &lo) {
 
 __device__ __forceinline__ half8 as_half8(u32x4 v) { return __builtin_bit_cast(half8, v); }
 
+// bytes of a Q8_0 block's codes, which start 2 bytes behind a 2-byte boundary
+struct __attribute__((packed, aligned(2))) Codes16 {
+    uint32_t w[4];
+};
+struct __attribute__((packed, aligned(2))) Codes8 {
+    uint32_t w[2];
+};
+__device__ __forceinline__ float code_f(uint32_t w, int e) { return (float)(int)(int8_t)((w >> (8 * e)) & 0xff); }
+
 // LDS bytes of one wave group's K and transposed V tile (+ the rows' score and
-// probability factors of a Turbo4 tile)
+// probability factors of a Turbo4 tile; Q8_0: K codes, V halves, K block scales)
 template <int HD, int KVT = 0>
-constexpr int tile_bytes() { return PT * (HD * 2 + 16) + HD * VROW + (KVT == 2 ? 2 * PT * 4 : 0); }
+constexpr int tile_bytes() {
+    return KVT == 1 ? PT * (HD + 16) + 2 * HD * VROW + PT * (HD / 32) * 4 : PT * (HD * 2 + 16) + HD * VROW + (KVT == 2 ? 2 * PT * 4 : 0);
+}
 // merge scratch of NW groups: running maxima and sums, then one 32-dim output tile per group
 template <int NW>
 constexpr int merge_bytes() { return NW > 1 ? 2 * NW * 256 * 4 + (NW - 1) * 256 * 16 * 4 : 0; }
@@ -101,12 +124,13 @@ constexpr int prompt_lds_bytes() {
 // online-softmax states are merged through LDS at the end.
 template <int HD, int NW, int KVT>
 __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
-    static_assert(KVT == 0 || (KVT == 2 && HD == 128), "Turbo4 tiles: one 128-dim rotation block per row");
+    static_assert(KVT != 2 || HD == 128, "Turbo4 tiles: one 128-dim rotation block per row");
     constexpr int KS = HD / 16;          // 16-dim k-steps of the score product
     constexpr int DT = HD / 32;          // 32-dim output tiles
-    constexpr int KROW = HD * 2 + 16;    // bytes per K row in LDS (padded)
-    constexpr int NCH = (PT * HD / 8 + 255) / 256;  // 16-byte chunks per thread per tile (K and V each)
-    constexpr int RB = KVT == 2 ? HD / 2 : HD * 2;   // cache row bytes
+    constexpr int KROW = (KVT == 1 ? HD : HD * 2) + 16;  // bytes per K row in LDS (padded)
+    constexpr int NCH = (PT * HD / (KVT == 1 ? 16 : 8) + 255) / 256;  // 16-byte K chunks per thread per tile
+    constexpr int NV = (2 * HD + 255) / 256;             // V pieces (two positions × 8 dims) per thread per tile
+    constexpr int RB = KVT == 1 ? HD / 32 * 34 : KVT == 2 ? HD / 2 : HD * 2;  // cache row bytes
     extern __shared__ __align__(16) uint8_t lds[];
     constexpr int TB = tile_bytes<HD, KVT>();
     const int grp = threadIdx.x >> 8;
@@ -151,8 +175,38 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     const bool w_full = wave_on && tb * 32 + 31 < a.n_tok;                        // all 32 tokens exist
 
     // query fragments: token col of the block, dims 16s + 8h .. +8 (f32 → hi + lo)
-    half8 qh[KS], ql[KS];
-    {
+    half8 qh[KVT == 1 ? 1 : KS], ql[KVT == 1 ? 1 : KS];
+    i32x4 q8[KVT == 1 ? DT : 1];  // Q8_0: codes 16h .. +16 of each block, and the blocks' scales in log2 units
+    float dq[KVT == 1 ? DT : 1];
+    if constexpr (KVT == 1) {
+        const float *qrow = a.q + (size_t)(tok_ok ? t : a.n_tok - 1) * qd + (size_t)(wave_on ? head : 0) * hd + 16 * h;
+#pragma unroll
+        for (int b = 0; b < DT; b++) {
+            float x[16], amax = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const f32x4 v = *(const f32x4 *)(qrow + 32 * b + 4 * i);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    x[4 * i + e] = v[e];
+                    amax = fmaxf(amax, fabsf(v[e]));
+                }
+            }
+            amax = fmaxf(amax, xor_f<32>(amax));
+            const float d = amax / 127.0f, id = d != 0.0f ? 1.0f / d : 0.0f;
+            dq[b] = d * LOG2E_F;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                uint32_t w = 0;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int q = (int)rintf(x[4 * i + e] * id);
+                    w |= (uint32_t)((q < -127 ? -127 : (q > 127 ? 127 : q)) & 0xff) << (8 * e);
+                }
+                q8[b][i] = (int)w;
+            }
+        }
+    } else {
         const int tq = tok_ok ? t : (a.n_tok - 1);
         const float *qrow = a.q + (size_t)tq * qd + (size_t)(wave_on ? head : 0) * hd;
 #pragma unroll
@@ -171,10 +225,13 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     // one tile in flight in registers: f16 K as 16-byte row chunks and V as two
     // positions × 8 dims; Turbo4 K as 8 code bytes of a row, V as 4 code bytes of two
     // rows, and the row scale of position tid (K) or tid − 32 (V)
+    // (Q8_0: K as 16 codes of a row, V as 8 codes of two rows with their blocks' scales,
+    // and the scale of K block tid / 32 of position tid % 32)
     struct Regs {
         u32x4 k[NCH];
-        u32x4 v[2];
+        u32x4 v[NV][2];
         uint32_t sc;
+        uint32_t vsc[KVT == 1 ? NV : 1][2];
     };
     // Every lane issues the same loads (indices past the tile's data repeat valid
     // ones, and ring slots wrap without a branch: slots ≥ 32 = the tile length).
@@ -192,19 +249,46 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
             r.k[0] = u32x4{kk.x, kk.y, 0u, 0u};
 #pragma unroll
             for (int rr = 0; rr < 2; rr++)  // positions 2·(tid/16) + rr, bytes 4·(tid%16)..+4
-                r.v[rr][0] = *(const uint32_t *)(vc + row(2 * (tid >> 4) + rr) + 4 * (tid & 15));
+                r.v[0][rr][0] = *(const uint32_t *)(vc + row(2 * (tid >> 4) + rr) + 4 * (tid & 15));
             r.sc = tid < 32 ? ksc[slot(tid)] : vsc[slot(min(tid - 32, PT - 1))];
+        } else if constexpr (KVT == 1) {
+#pragma unroll
+            for (int c = 0; c < NCH; c++) {
+                const int ch = min(tid + 256 * c, PT * HD / 16 - 1), cc = ch % (HD / 16);
+                r.k[c] = __builtin_bit_cast(u32x4, *(const Codes16 *)(kc + row(ch / (HD / 16)) + (cc >> 1) * 34 + 2 + (cc & 1) * 16));
+            }
+            const int kb = min(tid, PT * DT - 1);
+            r.sc = *(const uint16_t *)(kc + row(kb & 31) + (kb >> 5) * 34);
+#pragma unroll
+            for (int c = 0; c < NV; c++) {
+                const int vi = min(tid + 256 * c, 2 * HD - 1), d0 = (vi >> 4) * 8;
+#pragma unroll
+                for (int rr = 0; rr < 2; rr++) {
+                    const uint8_t *blk = vc + row(2 * (vi & 15) + rr) + d0 / 32 * 34;
+                    const Codes8 cd = *(const Codes8 *)(blk + 2 + d0 % 32);
+                    r.v[c][rr][0] = cd.w[0];
+                    r.v[c][rr][1] = cd.w[1];
+                    r.vsc[c][rr] = *(const uint16_t *)blk;
+                }
+            }
         } else {
 #pragma unroll
             for (int c = 0; c < NCH; c++) {
                 const int ch = min(tid + 256 * c, PT * HD / 8 - 1);
                 r.k[c] = *(const u32x4 *)(kc + row(ch / (HD / 8)) + (ch % (HD / 8)) * 16);
             }
-            const int vi = min(tid, 2 * HD - 1);  // positions 2·(vi % 16) + {0, 1}, dims 8·(vi / 16) .. +8
 #pragma unroll
-            for (int rr = 0; rr < 2; rr++) r.v[rr] = *(const u32x4 *)(vc + row(2 * (vi & 15) + rr) + (vi >> 4) * 16);
+            for (int c = 0; c < NV; c++) {
+                const int vi = min(tid + 256 * c, 2 * HD - 1);  // positions 2·(vi % 16) + {0, 1}, dims 8·(vi / 16) .. +8
+#pragma unroll
+                for (int rr = 0; rr < 2; rr++) r.v[c][rr] = *(const u32x4 *)(vc + row(2 * (vi & 15) + rr) + (vi >> 4) * 16);
+            }
         }
     };
+    // Q8_0: blocks of 32 dims with values past the f16 range, found by the first run over
+    // the tiles; their values are then staged ×2^-8 and their outputs multiplied by 2^8
+    __shared__ int vbig[KVT == 1 ? DT : 1];
+    uint32_t vsmall = 0;  // bit b: block b is staged ×2^-8
     auto stage = [&](const Regs &r, int buf) {
         uint8_t *kb = tiles + buf * TB, *vb = kb + PT * KROW;
         if constexpr (KVT == 2) {
@@ -227,8 +311,8 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
             const int pp = tid >> 4, j = tid & 15;
 #pragma unroll
             for (int half = 0; half < 2; half++) {
-                const uint32_t l0 = tq_levels4((half ? (r.v[0][0] >> 4) : r.v[0][0]) & 0x0F0F0F0Fu);
-                const uint32_t l1 = tq_levels4((half ? (r.v[1][0] >> 4) : r.v[1][0]) & 0x0F0F0F0Fu);
+                const uint32_t l0 = tq_levels4((half ? (r.v[0][0][0] >> 4) : r.v[0][0][0]) & 0x0F0F0F0Fu);
+                const uint32_t l1 = tq_levels4((half ? (r.v[0][1][0] >> 4) : r.v[0][1][0]) & 0x0F0F0F0Fu);
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const int dim = 32 * (j >> 2) + 4 * (j & 3) + 16 * half + e;
@@ -242,16 +326,48 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
             if (tid < 2 * PT) fac[tid] = h2f(r.sc) * (tid < PT ? LOG2E_F / 46.0f : 256.0f / 46.0f);
             return;
         }
+        if constexpr (KVT == 1) {
+#pragma unroll
+            for (int c = 0; c < NCH; c++) {
+                const int ch = tid + 256 * c;
+                if (ch < PT * HD / 16) *(u32x4 *)(kb + (ch / (HD / 16)) * KROW + (ch % (HD / 16)) * 16) = r.k[c];
+            }
+            uint8_t *vl = vb + HD * VROW;  // the low halves' rows
+            float *dk = (float *)(vl + HD * VROW);
+            if (tid < PT * DT) dk[tid] = h2f(r.sc);  // [block][position]
+#pragma unroll
+            for (int c = 0; c < NV; c++) {
+                const int vi = tid + 256 * c;
+                if (vi >= 2 * HD) continue;
+                const int b = vi >> 6;
+                const float f = (vsmall >> b & 1) ? 1.0f / 256.0f : 1.0f;
+                const float d0 = h2f(r.vsc[c][0]), d1 = h2f(r.vsc[c][1]);
+                if (fmaxf(fabsf(d0), fabsf(d1)) > 512.0f) vbig[b] = 1;
+                uint8_t *dst = vb + 8 * (vi >> 4) * VROW + 4 * (vi & 15);
+#pragma unroll
+                for (int i = 0; i < 8; i++) {  // one dword = the two positions of one dim
+                    const float x0 = code_f(r.v[c][0][i >> 2], i & 3) * (d0 * f), x1 = code_f(r.v[c][1][i >> 2], i & 3) * (d1 * f);
+                    const auto hi = __builtin_amdgcn_cvt_pkrtz(x0, x1);  // cut off: the rest fits 11 bits
+                    const auto lo = __builtin_amdgcn_cvt_pkrtz(x0 - (float)hi[0], x1 - (float)hi[1]);
+                    *(uint32_t *)(dst + i * VROW) = __builtin_bit_cast(uint32_t, hi);
+                    *(uint32_t *)(dst + HD * VROW + i * VROW) = __builtin_bit_cast(uint32_t, lo);
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int c = 0; c < NCH; c++) {
             const int ch = tid + 256 * c;
             if (ch < PT * HD / 8) *(u32x4 *)(kb + (ch / (HD / 8)) * KROW + (ch % (HD / 8)) * 16) = r.k[c];
         }
-        if (tid < 2 * HD) {  // Vᵀ[dim][pos]: one dword = the two positions of one dim
-            uint8_t *dst = vb + 8 * (tid >> 4) * VROW + 4 * (tid & 15);
+#pragma unroll
+        for (int c = 0; c < NV; c++) {  // Vᵀ[dim][pos]: one dword = the two positions of one dim
+            const int vi = tid + 256 * c;
+            if (vi >= 2 * HD) continue;
+            uint8_t *dst = vb + 8 * (vi >> 4) * VROW + 4 * (vi & 15);
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                const uint32_t w0 = r.v[0][i >> 1], w1 = r.v[1][i >> 1];
+                const uint32_t w0 = r.v[c][0][i >> 1], w1 = r.v[c][1][i >> 1];
                 const uint32_t pair = (i & 1) ? ((w0 >> 16) | (w1 & 0xFFFF0000u)) : ((w0 & 0xFFFFu) | (w1 << 16));
                 *(uint32_t *)(dst + i * VROW) = pair;
             }
@@ -259,27 +375,14 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     };
 
     const uint8_t *k_s = tiles, *v_s = tiles + PT * KROW;  // rebound per tile below
-    float m = -INFINITY, l_half = 0.0f;
+    float m, l_half;
     f32x16 o[DT];
-#pragma unroll
-    for (int d = 0; d < DT; d++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) o[d][v] = 0.0f;
 
     // group tile i is T(i) = t_lo + grp + i·NW; buffer i & 1 holds T(i) during iteration
     // i, and the register sets hold T(i+1) and T(i+2) (issued two iterations before
     // their use)
     const int n_iter = (t_hi - t_lo + NW - 1) / NW;
-    // Loads are issued unconditionally (tile indices past the end repeat the last
-    // tile; an empty split loads tile 0) so that every wait for a register set is an
-    // exact count of the loads issued after it.
-    Regs ra, rb;
     const int last = max(n_tiles - 1, 0);
-    fetch(min(t_lo + grp, last), ra);
-    stage(ra, 0);
-    fetch(min(t_lo + grp + NW, last), rb);
-    fetch(min(t_lo + grp + 2 * NW, last), ra);
-    __syncthreads();
     auto body = [&](int it, Regs &x) {
         const int tile = t_lo + grp + it * NW;
         stage(x, (it + 1) & 1);
@@ -292,8 +395,31 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
         if (work) {
             // Sᵀ[pos][tok] = Σ_d K[pos][d]·q[tok][d]; the hi and lo halves of q in two chains
             f32x16 s = {}, s2 = {};
+            if constexpr (KVT == 1) {
+                const float *dk = (const float *)(v_s + 2 * HD * VROW) + 4 * h;
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
+                for (int b0 = 0; b0 < DT; b0 += 2) {  // two blocks at a time: all of them do not fit the registers
+                    constexpr int NB2 = DT < 2 ? 1 : 2;
+                    i32x16 I[NB2];
+#pragma unroll
+                    for (int b = 0; b < NB2 && b0 + b < DT; b++) {
+                        const i32x4 kf = *(const i32x4 *)(k_s + col * KROW + 32 * (b0 + b) + 16 * h);
+                        I[b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf, q8[b0 + b], i32x16{}, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int b = 0; b < NB2 && b0 + b < DT; b++)
+#pragma unroll
+                        for (int q4 = 0; q4 < 4; q4++) {
+                            const f32x4 dkv = *(const f32x4 *)(dk + 32 * (b0 + b) + 8 * q4);
+#pragma unroll
+                            for (int e = 0; e < 4; e++)
+                                s[4 * q4 + e] = fmaf((float)I[b][4 * q4 + e] * dkv[e], dq[b0 + b], s[4 * q4 + e]);
+                        }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+#pragma unroll
+            for (int ks = 0; ks < (KVT == 1 ? 0 : KS); ks++) {
                 const half8 kf = as_half8(*(const u32x4 *)(k_s + col * KROW + (16 * ks + 8 * h) * 2));
                 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qh[ks], s, 0, 0, 0);
                 s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, ql[ks], s2, 0, 0, 0);
@@ -301,7 +427,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
             if constexpr (KVT == 2) {
 #pragma unroll
                 for (int v = 0; v < 16; v++) s[v] = (s[v] + s2[v]) * fk[8 * (v >> 2) + 4 * h + (v & 3)];
-            } else {
+            } else if constexpr (KVT == 0) {
 #pragma unroll
                 for (int v = 0; v < 16; v++) s[v] = (s[v] + s2[v]) * LOG2E_F;
             }
@@ -374,16 +500,55 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
                     const half8 vf = as_half8(vv);
                     o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, ph[u], o[d], 0, 0, 0);
                     o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pl[u], o[d], 0, 0, 0);
+                    if constexpr (KVT == 1) {  // the values' low halves
+                        const uint2 lo4l = *(const uint2 *)(vrow + HD * VROW + (16 * u + 4 * h) * 2);
+                        const uint2 hi4l = *(const uint2 *)(vrow + HD * VROW + (16 * u + 8 + 4 * h) * 2);
+                        const half8 vfl = as_half8(u32x4{lo4l.x, lo4l.y, hi4l.x, hi4l.y});
+                        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vfl, ph[u], o[d], 0, 0, 0);
+                        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vfl, pl[u], o[d], 0, 0, 0);
+                    }
                 }
             }
         }
         __syncthreads();
     };
-    // an even number of steps (the last one may be idle), so that the loop has one
-    // entry path per register set and every wait count is exact
-    for (int it = 0; it < n_iter; it += 2) {
-        body(it, rb);
-        body(it + 1, ra);
+    auto run = [&]() {
+        m = -INFINITY;
+        l_half = 0.0f;
+#pragma unroll
+        for (int d = 0; d < DT; d++) o[d] = f32x16{};
+        // Loads are issued unconditionally (tile indices past the end repeat the last
+        // tile; an empty split loads tile 0) so that every wait for a register set is an
+        // exact count of the loads issued after it.
+        Regs ra, rb;
+        fetch(min(t_lo + grp, last), ra);
+        stage(ra, 0);
+        fetch(min(t_lo + grp + NW, last), rb);
+        fetch(min(t_lo + grp + 2 * NW, last), ra);
+        __syncthreads();
+        // an even number of steps (the last one may be idle), so that the loop has one
+        // entry path per register set and every wait count is exact
+        for (int it = 0; it < n_iter; it += 2) {
+            body(it, rb);
+            body(it + 1, ra);
+        }
+    };
+    if constexpr (KVT == 1) {
+        if (threadIdx.x < DT) vbig[threadIdx.x] = 0;
+        __syncthreads();
+        for (int again = 0;; again = 1) {
+            run();  // ends with a barrier after the last staging, or stages tile 0 ahead of its only one
+            if (again) break;
+#pragma unroll
+            for (int b = 0; b < DT; b++) vsmall |= (uint32_t)(vbig[b] != 0) << b;
+            if (!vsmall) break;
+            __syncthreads();  // every flag is read before the second run's staging
+        }
+#pragma unroll
+        for (int d = 0; d < DT; d++)
+            if (vsmall >> d & 1) o[d] *= 256.0f;
+    } else {
+        run();
     }
     if constexpr (NW > 1) {  // merge the groups' states into group 0 (the tile buffers are free now)
         float *ms = (float *)lds, *ls = ms + NW * 256, *os = ls + NW * 256;
@@ -612,20 +777,22 @@ __global__ __launch_bounds__(64) void turbo_query_kernel(const float *__restrict
 
 bool attention_prompt_mfma_ok(const AttnArgs &a) {
     const int G = a.n_kv > 0 ? a.n_head / a.n_kv : 0;
-    const bool cache_ok = a.kv_type == 0 || (a.kv_type == 2 && a.hd == 128 && a.turbo_signs && a.k_scale && a.v_scale && a.part);
-    return cache_ok && a.n_tok > 1 && !a.d_pos0 && a.slots >= 32 && (a.hd == 32 || a.hd == 64 || a.hd == 96 || a.hd == 128) && G >= 1 &&
+    const bool cache_ok = a.kv_type == 0 || a.kv_type == 1 || (a.kv_type == 2 && a.hd == 128 && a.turbo_signs && a.k_scale && a.v_scale && a.part);
+    return cache_ok && a.n_tok > 1 && !a.d_pos0 && a.slots >= 32 && (a.hd == 32 || a.hd == 64 || a.hd == 96 || a.hd == 128 || (a.hd == 256 && a.kv_type == 1)) && G >= 1 &&
            G <= 8 && a.n_head == G * a.n_kv && (a.att_fmt != ACT_Q8_0 || (a.att_q.qs && a.att_q.d));
 }
 
-// KV splits of a launch: long rows are split over grid.z workgroups (at least 16
-// tiles of 32 positions each, up to about two workgroups per CU, at most 16) whose
-// partials attn_combine_kernel merges.  Rows under 1024 positions keep one pass:
-// at a 512-token prompt from position 0, two splits (8 tiles each) and the merge
-// launch measured 29.3 k tok/s against 31.1 k.
-static int prompt_kv_splits(const AttnArgs &a, const dim3 &grid) {
-    const int longest = (a.pos0 + a.n_tok - 1) / PT + 1;  // tiles of the last query row (no window)
-    const int by_work = longest / 16, by_grid = 512 / (int)(grid.x * grid.y);
-    return std::max(1, std::min(16, std::min(by_work, by_grid)));
+// KV splits of a launch, merged by a second kernel: at least 16 tiles of 32 positions
+// each, up to about two workgroups per CU, at most 16.  Rows under 1024 positions keep
+// one pass where the grid has 64 workgroups or more: at a 512-token prompt from position
+// 0, two splits (8 tiles each) and the merge launch measured 29.3 k tok/s against 31.1 k
+// (128 workgroups), 80 against 84 k (64).  Smaller grids (a few drafted tokens, one KV
+// head) take splits of at least 4 tiles: 5 tokens at 900, 8 workgroups, 39 us in one pass.
+static int prompt_kv_splits(const AttnArgs &a, const dim3 &grid, int tokens_per_wg) {
+    int longest = (a.pos0 + a.n_tok - 1) / PT + 1;  // tiles of the last query row
+    if (a.window > 0) longest = std::min(longest, (a.window + tokens_per_wg - 2) / PT + 2);
+    const int wgs = (int)(grid.x * grid.y);
+    return std::max({1, std::min({16, longest / 16, 512 / wgs}), std::min({16, longest / 4, 64 / wgs})});
 }
 
 bool launch_attention_prompt_mfma(const AttnArgs &a, hipStream_t st) {
@@ -633,7 +800,7 @@ bool launch_attention_prompt_mfma(const AttnArgs &a, hipStream_t st) {
     const int G = a.n_head / a.n_kv;
     const int wpt = G < 4 ? G : 4, tbw = 4 / wpt, hgroups = (G + 3) / 4;
     dim3 grid((a.n_tok + 32 * tbw - 1) / (32 * tbw), a.n_kv * hgroups);
-    const int S = a.window > 0 ? 1 : prompt_kv_splits(a, grid);
+    const int S = prompt_kv_splits(a, grid, 32 * tbw);
     grid.z = S;
     AttnArgs b = a;
     b.n_split = S;
@@ -644,6 +811,14 @@ bool launch_attention_prompt_mfma(const AttnArgs &a, hipStream_t st) {
         hipLaunchKernelGGL(turbo_query_kernel, dim3(a.n_head, a.n_tok), dim3(64), 0, st, a.q, a.n_head * 128, a.turbo_signs, qhat);
         b.q = qhat;
         launch_nw<128, 2, 2>(b, grid, st);
+    } else if (a.kv_type == 1) {
+        switch (a.hd) {
+        case 32: launch_nw<32, 2, 1>(b, grid, st); break;
+        case 64: launch_nw<64, 2, 1>(b, grid, st); break;
+        case 96: launch_nw<96, 2, 1>(b, grid, st); break;
+        case 128: launch_nw<128, 2, 1>(b, grid, st); break;
+        default: launch_nw<256, 1, 1>(b, grid, st); break;
+        }
     } else {
         switch (a.hd) {
         case 32: launch_nw<32, 2, 0>(b, grid, st); break;
