@@ -14,9 +14,13 @@
 //
 // Workgroup tile: 64 weight rows × 64 tokens, 4 waves as 2 × 2 (32 rows × 32
 // tokens each).  A stage is half a superblock (4 sub-blocks, 128 values): the
-// activation codes, the superblock's activation scale and 32-value sums, the
-// weight nibbles of the half and the row's d, dmin and unpacked 6-bit scales and
-// mins go to LDS; the next stage's global loads are in flight meanwhile.
+// activation codes, the weight nibbles and the half's 6-bit scales go to LDS, with
+// the second half also what the superblock's end reads (activation scale and 32-value
+// sums, d, dmin and mins); the next stage's global loads are in flight meanwhile.
+// The scales and mins are unpacked four to a dword and the min term's operands made
+// once per workgroup: one at a time, in every stage and wave, they were a third of the
+// kernel's vector instructions (421 tokens, gate/up 2 × 8192 × 3072 in Q5_K: 128 us, now
+// 91 us; Q6_K down of 3072 × 8192: 79 us, now 64 us).
 // Operand lane layout as in gemm.hip: lane l supplies row l mod 32 and values
 // 16·(l/32)..+16; tokens are permuted onto the A rows so that lane l's 16
 // results are the 16 consecutive tokens 16·(l/32) + v.
@@ -27,7 +31,7 @@
 // multiply loop reads its B operand without the nibble shifts of Q4_K, for 64 more LDS
 // bytes per row.  Bound like Q4_K by the int32 scale multiply-adds between the MFMAs.
 // A 421-token prompt through two layers of hidden 3072 (Q5_K, V and one down
-// projection Q6_K) takes 905 µs, against 7439 µs with its Q5_K weights in the batched
+// projection Q6_K) takes 768 µs, against 7439 µs with its Q5_K weights in the batched
 // GEMV, which reads and unpacks every weight once per 4 tokens.
 //
 // Q6_K weights × Q8_K activations (kernels/avx2.rs dot_q6_k 109-151): per
@@ -108,20 +112,25 @@ template <int TY> constexpr int kw_st() { return (TY == T_Q5_K ? 128 : 64) + 16;
 template <int TY> constexpr int kq_block() { return TY == T_Q5_K ? 176 : 144; }  // superblock bytes
 template <int TY> constexpr int kq_qs() { return TY == T_Q5_K ? 48 : 16; }       // offset of its nibbles
 
-// BN = 32 keeps the 6-bit scales and mins as bytes, so that two 128-row stages of
-// the gated pair fit two workgroups in a CU's LDS.
+// One half superblock; the sub-block scales stay 6-bit bytes, four to a dword.
 template <int TY, bool GLU, int BN = KQ_BN>
 struct __align__(16) KqStage {
     static constexpr int NW = GLU ? 2 : 1, BM = kq_bm<BN>();
-    using ScT = std::conditional_t<BN == 64, int, uint8_t>;
-    using MnT = std::conditional_t<BN == 64, float, uint8_t>;
     int8_t a[BN * KA_ST];
-    float da[BN];
-    float bs[BN * 8];              // the superblock's 32-value activation sums (both halves hold all 8)
     uint8_t wq[NW][BM * kw_st<TY>()];
+    uint32_t wsc[NW][BM];          // scales of the half's 4 sub-blocks
+};
+
+// What the end of a superblock reads: written with its second half, read in that half.
+// Operands of the min term (see below), made once per workgroup: 8 halves for sub-blocks
+// 0..3 and 8 for 4..7 of each token and row.
+template <bool GLU, int BN = KQ_BN>
+struct __align__(16) KqEnd {
+    static constexpr int NW = GLU ? 2 : 1, BM = kq_bm<BN>();
+    uint4 ab[BN * 2];              // base-64 digits of the tokens' 32-value sums
+    uint4 bb[NW][BM * 2];          // m, 64·m
+    float da[BN];
     float wd[NW][BM], wdm[NW][BM];
-    ScT wsc[NW][BM * 8];           // 6-bit scales of the 8 sub-blocks
-    MnT wm[NW][BM * 8];            // 6-bit mins
 };
 
 template <int TY, bool GLU, int BN = KQ_BN>
@@ -129,7 +138,7 @@ struct KqRegs {
     static constexpr int NA = BN == 64 ? 2 : 1, NQ = (BN == 32 && GLU) ? 4 : 2;
     v4i a[NA];        // 32 (BN 64) or 16 (BN 32) activation bytes of the thread's token
     float da;
-    v4i bs[2];        // the token's 16 bsums (int16)
+    v4i bs;           // 8 of the token's 16 bsums (int16)
     v4i wq[NQ];       // 32 nibble bytes of the thread's row (64, both units, in the 32-token gated form)
     v4i qh[TY == T_Q5_K ? 2 : 1];  // Q5_K: the superblock's 32 bytes of fifth bits
     v4i hdr;          // d, dmin, scales[12]
@@ -137,9 +146,9 @@ struct KqRegs {
 
 // stage loads for half hs of superblock sb
 // tokA: the activation row of the thread's token (tid/4, or tid/8 for BN 32); tokD: of
-// token tid (tid < BN); woff: the expert's byte offset in a grouped launch
-template <int TY, bool GLU, int BN = KQ_BN>
-__device__ __forceinline__ void kq_load(const KqP &p, int sg, int row0, int tokA, int tokD, size_t woff, int sb, int hs, int tid,
+// token tid % BN (tid < 2·BN); woff: the expert's byte offset in a grouped launch
+template <int TY, bool GLU, int BN, int hs>
+__device__ __forceinline__ void kq_load(const KqP &p, int sg, int row0, int tokA, int tokD, size_t woff, int sb, int tid,
                                         KqRegs<TY, GLU, BN> &R) {
     static_assert(TY == T_Q4_K || BN == 64, "32-token tiles serve Q4_K");
     const int K = p.K, nsb = K >> 8;
@@ -150,11 +159,9 @@ __device__ __forceinline__ void kq_load(const KqP &p, int sg, int row0, int tokA
     } else {
         R.a[0] = *(const v4i *)(p.qs + (size_t)tokA * K + 256 * sb + 128 * hs + 16 * (tid & 7));
     }
-    if (tid < BN) {
+    if (hs == 1 && tid < 2 * BN) {
         R.da = p.d[(size_t)tokD * nsb + sb];
-        const v4i *bsrc = (const v4i *)(p.bsums + (size_t)tokD * (K >> 4) + 16 * sb);
-        R.bs[0] = bsrc[0];
-        R.bs[1] = bsrc[1];
+        R.bs = *(const v4i *)(p.bsums + (size_t)tokD * (K >> 4) + 16 * sb + 8 * (tid / BN));
     }
     if constexpr (BN == 32 && GLU) {  // thread → (matrix, row): both units of the half
         const int nw = tid >> 7;
@@ -180,9 +187,11 @@ __device__ __forceinline__ void kq_load(const KqP &p, int sg, int row0, int tokA
     }
 }
 
-// hs: the half that R holds (Q5_K: which of its fifth-bit planes)
-template <int TY, bool GLU, int BN = KQ_BN>
-__device__ __forceinline__ void kq_store(KqStage<TY, GLU, BN> &S, int tid, int hs, const KqRegs<TY, GLU, BN> &R) {
+typedef _Float16 half2k __attribute__((ext_vector_type(2)));
+
+// hs: the half that R holds
+template <int TY, bool GLU, int BN, int hs>
+__device__ __forceinline__ void kq_store(KqStage<TY, GLU, BN> &S, KqEnd<GLU, BN> &E, int tid, const KqRegs<TY, GLU, BN> &R) {
     if constexpr (BN == 64) {
         v4i *dst = (v4i *)(S.a + (tid >> 2) * KA_ST + 32 * (tid & 3));
         dst[0] = R.a[0];
@@ -190,13 +199,16 @@ __device__ __forceinline__ void kq_store(KqStage<TY, GLU, BN> &S, int tid, int h
     } else {
         *(v4i *)(S.a + (tid >> 3) * KA_ST + 16 * (tid & 7)) = R.a[0];
     }
-    if (tid < BN) {
-        S.da[tid] = R.da;
-        const uint32_t w[8] = {(uint32_t)R.bs[0][0], (uint32_t)R.bs[0][1], (uint32_t)R.bs[0][2], (uint32_t)R.bs[0][3],
-                               (uint32_t)R.bs[1][0], (uint32_t)R.bs[1][1], (uint32_t)R.bs[1][2], (uint32_t)R.bs[1][3]};
+    if (hs == 1 && tid < 2 * BN) {
+        if (tid < BN) E.da[tid] = R.da;
+        uint32_t q[4];
 #pragma unroll
-        for (int j = 0; j < 8; j++)  // bsum_2j + bsum_2j+1 = the two int16 halves of dword j
-            S.bs[tid * 8 + j] = (float)((int)(int16_t)(w[j] & 0xffff) + (int)(int16_t)(w[j] >> 16));
+        for (int j = 0; j < 4; j++) {  // bsum_2j + bsum_2j+1 = the two int16 halves of dword j
+            const int bs = (int)(int16_t)(R.bs[j] & 0xffff) + (R.bs[j] >> 16);
+            const half2k d = {(_Float16)(int16_t)(bs & 63), (_Float16)(int16_t)(bs >> 6)};
+            q[j] = __builtin_bit_cast(uint32_t, d);
+        }
+        E.ab[2 * (tid % BN) + tid / BN] = make_uint4(q[0], q[1], q[2], q[3]);
     }
     if (GLU || BN == 32 || tid < 128) {
         int nw, row, u;
@@ -236,16 +248,27 @@ __device__ __forceinline__ void kq_store(KqStage<TY, GLU, BN> &S, int tid, int h
                 dst[1] = R.wq[1];
             }
         }
-        if (u == 0) {
-            const uint32_t h0 = (uint32_t)R.hdr[0], h1 = (uint32_t)R.hdr[1], h2 = (uint32_t)R.hdr[2], h3 = (uint32_t)R.hdr[3];
-            S.wd[nw][row] = h2f(h0 & 0xffff);
-            S.wdm[nw][row] = h2f(h0 >> 16);
+        // get_scale_min_k4 (quant/reference.rs:8-16), four sub-blocks at a time
+        const uint32_t h0 = (uint32_t)R.hdr[0], h1 = (uint32_t)R.hdr[1], h2 = (uint32_t)R.hdr[2], h3 = (uint32_t)R.hdr[3];
+        if (u == 0) S.wsc[nw][row] = hs == 0 ? h1 & 0x3F3F3F3Fu : (h3 & 0x0F0F0F0Fu) | ((h1 >> 2) & 0x30303030u);
+        if (hs == 1) {
+            constexpr bool BOTH = BN == 32 && GLU;  // one thread for the row's two units
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                int sc, mn;
-                q4k_scale_min(h1, h2, h3, j, sc, mn);  // get_scale_min_k4 (quant/reference.rs:8-16)
-                S.wsc[nw][row * 8 + j] = (typename KqStage<TY, GLU, BN>::ScT)sc;
-                S.wm[nw][row * 8 + j] = (typename KqStage<TY, GLU, BN>::MnT)mn;
+            for (int k = 0; k < (BOTH ? 2 : 1); k++) {
+                const int uu = BOTH ? k : u;
+                const uint32_t mn = uu == 0 ? h2 & 0x3F3F3F3Fu : ((h3 >> 4) & 0x0F0F0F0Fu) | ((h2 >> 2) & 0x30303030u);
+                uint32_t q[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {  // 0x6400 | m is the half 1024 + m
+                    const uint32_t b = __builtin_amdgcn_perm(0x64646464u, mn, 0x04000400u | (uint32_t)j | (uint32_t)j << 16);
+                    const half2k v = (__builtin_bit_cast(half2k, b) - half2k{1024, 1024}) * half2k{1, 64};
+                    q[j] = __builtin_bit_cast(uint32_t, v);
+                }
+                E.bb[nw][2 * row + uu] = make_uint4(q[0], q[1], q[2], q[3]);
+            }
+            if (u == 0) {
+                E.wd[nw][row] = h2f(h0 & 0xffff);
+                E.wdm[nw][row] = h2f(h0 >> 16);
             }
         }
     }
@@ -258,10 +281,19 @@ __device__ __forceinline__ void kq_store(KqStage<TY, GLU, BN> &S, int tid, int h
 // result only for instructions it generates itself.
 __device__ __forceinline__ int mad24(int a, int b, int c) { return c + __mul24(a, b); }
 
+// Keeps the 16 sums where they are computed: the compiler otherwise moves a product's
+// multiply-adds past the stage's barrier, to their next use, and splits them into
+// products and three-operand sums.
+__device__ __forceinline__ void pin16(int (&s)[16]) {
+    asm volatile("" : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]), "+v"(s[4]), "+v"(s[5]), "+v"(s[6]), "+v"(s[7]), "+v"(s[8]),
+                 "+v"(s[9]), "+v"(s[10]), "+v"(s[11]), "+v"(s[12]), "+v"(s[13]), "+v"(s[14]), "+v"(s[15]));
+}
+
 template <int TY, bool GLU, int BN = KQ_BN>
 __global__ __launch_bounds__(256) void gemm_q45k_kernel(KqP p) {
     constexpr int NW = GLU ? 2 : 1, BM = kq_bm<BN>(), WC = BN / 32;  // waves along the tokens
     __shared__ KqStage<TY, GLU, BN> st[2];
+    __shared__ KqEnd<GLU, BN> en;
     const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
     const int wr = wv / WC, wc = wv % WC;
     // workgroups of one row group share an XCD (id mod 8); the K splits of one tile
@@ -293,73 +325,78 @@ __global__ __launch_bounds__(256) void gemm_q45k_kernel(KqP p) {
 #pragma unroll
     for (int a = 0; a < NW; a++)
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            acc[a][v] = 0.0f;
-            s1[a][v] = 0;
-        }
-    // this workgroup's superblocks [sb0, sb0 + n_stages / 2) (its K split)
+        for (int v = 0; v < 16; v++) acc[a][v] = 0.0f;
+    // this workgroup's superblocks [sb0, sb1) (its K split)
     const int nsb = p.K >> 8;
-    const int sb0 = KSPLIT ? ksi * nsb / p.ks : 0;
-    const int n_stages = KSPLIT ? ((ksi + 1) * nsb / p.ks - sb0) * 2 : nsb * 2;
+    const int sb0 = KSPLIT ? ksi * nsb / p.ks : 0, sb1 = KSPLIT ? (ksi + 1) * nsb / p.ks : nsb;
     KqRegs<TY, GLU, BN> R;
-    kq_load<TY, GLU, BN>(p, sg, row0, tokA, tokD, woff, sb0, 0, tid, R);
-    kq_store<TY, GLU, BN>(st[0], tid, 0, R);
+    kq_load<TY, GLU, BN, 0>(p, sg, row0, tokA, tokD, woff, sb0, tid, R);
+    kq_store<TY, GLU, BN, 0>(st[0], en, tid, R);
     __syncthreads();
-    for (int s = 0; s < n_stages; s++) {
-        const int hs = s & 1;
-        if (s + 1 < n_stages) kq_load<TY, GLU, BN>(p, sg, row0, tokA, tokD, woff, sb0 + ((s + 1) >> 1), (s + 1) & 1, tid, R);
-        const KqStage<TY, GLU, BN> &S = st[s & 1];
+    auto half = [&](int sb, auto hc) {
+        constexpr int hs = decltype(hc)::value;
+        const bool more = hs == 0 || sb + 1 < sb1;
+        if (more) kq_load<TY, GLU, BN, 1 - hs>(p, sg, row0, tokA, tokD, woff, sb + hs, tid, R);
+        const KqStage<TY, GLU, BN> &S = st[hs];
+        uint32_t scw[NW];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const v4i av = *(const v4i *)(S.a + arow * KA_ST + 32 * j + 16 * h);
+        for (int a = 0; a < NW; a++) scw[a] = S.wsc[a][wrow];
+        // all operands of the half, then its 4·NW products with the MFMA of product q + 1
+        // issued ahead of the multiply-adds of q; the fences keep it so (left alone, the
+        // scheduler issues every MFMA first, at 250 to 490 registers)
+        constexpr int NQ = TY == T_Q5_K ? 4 : 2;
+        v4i av[4], wq[NW][NQ];
 #pragma unroll
-            for (int a = 0; a < NW; a++) {
-                v4i bw;
-                if constexpr (TY == T_Q5_K) {
-                    bw = *(const v4i *)(S.wq[a] + wrow * kw_st<TY>() + 32 * j + 16 * h);
-                } else {
-                    const uint4 q = *(const uint4 *)(S.wq[a] + wrow * kw_st<TY>() + 32 * (j >> 1) + 16 * h);
-                    const uint32_t sh = 4u * (uint32_t)(j & 1);
-                    bw = v4i{(int)((q.x >> sh) & 0x0F0F0F0Fu), (int)((q.y >> sh) & 0x0F0F0F0Fu), (int)((q.z >> sh) & 0x0F0F0F0Fu),
-                             (int)((q.w >> sh) & 0x0F0F0F0Fu)};
-                }
-                const v16i I = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, bw, zi, 0, 0, 0);
-                const int sc = (int)S.wsc[a][wrow * 8 + 4 * hs + j];  // |sc| < 64, |I| < 2^17
+        for (int j = 0; j < 4; j++) av[j] = *(const v4i *)(S.a + arow * KA_ST + 32 * j + 16 * h);
 #pragma unroll
-                for (int v = 0; v < 16; v++) s1[a][v] = mad24(sc, I[v], s1[a][v]);
-            }
+        for (int a = 0; a < NW; a++)
+#pragma unroll
+            for (int j = 0; j < NQ; j++) wq[a][j] = *(const v4i *)(S.wq[a] + wrow * kw_st<TY>() + 32 * j + 16 * h);
+        v16i I[2];
+        auto issue = [&](int q) {
+            const int j = q / NW, a = q % NW;
+            v4i bw;
+            if constexpr (TY == T_Q5_K) bw = wq[a][j];
+            else
+#pragma unroll
+                for (int i = 0; i < 4; i++) bw[i] = (int)(((uint32_t)wq[a][j >> 1][i] >> (4 * (j & 1))) & 0x0F0F0F0Fu);
+            I[q & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[j], bw, zi, 0, 0, 0);
+        };
+        issue(0);
+#pragma unroll
+        for (int q = 0; q < 4 * NW; q++) {
+            if (q + 1 < 4 * NW) issue(q + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            const int j = q / NW, a = q % NW;
+            const int sc = (int)(scw[a] >> (8 * j) & 0xff);  // sc < 64, |I| < 2^17
+#pragma unroll
+            for (int v = 0; v < 16; v++) s1[a][v] = hs == 0 && j == 0 ? __mul24(sc, I[q & 1][v]) : mad24(sc, I[q & 1][v], s1[a][v]);
+            pin16(s1[a]);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if (hs == 1) {  // end of the superblock: the min term and the two scale products
+        if constexpr (hs == 1) {  // end of the superblock: the min term and the two scale products
+            const half8k ab = __builtin_bit_cast(half8k, en.ab[2 * arow + h]);
 #pragma unroll
             for (int a = 0; a < NW; a++) {
                 // Σ_j m_j·bs_j exactly on one f16 MFMA: k-slots 2j, 2j + 1 hold the base-64
                 // digits of the block sum (bs = 64·hi + lo, |bs| ≤ 32·127) against m_j and
                 // 64·m_j; every product and partial sum is an integer below 2^24.  Lane half h
                 // supplies sub-blocks 4h..4h+3.
-                half8k ab, bb;
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const int j = 4 * h + q;
-                    const int bsj = (int)S.bs[arow * 8 + j];
-                    const float mj = (float)S.wm[a][wrow * 8 + j];
-                    ab[2 * q] = (_Float16)(float)(bsj & 63);
-                    ab[2 * q + 1] = (_Float16)(float)(bsj >> 6);
-                    bb[2 * q] = (_Float16)mj;
-                    bb[2 * q + 1] = (_Float16)(64.0f * mj);
-                }
+                const half8k bb = __builtin_bit_cast(half8k, en.bb[a][2 * wrow + h]);
                 const v16f s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ab, bb, zf, 0, 0, 0);
                 // d·d_a and dmin·d_a in one two-block outer product (block 0: lanes 0-31, d;
                 // block 1: lanes 32-63, dmin)
-                const v32f pp = __builtin_amdgcn_mfma_f32_32x32x1f32(S.da[arow], h == 0 ? S.wd[a][wrow] : S.wdm[a][wrow], zf32, 0, 0, 0);
+                const v32f pp = __builtin_amdgcn_mfma_f32_32x32x1f32(en.da[arow], h == 0 ? en.wd[a][wrow] : en.wdm[a][wrow], zf32, 0, 0, 0);
 #pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    acc[a][v] += pp[v] * (float)s1[a][v] - pp[16 + v] * s2[v];
-                    s1[a][v] = 0;
-                }
+                for (int v = 0; v < 16; v++) acc[a][v] = fmaf(pp[v], (float)s1[a][v], fmaf(-pp[16 + v], s2[v], acc[a][v]));
             }
         }
-        if (s + 1 < n_stages) kq_store<TY, GLU, BN>(st[(s + 1) & 1], tid, (s + 1) & 1, R);
+        if (more) kq_store<TY, GLU, BN, 1 - hs>(st[1 - hs], en, tid, R);
         __syncthreads();
+    };
+    for (int sb = sb0; sb < sb1; sb++) {
+        half(sb, std::integral_constant<int, 0>{});
+        half(sb, std::integral_constant<int, 1>{});
     }
     // ---- epilogue: lane holds weight row row0 + wrow for tokens t0 + wc·32 + 16h + v ----
     const int rows = p.rows[sg];
@@ -384,21 +421,27 @@ __global__ __launch_bounds__(256) void gemm_q45k_kernel(KqP p) {
 // ---- Q6_K ----------------------------------------------------------------
 constexpr int K6_ST = 128 + 16;  // weight code bytes per row in LDS (one half superblock, padded)
 
+// Codes lie in 8-byte groups in the order 0, 2, 1, 3 of each 32 values, so that a lane
+// half's groups of two 16-value sub-blocks are one 16-byte read.
 template <bool GLU>
 struct __align__(16) K6Stage {
     static constexpr int NW = GLU ? 2 : 1;
     int8_t a[KQ_BN * KA_ST];
+    int8_t wq[NW][KQ_BM * K6_ST];  // q6 − 32 of the half
+    uint2 wsc[NW][KQ_BM];          // the half's 8 signed sub-block scales
+};
+template <bool GLU>
+struct K6End {  // scales of the superblock: written with its second half, read in that half
     float da[KQ_BN];
-    int8_t wq[NW][KQ_BM * K6_ST];  // q6 − 32 of the half, in value order
-    float wd[NW][KQ_BM];
-    int wsc[NW][KQ_BM * 8];        // the half's 8 signed sub-block scales
+    float wd[GLU ? 2 : 1][KQ_BM];
 };
 
-struct K6W {  // one weight row's part of a half superblock
-    uint32_t lo[3], hi[3], qh[3];  // 8 bytes each from a 2-byte aligned address (+1 dword)
-    uint32_t sc[3];                // the half's 8 scale bytes
+struct __attribute__((packed, aligned(2))) K6B8 {
+    uint32_t w[2];
+};
+struct K6W {  // one weight row's part of a half superblock: 8 bytes each from a 2-byte boundary
+    K6B8 lo, hi, qh, sc;
     uint32_t d;
-    uint32_t sh_l, sh_h, sh_q, sh_s;
 };
 
 template <bool GLU>
@@ -408,80 +451,62 @@ struct K6Regs {
     K6W w[GLU ? 2 : 1];
 };
 
-// 3 dwords from the dword-aligned address at or below p; sh = p's offset in the first
-__device__ __forceinline__ void ld3_a2(const uint8_t *p, uint32_t (&w)[3], uint32_t &sh) {
-    const uintptr_t a = (uintptr_t)p;
-    const uint32_t *q = (const uint32_t *)(a & ~(uintptr_t)3);
-    sh = (uint32_t)(a & 3);
-#pragma unroll
-    for (int i = 0; i < 3; i++) w[i] = wload(q + i);
-}
-
 // thread → (row tid/4, part tid%4): values l + 32i of the half, l in 8·part..+8, i = 0..3
-template <bool GLU>
-__device__ __forceinline__ void k6_load(const KqP &p, int sg, int row0, int tokA, int tokD, size_t woff, int sb, int hs, int tid,
-                                        K6Regs<GLU> &R) {
+template <bool GLU, int hs>
+__device__ __forceinline__ void k6_load(const KqP &p, int sg, int row0, int tokA, int tokD, size_t woff, int sb, int tid, K6Regs<GLU> &R) {
     const int K = p.K, nsb = K >> 8;
     {
         const v4i *src = (const v4i *)(p.qs + (size_t)tokA * K + 256 * sb + 128 * hs + 32 * (tid & 3));
         R.a[0] = src[0];
         R.a[1] = src[1];
     }
-    if (tid < KQ_BN) R.da = p.d[(size_t)tokD * nsb + sb];
+    if (hs == 1 && tid < KQ_BN) R.da = p.d[(size_t)tokD * nsb + sb];
     const int row = min(row0 + (tid >> 2), p.rows[GLU ? 0 : sg] - 1), part = tid & 3;
 #pragma unroll
     for (int a = 0; a < (GLU ? 2 : 1); a++) {
         const int s = GLU ? a : sg;
         K6W &w = R.w[a];
         const uint8_t *blk = p.w[s] + woff + (size_t)row * p.rb[s] + 210 * (size_t)sb;
-        ld3_a2(blk + 64 * hs + 8 * part, w.lo, w.sh_l);
-        ld3_a2(blk + 64 * hs + 32 + 8 * part, w.hi, w.sh_h);
-        ld3_a2(blk + 128 + 32 * hs + 8 * part, w.qh, w.sh_q);
+        w.lo = *(const K6B8 *)(blk + 64 * hs + 8 * part);
+        w.hi = *(const K6B8 *)(blk + 64 * hs + 32 + 8 * part);
+        w.qh = *(const K6B8 *)(blk + 128 + 32 * hs + 8 * part);
         if (part == 0) {
-            ld3_a2(blk + 192 + 8 * hs, w.sc, w.sh_s);
-            w.d = wload((const uint16_t *)(blk + 208));
+            w.sc = *(const K6B8 *)(blk + 192 + 8 * hs);
+            if (hs == 1) w.d = *(const uint16_t *)(blk + 208);
         }
     }
 }
 
-template <bool GLU>
-__device__ __forceinline__ void k6_store(K6Stage<GLU> &S, int tid, const K6Regs<GLU> &R) {
+template <bool GLU, int hs>
+__device__ __forceinline__ void k6_store(K6Stage<GLU> &S, K6End<GLU> &E, int tid, const K6Regs<GLU> &R) {
     {
         v4i *dst = (v4i *)(S.a + (tid >> 2) * KA_ST + 32 * (tid & 3));
-        dst[0] = R.a[0];
-        dst[1] = R.a[1];
+        dst[0] = v4i{R.a[0][0], R.a[0][1], R.a[1][0], R.a[1][1]};
+        dst[1] = v4i{R.a[0][2], R.a[0][3], R.a[1][2], R.a[1][3]};
     }
-    if (tid < KQ_BN) S.da[tid] = R.da;
+    if (hs == 1 && tid < KQ_BN) E.da[tid] = R.da;
     const int row = tid >> 2, part = tid & 3;
 #pragma unroll
     for (int a = 0; a < (GLU ? 2 : 1); a++) {
         const K6W &R6 = R.w[a];
-        const uint32_t lo[2] = {__builtin_amdgcn_alignbyte(R6.lo[1], R6.lo[0], R6.sh_l), __builtin_amdgcn_alignbyte(R6.lo[2], R6.lo[1], R6.sh_l)};
-        const uint32_t hi[2] = {__builtin_amdgcn_alignbyte(R6.hi[1], R6.hi[0], R6.sh_h), __builtin_amdgcn_alignbyte(R6.hi[2], R6.hi[1], R6.sh_h)};
-        const uint32_t qh[2] = {__builtin_amdgcn_alignbyte(R6.qh[1], R6.qh[0], R6.sh_q), __builtin_amdgcn_alignbyte(R6.qh[2], R6.qh[1], R6.sh_q)};
         // value l + 32i: low nibble of ql[l] (i = 0), ql[l + 32] (i = 1), high nibbles (i = 2, 3);
         // bits 2i, 2i+1 of qh[l] on top (quant/reference.rs:190-212).  Four codes per dword:
         // (q | 0x80) − 32, then bit 7 flipped back, is the int8 q − 32 without cross-byte borrows.
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const uint32_t *src = (i & 1) ? hi : lo;
+            const uint32_t *src = (i & 1) ? R6.hi.w : R6.lo.w;
             const int sl = 4 * (i >> 1), sq = 2 * i;
             uint32_t w[2];
 #pragma unroll
             for (int k = 0; k < 2; k++) {
-                const uint32_t q = ((src[k] >> sl) & 0x0F0F0F0Fu) | (((qh[k] >> sq) & 0x03030303u) << 4);
+                const uint32_t q = ((src[k] >> sl) & 0x0F0F0F0Fu) | (((R6.qh.w[k] >> sq) & 0x03030303u) << 4);
                 w[k] = ((q | 0x80808080u) - 0x20202020u) ^ 0x80808080u;
             }
-            *(uint2 *)(S.wq[a] + row * K6_ST + 32 * i + 8 * part) = make_uint2(w[0], w[1]);
+            *(uint2 *)(S.wq[a] + row * K6_ST + 32 * i + 16 * (part & 1) + 8 * (part >> 1)) = make_uint2(w[0], w[1]);
         }
         if (part == 0) {
-            const uint32_t s0 = __builtin_amdgcn_alignbyte(R6.sc[1], R6.sc[0], R6.sh_s), s1 = __builtin_amdgcn_alignbyte(R6.sc[2], R6.sc[1], R6.sh_s);
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                S.wsc[a][row * 8 + k] = (int)(int8_t)(s0 >> (8 * k));
-                S.wsc[a][row * 8 + 4 + k] = (int)(int8_t)(s1 >> (8 * k));
-            }
-            S.wd[a][row] = h2f(R6.d);
+            S.wsc[a][row] = make_uint2(R6.sc.w[0], R6.sc.w[1]);
+            if (hs == 1) E.wd[a][row] = h2f(R6.d);
         }
     }
 }
@@ -490,6 +515,7 @@ template <bool GLU>
 __global__ __launch_bounds__(256) void gemm_q6k_kernel(KqP p) {
     constexpr int NW = GLU ? 2 : 1;
     __shared__ K6Stage<GLU> st[2];
+    __shared__ K6End<GLU> en;
     const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
     const int wr = wv >> 1, wc = wv & 1;
     // workgroups of one row group share an XCD (id mod 8); the K splits of one tile
@@ -518,47 +544,62 @@ __global__ __launch_bounds__(256) void gemm_q6k_kernel(KqP p) {
 #pragma unroll
     for (int a = 0; a < NW; a++)
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            acc[a][v] = 0.0f;
-            s1[a][v] = 0;
-        }
-    // this workgroup's superblocks [sb0, sb0 + n_stages / 2) (its K split)
+        for (int v = 0; v < 16; v++) acc[a][v] = 0.0f;
+    // this workgroup's superblocks [sb0, sb1) (its K split)
     const int nsb = p.K >> 8;
-    const int sb0 = ksi * nsb / p.ks;
-    const int n_stages = ((ksi + 1) * nsb / p.ks - sb0) * 2;
+    const int sb0 = ksi * nsb / p.ks, sb1 = (ksi + 1) * nsb / p.ks;
     K6Regs<GLU> R;
-    k6_load<GLU>(p, sg, row0, tokA, tokD, woff, sb0, 0, tid, R);
-    k6_store<GLU>(st[0], tid, R);
+    k6_load<GLU, 0>(p, sg, row0, tokA, tokD, woff, sb0, tid, R);
+    k6_store<GLU, 0>(st[0], en, tid, R);
     __syncthreads();
-    for (int s = 0; s < n_stages; s++) {
-        const int hs = s & 1;
-        if (s + 1 < n_stages) k6_load<GLU>(p, sg, row0, tokA, tokD, woff, sb0 + ((s + 1) >> 1), (s + 1) & 1, tid, R);
-        const K6Stage<GLU> &S = st[s & 1];
+    auto half = [&](int sb, auto hc) {
+        constexpr int hs = decltype(hc)::value;
+        const bool more = hs == 0 || sb + 1 < sb1;
+        if (more) k6_load<GLU, 1 - hs>(p, sg, row0, tokA, tokD, woff, sb + hs, tid, R);
+        const K6Stage<GLU> &S = st[hs];
+        // operands of the half, then its 8·NW products, as in gemm_q45k_kernel
+        v4i av[4], bw[NW][4];
+        uint2 scw[NW];
 #pragma unroll
-        for (int k = 0; k < 8; k++) {  // 16-value sub-blocks of the half
-            const long av = *(const long *)(S.a + arow * KA_ST + 16 * k + 8 * h);
+        for (int k = 0; k < 4; k++) av[k] = *(const v4i *)(S.a + arow * KA_ST + 32 * k + 16 * h);
+#pragma unroll
+        for (int a = 0; a < NW; a++) {
+            scw[a] = S.wsc[a][wrow];
+#pragma unroll
+            for (int k = 0; k < 4; k++) bw[a][k] = *(const v4i *)(S.wq[a] + wrow * K6_ST + 32 * k + 16 * h);
+        }
+        auto sub8 = [](const v4i &v, int k) { return (long)(((uint64_t)(uint32_t)v[2 * k + 1] << 32) | (uint32_t)v[2 * k]); };
+        v16i D[2];
+        auto issue = [&](int q) {
+            const int k = q / NW, a = q % NW;  // 16-value sub-block k of the half
+            D[q & 1] = __builtin_amdgcn_mfma_i32_32x32x16_i8(sub8(av[k >> 1], k & 1), sub8(bw[a][k >> 1], k & 1), zi, 0, 0, 0);
+        };
+        issue(0);
+#pragma unroll
+        for (int q = 0; q < 8 * NW; q++) {
+            if (q + 1 < 8 * NW) issue(q + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            const int k = q / NW, a = q % NW;
+            const int sc = (int)(int8_t)((k < 4 ? scw[a].x : scw[a].y) >> (8 * (k & 3)));
+#pragma unroll
+            for (int v = 0; v < 16; v++) s1[a][v] = hs == 0 && k == 0 ? __mul24(sc, D[q & 1][v]) : mad24(sc, D[q & 1][v], s1[a][v]);
+            pin16(s1[a]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (hs == 1) {  // end of the superblock: (d_r·d_t)·Σ sc·D
 #pragma unroll
             for (int a = 0; a < NW; a++) {
-                const long bw = *(const long *)(S.wq[a] + wrow * K6_ST + 16 * k + 8 * h);
-                const v16i D = __builtin_amdgcn_mfma_i32_32x32x16_i8(av, bw, zi, 0, 0, 0);
-                const int sc = S.wsc[a][wrow * 8 + k];
+                const v16f p1 = __builtin_amdgcn_mfma_f32_32x32x2f32(h == 0 ? en.da[arow] : 0.0f, h == 0 ? en.wd[a][wrow] : 0.0f, zf, 0, 0, 0);
 #pragma unroll
-                for (int v = 0; v < 16; v++) s1[a][v] = mad24(sc, D[v], s1[a][v]);
+                for (int v = 0; v < 16; v++) acc[a][v] = fmaf(p1[v], (float)s1[a][v], acc[a][v]);
             }
         }
-        if (hs == 1) {  // end of the superblock: (d_r·d_t)·Σ sc·D
-#pragma unroll
-            for (int a = 0; a < NW; a++) {
-                const v16f p1 = __builtin_amdgcn_mfma_f32_32x32x2f32(h == 0 ? S.da[arow] : 0.0f, h == 0 ? S.wd[a][wrow] : 0.0f, zf, 0, 0, 0);
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    acc[a][v] = fmaf(p1[v], (float)s1[a][v], acc[a][v]);
-                    s1[a][v] = 0;
-                }
-            }
-        }
-        if (s + 1 < n_stages) k6_store<GLU>(st[(s + 1) & 1], tid, R);
+        if (more) k6_store<GLU, 1 - hs>(st[1 - hs], en, tid, R);
         __syncthreads();
+    };
+    for (int sb = sb0; sb < sb1; sb++) {
+        half(sb, std::integral_constant<int, 0>{});
+        half(sb, std::integral_constant<int, 1>{});
     }
     const int rows = p.rows[sg];
     const int row = row0 + wrow;
