@@ -180,6 +180,28 @@ __device__ __forceinline__ void load32_a2(const uint8_t *p, uint32_t out[8]) {
     for (int i = 0; i < 8; i++) out[i] = __builtin_amdgcn_alignbyte(w[i + 1], w[i], sh);
 }
 
+// Workgroup of a prompt GEMM → row group, token tile and K split; rg < 0: no tile.  The
+// hardware hands workgroups out round the 8 XCDs (id mod 8).  Each XCD takes a
+// contiguous eighth of the tiles in row-group order, so that a row group's weights go
+// through one L2 and the XCDs have equal shares (row groups round the XCDs left two of
+// them idle at 6 row groups).  Expert groupings deal their token tiles round the XCDs
+// instead: a table may hold fewer tiles than the grid, and few experts have a second.
+struct GemmTile {
+    int rg, tg, ks;
+};
+__device__ __forceinline__ GemmTile gemm_tile(int id, int n_rg, int n_tg, int ks, bool grouped) {
+    const int xcd = id & 7, u = id >> 3;
+    if (grouped) {
+        const int tg = (u / n_rg) * 8 + xcd;
+        return GemmTile{tg < n_tg ? u % n_rg : -1, tg, 0};
+    }
+    const int total = n_rg * n_tg * ks, i = xcd * ((total + 7) / 8) + u;
+    return GemmTile{u < (total + 7) / 8 && i < total ? i / ks / n_tg : -1, i / ks % n_tg, i % ks};
+}
+inline int gemm_grid(int n_rg, int n_tg, int ks, bool grouped) {
+    return grouped ? (n_tg + 7) / 8 * 8 * n_rg : (n_rg * n_tg * ks + 7) / 8 * 8;
+}
+
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + expf(-x)); }
 
 __device__ __forceinline__ float gelu_tanh_f(float x) {

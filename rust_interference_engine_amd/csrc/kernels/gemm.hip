@@ -204,14 +204,9 @@ __global__ __launch_bounds__(256, (!GLU && NT == 1) ? 3 : 2) void gemm_kernel(Ge
     const int tid = threadIdx.x;
     const int wv = tid >> 6, l = tid & 63;
     const int wr = wv >> 1, wc = wv & 1;
-    // workgroups of one row group share an XCD (id mod 8) and are dispatched together
-    // (the K splits of one tile are neighbours in u: the same XCD)
-    const int bid = blockIdx.x;
-    const int xcd = bid & 7, uk = bid >> 3;
-    const int ksi = uk % p.ks, u = uk / p.ks;
-    const int tg = u % p.n_tg;
-    const int rg = (u / p.n_tg) * 8 + xcd;
-    if (rg >= p.n_rg) return;  // whole workgroup: uniform
+    const GemmTile gt = gemm_tile(blockIdx.x, p.n_rg, p.n_tg, p.ks, p.grouped);
+    const int rg = gt.rg, tg = gt.tg, ksi = gt.ks;
+    if (rg < 0) return;  // whole workgroup: uniform
     const int sg = (!GLU && p.nseg > 1 && rg >= p.rg_end[0]) ? ((p.nseg > 2 && rg >= p.rg_end[1]) ? 2 : 1) : 0;
     const int row0 = (rg - (sg ? p.rg_end[sg - 1] : 0)) * G_BM;
     const GTileRows tr = gtile_rows(p, tg, BN);
@@ -368,8 +363,7 @@ __global__ __launch_bounds__(256) void gemm_add_parts_kernel(float *__restrict__
 // stages) while part holds the extra splits' partial sums (part_cap floats).
 template <int TY, bool GLU>
 static void launch_t(GemmP p, hipStream_t st, const GroupTiles *grp, float *part, size_t part_cap) {
-    const int slots = (p.n_rg + 7) / 8;
-    const int tiles128 = slots * 8 * ((p.n_tok + 127) / 128);
+    const int tiles128 = p.n_rg * ((p.n_tok + 127) / 128);
     const int n_st = p.K / (32 * G_KC);
     p.ks = 1;
     if (!GLU && !grp && p.nseg == 1 && part && n_st >= 48 && p.n_tok > 64) {
@@ -388,7 +382,7 @@ static void launch_t(GemmP p, hipStream_t st, const GroupTiles *grp, float *part
         p.grp = *grp;
         p.n_tg = grp->max_tiles;
     }
-    const dim3 grid(slots * 8 * p.n_tg * p.ks);
+    const dim3 grid(gemm_grid(p.n_rg, p.n_tg, p.ks, p.grouped));
     if constexpr (!GLU) {
         if (nt == 2) hipLaunchKernelGGL((gemm_kernel<TY, GLU, 2>), grid, dim3(256), 0, st, p);
         else hipLaunchKernelGGL((gemm_kernel<TY, GLU, 1>), grid, dim3(256), 0, st, p);

@@ -203,11 +203,9 @@ __global__ __launch_bounds__(256, 3) void gemm_float_kernel(FGemmP p) {
     __shared__ Stage st[2];
     const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, h = l >> 5, m = l & 31;
     const int wr = wv >> 1, wc = wv & 1;
-    // a row tile's token tiles and K splits share an XCD (id mod 8): its weights are
-    // read from HBM once
-    const int xcd = blockIdx.x & 7, u = blockIdx.x >> 3;
-    const int tt = u % p.n_tt, ksi = u / p.n_tt % p.ks, rt = (u / p.n_tt / p.ks) * 8 + xcd;
-    if (rt >= p.n_rt) return;  // whole workgroup
+    const GemmTile gt = gemm_tile(blockIdx.x, p.n_rt, p.n_tt, p.ks, false);
+    const int rt = gt.rg, tt = gt.tg, ksi = gt.ks;
+    if (rt < 0) return;  // whole workgroup
     const int sg = (!GLU && p.nseg > 1 && rt >= p.rt_end[0]) ? ((p.nseg > 2 && rt >= p.rt_end[1]) ? 2 : 1) : 0;
     const int row0 = (rt - (sg ? p.rt_end[sg - 1] : 0)) * (GLU ? F_BM / 2 : F_BM);
     const int rows = p.rows[sg], t0 = tt * BN, K = p.K;
@@ -345,7 +343,7 @@ __global__ __launch_bounds__(256) void gemm_float_sum_kernel(FGemmP p) {
 
 template <int TY, bool GLU>
 void launch_ty(const FGemmP &p, hipStream_t st) {
-    const dim3 grid((p.n_rt + 7) / 8 * 8 * p.n_tt * p.ks);
+    const dim3 grid(gemm_grid(p.n_rt, p.n_tt, p.ks, false));
     hipLaunchKernelGGL((gemm_float_kernel<TY, GLU>), grid, dim3(256), 0, st, p);
     if (p.ks > 1) hipLaunchKernelGGL(gemm_float_sum_kernel, dim3((p.part_ld + 255) / 256, p.n_tok), dim3(256), 0, st, p);
 }

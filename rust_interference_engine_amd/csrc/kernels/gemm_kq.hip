@@ -296,15 +296,10 @@ __global__ __launch_bounds__(256) void gemm_q45k_kernel(KqP p) {
     __shared__ KqEnd<GLU, BN> en;
     const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
     const int wr = wv / WC, wc = wv % WC;
-    // workgroups of one row group share an XCD (id mod 8); the K splits of one tile
-    // (non-gated 64-token tiles only) are neighbours in u (the same XCD)
     constexpr bool KSPLIT = !GLU && BN == 64;
-    const int bid = blockIdx.x;
-    const int xcd = bid & 7, uk = bid >> 3;
-    const int ksi = KSPLIT ? uk % p.ks : 0, u = KSPLIT ? uk / p.ks : uk;
-    const int tg = u % p.n_tg;
-    const int rg = (u / p.n_tg) * 8 + xcd;
-    if (rg >= p.n_rg) return;  // whole workgroup: uniform
+    const GemmTile gt = gemm_tile(blockIdx.x, p.n_rg, p.n_tg, KSPLIT ? p.ks : 1, p.grouped);
+    const int rg = gt.rg, tg = gt.tg, ksi = gt.ks;
+    if (rg < 0) return;  // whole workgroup: uniform
     const int sg = (!GLU && p.nseg > 1 && rg >= p.rg_end[0]) ? ((p.nseg > 2 && rg >= p.rg_end[1]) ? 2 : 1) : 0;
     const int row0 = (rg - (sg ? p.rg_end[sg - 1] : 0)) * BM;
     const TileRows tr = tile_rows<BN>(p, tg);
@@ -518,14 +513,9 @@ __global__ __launch_bounds__(256) void gemm_q6k_kernel(KqP p) {
     __shared__ K6End<GLU> en;
     const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
     const int wr = wv >> 1, wc = wv & 1;
-    // workgroups of one row group share an XCD (id mod 8); the K splits of one tile
-    // are neighbours in u (the same XCD)
-    const int bid = blockIdx.x;
-    const int xcd = bid & 7, uk = bid >> 3;
-    const int ksi = uk % p.ks, u = uk / p.ks;
-    const int tg = u % p.n_tg;
-    const int rg = (u / p.n_tg) * 8 + xcd;
-    if (rg >= p.n_rg) return;  // whole workgroup: uniform
+    const GemmTile gt = gemm_tile(blockIdx.x, p.n_rg, p.n_tg, p.ks, p.grouped);
+    const int rg = gt.rg, tg = gt.tg, ksi = gt.ks;
+    if (rg < 0) return;  // whole workgroup: uniform
     const int sg = (!GLU && p.nseg > 1 && rg >= p.rg_end[0]) ? ((p.nseg > 2 && rg >= p.rg_end[1]) ? 2 : 1) : 0;
     const int row0 = (rg - (sg ? p.rg_end[sg - 1] : 0)) * KQ_BM;
     const TileRows tr = tile_rows(p, tg);
@@ -638,8 +628,7 @@ void kq_groups(KqP &p, int nseg, const GroupTiles *grp, int bm = KQ_BM) {
 // The non-gated 64-token form splits K as k6_launch does (below).
 template <int TY, bool GLU, int BN = KQ_BN>
 void kq_launch(KqP p, hipStream_t st, float *part = nullptr, size_t part_cap = 0) {
-    const int slots = (p.n_rg + 7) / 8;
-    const int tiles = slots * 8 * p.n_tg, nsb = p.K >> 8;
+    const int tiles = p.n_rg * p.n_tg, nsb = p.K >> 8;
     p.ks = 1;
     if (!GLU && BN == 64 && !p.grouped && p.nseg == 1 && part && p.n_tok > 64) {
         const size_t plane = (size_t)p.n_tok * p.ld[0];
@@ -647,7 +636,7 @@ void kq_launch(KqP p, hipStream_t st, float *part = nullptr, size_t part_cap = 0
         p.part = part;
         p.part_stride = plane;
     }
-    hipLaunchKernelGGL((gemm_q45k_kernel<TY, GLU, BN>), dim3(tiles * p.ks), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((gemm_q45k_kernel<TY, GLU, BN>), dim3(gemm_grid(p.n_rg, p.n_tg, p.ks, p.grouped)), dim3(256), 0, st, p);
     if (p.ks > 1) launch_gemm_add_parts(p.out[0], p.part, p.part_stride, p.ks - 1, p.rows[0], p.ld[0], p.n_tok, st);
 }
 
@@ -656,8 +645,7 @@ void kq_launch(KqP p, hipStream_t st, float *part = nullptr, size_t part_cap = 0
 // (part_cap floats); the partials are added by a second launch.
 template <bool GLU>
 void k6_launch(KqP p, hipStream_t st, float *part = nullptr, size_t part_cap = 0) {
-    const int slots = (p.n_rg + 7) / 8;
-    const int tiles = slots * 8 * p.n_tg, nsb = p.K >> 8;
+    const int tiles = p.n_rg * p.n_tg, nsb = p.K >> 8;
     p.ks = 1;
     if (!GLU && !p.grouped && p.nseg == 1 && part && p.n_tok > 64) {
         const size_t plane = (size_t)p.n_tok * p.ld[0];
@@ -665,7 +653,7 @@ void k6_launch(KqP p, hipStream_t st, float *part = nullptr, size_t part_cap = 0
         p.part = part;
         p.part_stride = plane;
     }
-    hipLaunchKernelGGL((gemm_q6k_kernel<GLU>), dim3(tiles * p.ks), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((gemm_q6k_kernel<GLU>), dim3(gemm_grid(p.n_rg, p.n_tg, p.ks, p.grouped)), dim3(256), 0, st, p);
     if (p.ks > 1) launch_gemm_add_parts(p.out[0], p.part, p.part_stride, p.ks - 1, p.rows[0], p.ld[0], p.n_tok, st);
 }
 
