@@ -220,6 +220,13 @@ HipBackend::HipBackend(const uint8_t *gguf, size_t len, const BackendConfig &cfg
     const size_t nu = std::max<size_t>(n_used_max_, 1);
     d_h_ = dalloc<float>(allocs_, mb * ff_max_ * nu);
     d_logits_ = dalloc<float>(allocs_, mb * c.n_vocab);
+    // one row, and the rows of a short or small-vocabulary call up to 1 MiB
+    h_out_cap_ = std::max(c.n_vocab, std::min<size_t>(mb * c.n_vocab, (size_t)1 << 18));
+    h_out_cap_ = (h_out_cap_ + 15) / 16 * 16;
+    RIE_HIP_CHECK(hipHostMalloc((void **)&h_out_, h_out_cap_ * 4 + 64, hipHostMallocCoherent));
+    h_flag_ = (uint32_t *)(h_out_ + h_out_cap_);
+    *h_flag_ = 0;
+    d_out_cnt_ = dalloc<int>(allocs_, 1);
     const size_t kq = mb * kmax_ * nu;
     act0_.qs = dalloc<int8_t>(allocs_, kq);
     act0_.d = dalloc<float>(allocs_, kq / 32);
@@ -274,6 +281,7 @@ HipBackend::~HipBackend() {
         }
     for (void *p : allocs_) (void)hipFree(p);
     if (d_blob_) (void)hipFree(d_blob_);
+    if (h_out_) (void)hipHostFree(h_out_);
     if (st_) (void)hipStreamDestroy(st_);
 }
 
@@ -845,24 +853,46 @@ void HipBackend::forward(const uint32_t *tokens, size_t n, size_t pos, bool all_
     const size_t m = all_logits ? n : 1;
     if (logits_len < m * c.n_vocab) throw rt_err("logits buffer too small");
     RIE_HIP_CHECK(hipSetDevice(device_));
-    RIE_HIP_CHECK(hipMemcpyAsync(d_tokens_, tokens, n * 4, hipMemcpyHostToDevice, st_));
+    launch_set_tokens(d_tokens_, tokens, n, d_pos_, (int)pos, st_);
     if (n == 1 && use_graph_ && !capture_) {
         decode_step_graph(pos);
     } else {
         run_layers((int)n, pos, nullptr, all_logits, splits_for(n, pos));
     }
-    RIE_HIP_CHECK(hipMemcpyAsync(logits, d_logits_, m * c.n_vocab * 4, hipMemcpyDeviceToHost, st_));
-    RIE_HIP_CHECK(hipStreamSynchronize(st_));
+    if (m * c.n_vocab <= h_out_cap_) {
+        launch_copy_out(d_logits_, h_out_, m * c.n_vocab, d_out_cnt_, h_flag_, ++out_seq_, st_);
+        check_launch("logits");
+        wait_out();
+        std::memcpy(logits, h_out_, m * c.n_vocab * 4);
+    } else {
+        RIE_HIP_CHECK(hipMemcpyAsync(logits, d_logits_, m * c.n_vocab * 4, hipMemcpyDeviceToHost, st_));
+        RIE_HIP_CHECK(hipStreamSynchronize(st_));
+    }
     hidden_rows_ = m;
 }
 
+// Until the logits of call out_seq_ are in h_out_.  A look at the flag costs a cache
+// hit, where hipStreamSynchronize returns several µs after the stream has drained; the
+// stream is asked every so often, so that an error or a lost flag ends the wait.
+void HipBackend::wait_out() {
+    for (uint32_t i = 1;; i++) {
+        if (__atomic_load_n(h_flag_, __ATOMIC_ACQUIRE) == out_seq_) return;
+        __builtin_ia32_pause();
+        if (i % 4096) continue;
+        const hipError_t e = hipStreamQuery(st_);
+        if (e == hipErrorNotReady) {
+            (void)hipGetLastError();  // not an error of the next launch
+            continue;
+        }
+        RIE_HIP_CHECK(e);
+        if (__atomic_load_n(h_flag_, __ATOMIC_ACQUIRE) != out_seq_) throw rt_err("logits did not arrive");
+    }
+}
+
 // The decode step as a graph: kernels read pos from d_pos_ and the token from
-// d_tokens_[0].  One graph per attention range count (it grows with the context).
+// d_tokens_[0], which the caller has set by kernel arguments (copied at launch, so
+// queued steps never share a host-side slot).  One graph per attention range count (it grows with the context).
 void HipBackend::decode_step_graph(size_t pos) {
-    // the position travels as a kernel argument (copied at launch), so queued
-    // steps never share a host-side slot
-    launch_set_int(d_pos_, (int)pos, st_);
-    check_launch("set pos");
     const int ns = splits_for(1, pos);
     auto it = graphs_.find(ns);
     if (it == graphs_.end()) {
@@ -962,7 +992,7 @@ uint32_t HipBackend::forward_argmax(const uint32_t *tokens, size_t n, size_t pos
     for (size_t t = 0; t < n; t++)
         if (tokens[t] >= m_.token_embd.rows) throw rt_err("token id " + std::to_string(tokens[t]) + " out of range");
     RIE_HIP_CHECK(hipSetDevice(device_));
-    RIE_HIP_CHECK(hipMemcpyAsync(d_tokens_, tokens, n * 4, hipMemcpyHostToDevice, st_));
+    launch_set_tokens(d_tokens_, tokens, n, d_pos_, (int)pos, st_);
     if (n == 1 && use_graph_ && !capture_) {
         decode_step_graph(pos);
     } else {
@@ -999,11 +1029,7 @@ void HipBackend::generate_greedy(size_t pos, size_t n_gen, uint32_t *out) {
     }
     for (size_t i = 0; i < n_gen; i++) {
         RIE_HIP_CHECK(hipMemcpyAsync(d_gen_ + i, d_tokens_, 4, hipMemcpyDeviceToDevice, st_));
-        if (use_graph_ && !capture_) {
-            decode_step_graph(pos + i);
-        } else {
-            run_layers(1, pos + i, nullptr, false, splits_for(1, pos + i));
-        }
+        run_layers(1, pos + i, nullptr, false, splits_for(1, pos + i));
         launch_argmax(d_logits_, (int)c.n_vocab, d_amax_idx_, d_amax_val_, n_amax_part_, d_tokens_, st_, d_amax_cnt_);
         check_launch("argmax");
     }

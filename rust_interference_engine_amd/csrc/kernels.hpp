@@ -136,6 +136,11 @@ void launch_argmax_noalloc(const float *x, int n, uint32_t *out_idx, hipStream_t
 void launch_add_inplace(float *x, const float *y, size_t n, float scale, hipStream_t st);
 void launch_scale(float *x, size_t n, float div, hipStream_t st);
 void launch_set_int(int *p, int v, hipStream_t st);
+// dst[0..n) = tokens (read before the call returns), and *pos = posv when pos is given
+void launch_set_tokens(uint32_t *dst, const uint32_t *tokens, size_t n, int *pos, int posv, hipStream_t st);
+// n floats to pinned, coherent host memory (both 16-byte aligned), then *flag = seq there;
+// cnt: one zeroed int (left zeroed)
+void launch_copy_out(const float *x, float *host, size_t n, int *cnt, uint32_t *flag, uint32_t seq, hipStream_t st);
 void launch_softcap(float *x, size_t n, float cap, hipStream_t st);
 void launch_quant_only(const float *x, int ldx, int n_rows, int K, int fmt, const ActQ8 &act, hipStream_t st);
 // MoE routing: softmax over n_exp logits per token, top-k with index tie-break, renorm.
