@@ -1,4 +1,4 @@
-// gemm.hip — prompt-batch matmul on CDNA4 int8 MFMA (Q4_0 / Q8_0 weights ×
+// gemm.hip — prompt-batch matmul on CDNA4 int8 MFMA (Q4_0 / Q5_0 / Q8_0 weights ×
 // Q8_0 activations), the batched counterpart of vec_dot / vec_dot_x4
 // (crates/rie-core/src/kernels/mod.rs:136-284, kernels/matmul.rs:119-241).
 //
@@ -7,13 +7,13 @@
 //   S[t][r]  = d_a[t][b]·d_w[r][b]                v_mfma_f32_32x32x1f32 (outer product;
 //                                                  two blocks' S per instruction)
 //   acc      = fma((float)I, S, acc)              VALU
-// (Q4_0 codes enter the MFMA as 16·(w_q − 8) and d_w as d_w/16: the same I·S)
+// (Q4_0 codes enter the MFMA as 16·(w_q − 8) and d_w as d_w/16, Q5_0 codes as
+// 8·(w_q − 16) and d_w/8: the same I·S)
 // so each block contributes (d_w·d_a)·isum exactly as the reference's block dot
 // does; only the order of the f32 sum over blocks differs.  Weights stay in
-// their ggml layout: a lane loads its row's 2-block unit (36 / 68 bytes, dword
-// aligned) per stage and writes its codes to LDS as int8, for Q4_0 with the
-// nibbles unpacked to 16·(q − 8) and the 1/16 on the block scale (once per
-// workgroup, not per wave).
+// their ggml layout: a thread loads a block (two of a gated pair) per stage and
+// writes its codes to LDS as int8, for Q4_0 with the nibbles unpacked to 16·(q − 8)
+// and the 1/16 on the block scale (once per workgroup, not per wave).
 //
 // Operand lane layout (checked by the parity tests): lane l supplies row
 // (l mod 32) and values 16·(l/32)..+16 of the block, for A (tokens) and B
@@ -25,6 +25,7 @@
 #include "../kernels.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace rie {
 
@@ -75,17 +76,49 @@ __device__ __forceinline__ GTileRows gtile_rows(const GemmP &p, int tg, int bn) 
 __device__ __forceinline__ int gact_row(const GemmP &p, int r) { return p.grouped && p.grp.amap ? p.grp.amap[r] : r; }
 __device__ __forceinline__ int gout_row(const GemmP &p, int r) { return p.grouped && p.grp.omap ? p.grp.omap[r] : r; }
 
-// weight unit: blocks b and b+1 of one row (36 or 68 bytes from a dword boundary)
+template <int TY> constexpr int block_dwords() { return TY == T_Q8_0 ? 8 : 4; }  // of codes
+
+// Weight unit: blocks b and b+1 of one row (36, 44 or 68 bytes from a dword boundary),
+// for the gated pair, whose 256 threads have two blocks each.
+template <int TY> constexpr int unit_dwords() { return 2 * block_dwords<TY>() + (TY == T_Q5_0 ? 3 : 1); }
 template <int TY>
 struct WUnit {
-    uint32_t w[TY == T_Q4_0 ? 9 : 17];
+    uint32_t w[unit_dwords<TY>()];
 };
 
 template <int TY>
 __device__ __forceinline__ void load_wunit(const uint8_t *row, int b, WUnit<TY> &u) {
-    const uint32_t *p = (const uint32_t *)(row + (size_t)b * (TY == T_Q4_0 ? 18 : 34));
+    const uint32_t *p = (const uint32_t *)(row + (size_t)b * (2 * unit_dwords<TY>()));
 #pragma unroll
-    for (int i = 0; i < (TY == T_Q4_0 ? 9 : 17); i++) u.w[i] = wload(p + i);
+    for (int i = 0; i < unit_dwords<TY>(); i++) u.w[i] = wload(p + i);
+}
+
+// One block's bytes, for the other launches, whose 256 threads have one block each: in
+// units, half of the threads held two and the staging was two of the four waves' work
+// (512 tokens, Q8_0, Q/K/V 6144 × 4096: 84 us, wo 4096 × 4096: 81 us; now 64 and 50 us;
+// the gated pair by blocks 291 us against 237 us by units).  Blocks start at any even
+// address.  Q4_0 in 128-token tiles keeps units (down 4096 × 14336: 115 against 118 us).
+struct __attribute__((packed, aligned(2))) Bytes16 {
+    uint32_t w[4];
+};
+struct __attribute__((packed, aligned(2))) Bytes4 {
+    uint32_t w;
+};
+template <int TY>
+struct WBlk {
+    Bytes16 q[block_dwords<TY>() / 4];
+    uint32_t qh;  // Q5_0
+    uint32_t d;
+};
+
+template <int TY>
+__device__ __forceinline__ void load_wblk(const uint8_t *row, int b, WBlk<TY> &u) {
+    constexpr int HD = TY == T_Q5_0 ? 6 : 2, BB = HD + 4 * block_dwords<TY>();
+    const uint8_t *p = row + (size_t)b * BB;
+    u.d = *(const uint16_t *)p;
+    if constexpr (TY == T_Q5_0) u.qh = ((const Bytes4 *)(p + 2))->w;
+#pragma unroll
+    for (int i = 0; i < block_dwords<TY>() / 4; i++) u.q[i] = *(const Bytes16 *)(p + HD + 16 * i);
 }
 
 // ---- LDS-tiled kernel ---------------------------------------------------------
@@ -105,6 +138,9 @@ struct GemmLds {
 
 // BN tokens per workgroup tile: 128 (two 32-token tiles per wave) or 64 (one)
 template <int TY, bool GLU, int BN>
+constexpr bool by_units() { return GLU || (TY == T_Q4_0 && BN == 128); }
+
+template <int TY, bool GLU, int BN>
 struct __align__(16) GemmStage {
     static constexpr int NW = GLU ? 2 : 1;
     int8_t a[BN * G_AST];
@@ -119,30 +155,86 @@ struct StageRegs {
     static constexpr int NW = GLU ? 2 : 1;
     v4i a[BN / 32];  // the thread's part of its token's 128-byte chunk
     float4 da;
-    WUnit<TY> w;
+    std::conditional_t<by_units<TY, GLU, BN>(), WUnit<TY>, WBlk<TY>> w;
 };
 
 // tokA: the activation row of the thread's token (tid / (256/BN)); tokD: of token tid
 // (tid < BN); woff: the expert's byte offset in a grouped launch
-template <int TY, bool GLU, int BN>
+// TAIL: K is an odd multiple of 64, so the last stage holds two blocks.  Its other two
+// repeat the row's last ones (in bounds) with activation scales of 0.  (As a run-time
+// check in every launch this took a 512-token Q8_0 prompt from 1353 to 1478 us.)
+template <int TY, bool GLU, int BN, bool TAIL>
 __device__ __forceinline__ void stage_load(const GemmP &p, int sg, int row0, int tokA, int tokD, size_t woff, int b0, int tid,
                                            StageRegs<TY, GLU, BN> &R) {
     const int K = p.K, nb = K >> 5;
+    const bool tail = TAIL && b0 + G_KC > nb;  // workgroup-uniform
     {   // activation codes: thread → (token, part of its 128-byte chunk)
         constexpr int TPT = 256 / BN, NV = 128 / TPT / 16;  // threads per token, 16-byte loads per thread
-        const v4i *src = (const v4i *)(p.qs + (size_t)tokA * K + 32 * b0 + 16 * NV * (tid % TPT));
+        const int k = 32 * b0 + 16 * NV * (tid % TPT);
+        const v4i *src = (const v4i *)(p.qs + (size_t)tokA * K + (tail ? min(k, K - 16 * NV) : k));
 #pragma unroll
         for (int i = 0; i < NV; i++) R.a[i] = src[i];
     }
-    if (tid < BN) R.da = *(const float4 *)(p.d + (size_t)tokD * nb + b0);
-    {   // weights: thread → (matrix, row, 2-block unit)
-        const int nw = GLU ? (tid >> 7) : 0;
-        const int idx = tid & 127;
+    if (!TAIL && tid < BN) R.da = *(const float4 *)(p.d + (size_t)tokD * nb + b0);
+    if (TAIL && tid < BN) {
+        const float *d = p.d + (size_t)tokD * nb + b0;
+        const float2 d01 = *(const float2 *)d;
+        const float2 d23 = *(const float2 *)(tail ? d : d + 2);
+        R.da = make_float4(d01.x, d01.y, tail ? 0.0f : d23.x, tail ? 0.0f : d23.y);
+    }
+    if constexpr (by_units<TY, GLU, BN>()) {  // weights: thread → (matrix, row, unit)
+        const int idx = tid & 127, sm = GLU ? (tid >> 7) : sg;
         const int row = min(row0 + (idx >> 1), p.rows[GLU ? 0 : sg] - 1);
-        if (GLU || tid < 128) {
-            const int s = GLU ? nw : sg;
-            load_wunit<TY>(p.w[s] + woff + (size_t)row * p.rb[s], b0 + 2 * (idx & 1), R.w);
+        if (GLU || tid < 128) load_wunit<TY>(p.w[sm] + woff + (size_t)row * p.rb[sm], b0 + (tail ? 0 : 2 * (idx & 1)), R.w);
+    } else {  // thread → (row, block)
+        const int row = min(row0 + (tid >> 2), p.rows[sg] - 1), b = b0 + (tid & 3);
+        load_wblk<TY>(p.w[sg] + woff + (size_t)row * p.rb[sg], tail ? min(b, nb - 1) : b, R.w);
+    }
+}
+
+// a block's codes as int8 to LDS, and its scale
+template <int TY>
+__device__ __forceinline__ void put_block(const uint32_t (&q)[block_dwords<TY>()], uint32_t qh, uint32_t d, uint8_t *wq, float *dw) {
+    if constexpr (TY == T_Q4_0) {
+        // nibbles → int8 16·(q − 8) once per workgroup: bytes 0..15 of a block are
+        // values 0..15 (low nibbles), bytes 16..31 values 16..31 (high nibbles).
+        // q ^ 8 is q − 8 as a 4-bit two's complement number, so with every nibble
+        // flipped by one XOR, a nibble moved into (or left in) the high half of its
+        // byte, low half zero, is the int8 16·(q − 8): 4 instructions per 8 codes.
+        // The block's product is then 16·I exactly (|16·I| < 2²⁴) and its weight
+        // scale carries the 1/16 (a power of two: d_a·d_w/16 and the fma with 16·I
+        // round exactly as d_a·d_w and I do).
+        uint32_t lo[4], hi[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint32_t f = q[k] ^ 0x88888888u;
+            lo[k] = (f << 4) & 0xF0F0F0F0u;
+            hi[k] = f & 0xF0F0F0F0u;
         }
+        *(uint4 *)wq = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        *(uint4 *)(wq + 16) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        *dw = h2f(d) * 0.0625f;
+    } else if constexpr (TY == T_Q5_0) {
+        // a nibble with its fifth bit (bit j of qh for value j) put above it is the
+        // 5-bit code q; q ^ 16 is q − 16 as a two's complement number, and moved to
+        // the top of its byte the int8 8·(q − 16)
+        auto code = [](uint32_t nib, uint32_t bits) {  // 4 nibbles in bytes, their fifth bits in bits 0..3
+            const uint32_t e = (bits << 4 | bits << 11 | bits << 18 | bits << 25) & 0x10101010u;
+            return ((nib & 0x0F0F0F0Fu) | (e ^ 0x10101010u)) << 3;
+        };
+        uint32_t lo[4], hi[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            lo[k] = code(q[k], (qh >> (4 * k)) & 15u);
+            hi[k] = code(q[k] >> 4, (qh >> (16 + 4 * k)) & 15u);
+        }
+        *(uint4 *)wq = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        *(uint4 *)(wq + 16) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        *dw = h2f(d) * 0.125f;
+    } else {
+#pragma unroll
+        for (int k = 0; k < 2; k++) *(uint4 *)(wq + 16 * k) = make_uint4(q[4 * k], q[4 * k + 1], q[4 * k + 2], q[4 * k + 3]);
+        *dw = h2f(d);
     }
 }
 
@@ -155,47 +247,29 @@ __device__ __forceinline__ void stage_store(GemmStage<TY, GLU, BN> &S, int tid, 
         for (int i = 0; i < NV; i++) dst[i] = R.a[i];
     }
     if (tid < BN) *(float4 *)(S.da + tid * G_KC) = R.da;
-    if (GLU || tid < 128) {
-        const int nw = GLU ? (tid >> 7) : 0;
-        const int idx = tid & 127, row = idx >> 1, u = idx & 1;
-        constexpr int QB = GemmLds<TY>::QB, WST = GemmLds<TY>::WST;
-        uint8_t *wq = S.wq[nw] + row * WST + 2 * u * QB;
-        float *dw = S.dw[nw] + row * G_KC + 2 * u;
-        if constexpr (TY == T_Q4_0) {
-            // nibbles → int8 16·(q − 8) once per workgroup: bytes 0..15 of a block are
-            // values 0..15 (low nibbles), bytes 16..31 values 16..31 (high nibbles).
-            // q ^ 8 is q − 8 as a 4-bit two's complement number, so with every nibble
-            // flipped by one XOR, a nibble moved into (or left in) the high half of its
-            // byte, low half zero, is the int8 16·(q − 8): 4 instructions per 8 codes.
-            // The block's product is then 16·I exactly (|16·I| < 2²⁴) and its weight
-            // scale carries the 1/16 (a power of two: d_a·d_w/16 and the fma with 16·I
-            // round exactly as d_a·d_w and I do).
-            uint32_t q[8];
+    constexpr int QB = GemmLds<TY>::QB, WST = GemmLds<TY>::WST, ND = block_dwords<TY>();
+    uint32_t q[ND];
+    if constexpr (by_units<TY, GLU, BN>()) {
+        if (!GLU && tid >= 128) return;
+        const int nw = GLU ? (tid >> 7) : 0, row = (tid & 127) >> 1, u = tid & 1;
+        const uint32_t *w = R.w.w;
+        constexpr int C0 = TY == T_Q5_0 ? 1 : 0;  // the dword whose upper half starts block 0's codes
 #pragma unroll
-            for (int i = 0; i < 4; i++) q[i] = __builtin_amdgcn_alignbyte(R.w.w[i + 1], R.w.w[i], 2) ^ 0x88888888u;
+        for (int b = 0; b < 2; b++) {
+            // block 0's codes start 2 bytes into a dword, block 1's at one
 #pragma unroll
-            for (int i = 0; i < 4; i++) q[4 + i] = R.w.w[5 + i] ^ 0x88888888u;
-            auto lo16 = [](uint32_t v) { return (v << 4) & 0xF0F0F0F0u; };
-            auto hi16 = [](uint32_t v) { return v & 0xF0F0F0F0u; };
-#pragma unroll
-            for (int b = 0; b < 2; b++) {
-                *(uint4 *)(wq + 32 * b) = make_uint4(lo16(q[4 * b]), lo16(q[4 * b + 1]), lo16(q[4 * b + 2]), lo16(q[4 * b + 3]));
-                *(uint4 *)(wq + 32 * b + 16) = make_uint4(hi16(q[4 * b]), hi16(q[4 * b + 1]), hi16(q[4 * b + 2]), hi16(q[4 * b + 3]));
-            }
-            dw[0] = h2f(R.w.w[0] & 0xffff) * 0.0625f;
-            dw[1] = h2f(R.w.w[4] >> 16) * 0.0625f;
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; i++) ((uint32_t *)wq)[i] = __builtin_amdgcn_alignbyte(R.w.w[i + 1], R.w.w[i], 2);
-#pragma unroll
-            for (int i = 0; i < 8; i++) ((uint32_t *)wq)[8 + i] = R.w.w[9 + i];
-            dw[0] = h2f(R.w.w[0] & 0xffff);
-            dw[1] = h2f(R.w.w[8] >> 16);
+            for (int i = 0; i < ND; i++) q[i] = b ? w[unit_dwords<TY>() - ND + i] : __builtin_amdgcn_alignbyte(w[C0 + i + 1], w[C0 + i], 2);
+            const uint32_t qh = TY == T_Q5_0 ? (b ? w[6] : __builtin_amdgcn_alignbyte(w[1], w[0], 2)) : 0u;
+            put_block<TY>(q, qh, b ? w[C0 + ND] >> 16 : w[0] & 0xffff, S.wq[nw] + row * WST + (2 * u + b) * QB, S.dw[nw] + row * G_KC + 2 * u + b);
         }
+    } else {
+#pragma unroll
+        for (int i = 0; i < ND; i++) q[i] = R.w.q[i / 4].w[i % 4];
+        put_block<TY>(q, R.w.qh, R.w.d, S.wq[0] + (tid >> 2) * WST + (tid & 3) * QB, S.dw[0] + (tid >> 2) * G_KC + (tid & 3));
     }
 }
 
-template <int TY, bool GLU, int NT>
+template <int TY, bool GLU, int NT, bool TAIL>
 __global__ __launch_bounds__(256, (!GLU && NT == 1) ? 3 : 2) void gemm_kernel(GemmP p) {  // one-tile non-gated: three waves per SIMD
     constexpr int NW = GLU ? 2 : 1;
     constexpr int BN = 64 * NT;  // tokens per workgroup tile: NT 32-token tiles per wave, 2 waves along tokens
@@ -236,15 +310,15 @@ __global__ __launch_bounds__(256, (!GLU && NT == 1) ? 3 : 2) void gemm_kernel(Ge
     // two stages before their LDS store.  Load indices past the last stage repeat the
     // last stage and the step count is even, so every load is unconditional and the
     // compiler's wait for a register set counts exactly the loads issued after it.
-    // this workgroup's stages: [k0, k0 + n_stages) of the K / 128 (its K split)
-    const int all_stages = p.K / (32 * G_KC);
+    // this workgroup's stages: [k0, k0 + n_stages) of the K / 128, rounded up (its K split)
+    const int all_stages = (p.K + 32 * G_KC - 1) / (32 * G_KC);
     const int k0 = ksi * all_stages / p.ks;
     const int n_stages = (ksi + 1) * all_stages / p.ks - k0;
     const int last_stage = n_stages - 1;
     StageRegs<TY, GLU, BN> ra, rb;
-    stage_load<TY, GLU, BN>(p, sg, row0, tokA, tokD, woff, k0 * G_KC, tid, ra);
+    stage_load<TY, GLU, BN, TAIL>(p, sg, row0, tokA, tokD, woff, k0 * G_KC, tid, ra);
     stage_store<TY, GLU, BN>(st[0], tid, ra);
-    stage_load<TY, GLU, BN>(p, sg, row0, tokA, tokD, woff, (k0 + min(1, last_stage)) * G_KC, tid, rb);
+    stage_load<TY, GLU, BN, TAIL>(p, sg, row0, tokA, tokD, woff, (k0 + min(1, last_stage)) * G_KC, tid, rb);
     __syncthreads();
     // Per stage: all operands of the stage's KC blocks from LDS, then the
     // P = KC·NT·NW tile products in a software pipeline: the MFMAs of product
@@ -252,7 +326,7 @@ __global__ __launch_bounds__(256, (!GLU && NT == 1) ? 3 : 2) void gemm_kernel(Ge
     constexpr int P = G_KC * NT * NW;
     // rl: receives stage s + 2; rs: holds stage s + 1, stored to LDS after stage s
     auto body = [&](int s, StageRegs<TY, GLU, BN> &rl, const StageRegs<TY, GLU, BN> &rs) {
-        stage_load<TY, GLU, BN>(p, sg, row0, tokA, tokD, woff, (k0 + min(s + 2, last_stage)) * G_KC, tid, rl);
+        stage_load<TY, GLU, BN, TAIL>(p, sg, row0, tokA, tokD, woff, (k0 + min(s + 2, last_stage)) * G_KC, tid, rl);
         if (s < n_stages) {  // workgroup-uniform; the idle step of an odd stage count skips it
             const GemmStage<TY, GLU, BN> &S = st[s & 1];
             v4i bw[G_KC][NW], av[G_KC][NT];
@@ -342,7 +416,7 @@ __global__ __launch_bounds__(256, (!GLU && NT == 1) ? 3 : 2) void gemm_kernel(Ge
 }
 
 bool gemm_supported(int ty, size_t K) {
-    return ((ty == T_Q4_0 || ty == T_Q8_0) && K % (32 * G_KC) == 0 && K > 0) || gemm_kq_supported(ty, K);
+    return ((ty == T_Q4_0 || ty == T_Q5_0 || ty == T_Q8_0) && K % 64 == 0 && K > 0) || gemm_kq_supported(ty, K);
 }
 
 // out[t·ld + r] += part[0][…] + … + part[n_part−1][…] for r < rows, in split order
@@ -364,7 +438,7 @@ __global__ __launch_bounds__(256) void gemm_add_parts_kernel(float *__restrict__
 template <int TY, bool GLU>
 static void launch_t(GemmP p, hipStream_t st, const GroupTiles *grp, float *part, size_t part_cap) {
     const int tiles128 = p.n_rg * ((p.n_tok + 127) / 128);
-    const int n_st = p.K / (32 * G_KC);
+    const int n_st = (p.K + 32 * G_KC - 1) / (32 * G_KC);
     p.ks = 1;
     if (!GLU && !grp && p.nseg == 1 && part && n_st >= 48 && p.n_tok > 64) {
         const size_t plane = (size_t)p.n_tok * p.ld[0];
@@ -383,15 +457,19 @@ static void launch_t(GemmP p, hipStream_t st, const GroupTiles *grp, float *part
         p.n_tg = grp->max_tiles;
     }
     const dim3 grid(gemm_grid(p.n_rg, p.n_tg, p.ks, p.grouped));
+    const bool tail = p.K % (32 * G_KC) != 0;
     if constexpr (!GLU) {
-        if (nt == 2) hipLaunchKernelGGL((gemm_kernel<TY, GLU, 2>), grid, dim3(256), 0, st, p);
-        else hipLaunchKernelGGL((gemm_kernel<TY, GLU, 1>), grid, dim3(256), 0, st, p);
+        if (nt == 2 && tail) hipLaunchKernelGGL((gemm_kernel<TY, GLU, 2, true>), grid, dim3(256), 0, st, p);
+        else if (nt == 2) hipLaunchKernelGGL((gemm_kernel<TY, GLU, 2, false>), grid, dim3(256), 0, st, p);
+        else if (tail) hipLaunchKernelGGL((gemm_kernel<TY, GLU, 1, true>), grid, dim3(256), 0, st, p);
+        else hipLaunchKernelGGL((gemm_kernel<TY, GLU, 1, false>), grid, dim3(256), 0, st, p);
         if (p.ks > 1)
             hipLaunchKernelGGL(gemm_add_parts_kernel, dim3((p.rows[0] + 255) / 256, p.n_tok), dim3(256), 0, st, p.out[0], p.part,
                                p.part_stride, p.ks - 1, p.rows[0], p.ld[0]);
         return;
     }
-    hipLaunchKernelGGL((gemm_kernel<TY, GLU, 1>), grid, dim3(256), 0, st, p);
+    if (tail) hipLaunchKernelGGL((gemm_kernel<TY, GLU, 1, true>), grid, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((gemm_kernel<TY, GLU, 1, false>), grid, dim3(256), 0, st, p);
 }
 
 void launch_gemm_add_parts(float *out, const float *part, size_t stride, int n_part, int rows, int ld, int n_tok, hipStream_t st) {
@@ -434,6 +512,7 @@ bool launch_gemm(const GemvSeg *segs, int nseg, const ActQ8 &act, int n_tok, int
     p.n_tok = n_tok;
     p.K = K;
     if (ty == T_Q4_0) launch_t<T_Q4_0, false>(p, st, grp, part, part_cap);
+    else if (ty == T_Q5_0) launch_t<T_Q5_0, false>(p, st, grp, part, part_cap);
     else launch_t<T_Q8_0, false>(p, st, grp, part, part_cap);
     return true;
 }
@@ -464,6 +543,7 @@ bool launch_gemm_glu(const DevWeight &gate, const DevWeight &up, const ActQ8 &ac
     p.n_tok = n_tok;
     p.K = K;
     if (gate.ty == T_Q4_0) launch_t<T_Q4_0, true>(p, st, grp, nullptr, 0);
+    else if (gate.ty == T_Q5_0) launch_t<T_Q5_0, true>(p, st, grp, nullptr, 0);
     else launch_t<T_Q8_0, true>(p, st, grp, nullptr, 0);
     return true;
 }

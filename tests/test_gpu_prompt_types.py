@@ -1,4 +1,4 @@
-"""Prompt matmuls of the weight types beyond Q4_0 / Q8_0 / Q4_K on the matrix cores,
+"""Prompt matmuls of the weight types and widths beyond 128-multiples of Q4_0 / Q8_0 and Q4_K on the matrix cores,
 against the oracle: kernels through rie_hip_k_gemm, gated and grouped forms
 through small models."""
 import numpy as np
@@ -7,7 +7,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
-from test_gpu_parity import Q5_K, Q6_K, _gemv, _pair, _quant_on_gpu, act_fmt, cuda  # noqa: E402,F401
+from test_gpu_parity import Q4_0, Q5_0, Q5_K, Q6_K, Q8_0, _gemv, _pair, _quant_on_gpu, act_fmt, cuda  # noqa: E402,F401
 
 
 def _check_rows(oracle, cuda, ty, k, rows, n_tok):
@@ -19,7 +19,7 @@ def _check_rows(oracle, cuda, ty, k, rows, n_tok):
     got = _gemv(ty, w, rows, k, _quant_on_gpu(x, act_fmt(ty), cuda)["dev"], None, n_tok, cuda, gemm=True)
     wf = G.dequantize(ty, w, rows * k).reshape(rows, k).astype(np.float64)
     rb = G.row_bytes(ty, k)
-    for t in range(n_tok):
+    for t in range(n_tok) if rows < 1000 else (0, 127, 128, n_tok - 1):
         a = oracle.quantize_act(ty, x[t])
         want = np.array([oracle.vec_dot(ty, w[i * rb:(i + 1) * rb], a, k) for i in range(rows)])
         mag = np.abs(wf * x[t].astype(np.float64)).sum(axis=1)
@@ -32,7 +32,16 @@ def test_q5_k_gemm_matches_oracle_rows(oracle, cuda, k, rows, n_tok):
     _check_rows(oracle, cuda, Q5_K, k, rows, n_tok)
 
 
-@pytest.mark.parametrize("arch,ty", [("llama", Q5_K), ("gemma2", Q5_K), ("gemma2", Q6_K), ("qwen3moe", Q5_K), ("qwen3moe", Q6_K)])
+# K of one whole stage, of one and a half, of half a stage, 128-token tiles over an odd
+# number of stages, a K split in uneven parts with half a stage at the end (49 stages)
+@pytest.mark.parametrize("ty", [Q4_0, Q5_0, Q8_0])
+@pytest.mark.parametrize("k,rows,n_tok", [(128, 40, 9), (192, 70, 33), (64, 64, 65), (960, 4200, 520), (6208, 96, 70)])
+def test_32_block_gemm_matches_oracle_rows(oracle, cuda, ty, k, rows, n_tok):
+    _check_rows(oracle, cuda, ty, k, rows, n_tok)
+
+
+@pytest.mark.parametrize("arch,ty", [("llama", Q5_K), ("gemma2", Q5_K), ("gemma2", Q6_K), ("qwen3moe", Q5_K), ("qwen3moe", Q6_K),
+                                     ("gemma2", Q5_0), ("qwen3moe", Q5_0)])
 def test_gated_and_grouped_k_quant_prompts_match_oracle(oracle, cuda, arch, ty):
     """Gate/up with SwiGLU or GELU in one launch, and experts grouped on the device."""
     from naive_model import max_rel_err
