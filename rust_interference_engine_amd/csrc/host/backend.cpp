@@ -201,9 +201,9 @@ HipBackend::HipBackend(const uint8_t *gguf, size_t len, const BackendConfig &cfg
     d_kcap_ = dalloc<float>(allocs_, mb * kvd);
     d_att_ = dalloc<float>(allocs_, mb * qd);
     d_o_ = dalloc<float>(allocs_, mb * E);
-    // partial sums of K-split prompt GEMMs (up to three planes of a batch's E-wide
-    // outputs, at most 64 MiB): only batches above 64 tokens split
-    gemm_ws_cap_ = mb > 64 ? std::min<size_t>(3 * mb * E, (size_t)1 << 24) : 0;
+    // partial sums of K-split prompt GEMMs (batches above 8 tokens): 5 MB added up in the
+    // launch, or up to three planes of a batch's E-wide outputs, at most 64 MiB
+    gemm_ws_cap_ = mb > 8 ? std::max((size_t)320 * 16 * 256, std::min<size_t>(3 * mb * E, (size_t)1 << 24)) : 0;
     // BF16 / F16 matrices: the parts of a prompt's rows, and the partial sums of up to
     // four splits of Q/K/V (at most 64 MiB)
     bool halves = act_format(out_w_.ty) == ACT_F32 && out_w_.ty != T_F32;
@@ -215,7 +215,10 @@ HipBackend::HipBackend(const uint8_t *gguf, size_t len, const BackendConfig &cfg
         split_.scale = dalloc<float>(allocs_, mb);
         gemm_ws_cap_ = std::max(gemm_ws_cap_, std::min<size_t>(4 * mb * std::max(E, qd + 2 * kvd), (size_t)1 << 24));
     }
-    if (gemm_ws_cap_) d_gemm_ws_ = dalloc<float>(allocs_, gemm_ws_cap_);
+    if (gemm_ws_cap_) {
+        d_gemm_ws_ = dalloc<float>(allocs_, gemm_ws_cap_);
+        gemm_ws_ = GemmWs{d_gemm_ws_, gemm_ws_cap_, dalloc<int>(allocs_, 512), 512};
+    }
     // routed experts per token as the layers run them (clamped to [1, n_expert], model/mod.rs:176)
     const size_t nu = std::max<size_t>(n_used_max_, 1);
     d_h_ = dalloc<float>(allocs_, mb * ff_max_ * nu);
@@ -366,7 +369,7 @@ void HipBackend::matmul(const GemvSeg *segs, int nseg, int n, int K, const ActQ8
         while (n > 8 && s < j && gemm_supported(segs[s].w.ty, K)) {
             int e = s + 1;
             while (e < j && e - s < 3 && segs[e].w.ty == segs[s].w.ty) e++;
-            if (!launch_gemm(&segs[s], e - s, a, n, K, st_, nullptr, d_gemm_ws_, gemm_ws_cap_)) break;
+            if (!launch_gemm(&segs[s], e - s, a, n, K, st_, nullptr, gemm_ws_)) break;
             s = e;
         }
         while (n > 8 && s < j && split_.p[0] && gemm_float_supported(segs[s].w.ty, K)) {
@@ -399,7 +402,7 @@ void HipBackend::ffn_dense(const DevLayer &L, int n, float *out, int epi) {
     }
     const ActQ8 &a = act_format(L.gate.ty) == ACT_Q8K ? actk_ : act0_;
     bool done = false;
-    if (n > 8 && gemm_supported(L.gate.ty, E)) done = launch_gemm_glu(L.gate, L.up, a, n, E, d_h_, ff, c.gelu, nullptr, st_);
+    if (n > 8 && gemm_supported(L.gate.ty, E)) done = launch_gemm_glu(L.gate, L.up, a, n, E, d_h_, ff, c.gelu, st_, nullptr, gemm_ws_);
     if (n > 8 && L.gate.ty == split_ty_) done = launch_gemm_float_glu(L.gate, L.up, split_, n, E, d_h_, ff, c.gelu, st_);
     const int fmt = act_format(L.down.ty);
     // single-token Q8_0 down projection: the gate/up kernel quantizes h itself
@@ -642,7 +645,7 @@ void HipBackend::expert_ffn(const DevWeight &g, const DevWeight &u, const DevWei
     prepare(x, nullptr, m, E, ws, 2, false);
     const ActQ8 &a = act_format(g.ty) == ACT_Q8K ? actk_ : act0_;
     bool done = false;
-    if (m > 8 && gemm_supported(g.ty, E)) done = launch_gemm_glu(g, u, a, m, E, d_h_, ff, c.gelu, nullptr, st_);
+    if (m > 8 && gemm_supported(g.ty, E)) done = launch_gemm_glu(g, u, a, m, E, d_h_, ff, c.gelu, st_, nullptr, gemm_ws_);
     if (m > 8 && g.ty == split_ty_) done = launch_gemm_float_glu(g, u, split_, m, E, d_h_, ff, c.gelu, st_);
     if (!done && !launch_gemv_glu(g, u, a, d_xn_, m, E, d_h_, ff, c.gelu, nullptr, st_))
         throw Error{E_UNSUPPORTED, "unsupported: expert FFN weights"};
@@ -766,7 +769,7 @@ bool HipBackend::ffn_moe(const DevLayer &L, int n, bool direct) {
         de.rows = (size_t)E;
         g.wstride = (size_t)ff * L.gate.rb();
         const ActQ8 &ax = act_format(L.gate.ty) == ACT_Q8K ? actk_ : act0_;
-        if (!launch_gemm_glu(ge, ue, ax, n * k, E, d_h_, ff, c.gelu, nullptr, st_, &g)) throw rt_err("grouped expert gate/up launch rejected");
+        if (!launch_gemm_glu(ge, ue, ax, n * k, E, d_h_, ff, c.gelu, st_, &g)) throw rt_err("grouped expert gate/up launch rejected");
         check_launch("moe gate/up");
         mark("moe_gate_up_glu");
         const int dfmt = act_format(L.down.ty);

@@ -128,6 +128,7 @@ class HipBackend {
     float *d_x_ = nullptr, *d_xn_ = nullptr, *d_q_ = nullptr, *d_k_ = nullptr, *d_v_ = nullptr, *d_att_ = nullptr, *d_h_ = nullptr,
           *d_o_ = nullptr, *d_logits_ = nullptr, *d_part_ = nullptr, *d_amax_val_ = nullptr, *d_gemm_ws_ = nullptr;
     size_t gemm_ws_cap_ = 0;  // floats at d_gemm_ws_
+    GemmWs gemm_ws_;          // the same with arrival counters, for the int8 GEMMs
     float *h_out_ = nullptr;  // pinned host memory for the logits of a call, up to h_out_cap_ floats
     size_t h_out_cap_ = 0;
     uint32_t *h_flag_ = nullptr;  // behind them: the sequence number of the last call whose logits have arrived

@@ -299,19 +299,17 @@ int32_t rie_hip_k_gemm(int32_t ty, const uint8_t *w, int32_t rows, int32_t k, co
         a.bsums = const_cast<int16_t *>(bsums);
         PaddedWeight pw(ty, w, rows, k);
         rie::GemvSeg sg{mkw(ty, pw.data, rows, k), out, rows, rie::EPI_STORE};
-        // room for the partial sums of a K split (up to three planes, capped at
-        // 64 MiB like the backend's workspace), only where a split can happen:
-        // Q4_0/Q5_0/Q8_0 weights with at least 48 stages of 128 values, or Q4_K/Q5_K/Q6_K
-        // with at least 8 superblocks, over 64 tokens
-        const bool can_split = ((ty == rie::T_Q4_0 || ty == rie::T_Q5_0 || ty == rie::T_Q8_0) && (k + 127) / 128 >= 48 && n_tok > 64) ||
-                               ((ty == rie::T_Q4_K || ty == rie::T_Q5_K || ty == rie::T_Q6_K) && k / 256 >= 8 && n_tok > 64);
-        const size_t cap = can_split ? std::min<size_t>(3 * (size_t)n_tok * (size_t)std::max(rows, 0), (size_t)1 << 24) : 0;
-        float *part = nullptr;
-        if (cap) RIE_HIP_CHECK(hipMalloc(&part, cap * sizeof(float)));
-        const bool ok = rie::gemm_supported(ty, (size_t)k) && rie::launch_gemm(&sg, 1, a, n_tok, k, 0, nullptr, part, cap);
-        hipError_t e = hipGetLastError();
+        // room for the partial sums of K splits, as the backend's
+        rie::GemmWs ws;
+        ws.cap = (size_t)1 << 22;
+        ws.n_cnt = 512;
+        RIE_HIP_CHECK(hipMalloc(&ws.part, ws.cap * sizeof(float) + ws.n_cnt * sizeof(int)));
+        ws.cnt = (int *)(ws.part + ws.cap);
+        hipError_t e = hipMemset(ws.cnt, 0, ws.n_cnt * sizeof(int));
+        const bool ok = e == hipSuccess && rie::gemm_supported(ty, (size_t)k) && rie::launch_gemm(&sg, 1, a, n_tok, k, 0, nullptr, ws);
+        if (e == hipSuccess) e = hipGetLastError();
         hipError_t e2 = hipDeviceSynchronize();
-        if (part) (void)hipFree(part);
+        (void)hipFree(ws.part);
         if (!ok) throw Error{rie::E_UNSUPPORTED, "no GEMM kernel for this weight type/shape"};
         RIE_HIP_CHECK(e);
         RIE_HIP_CHECK(e2);

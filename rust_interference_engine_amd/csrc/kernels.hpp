@@ -188,16 +188,24 @@ void launch_moe_group(const int *sel, int n_tok, int k, int n_exp, int *off, int
                       int *n_tiles, int bn, hipStream_t st);
 int moe_group_max_tiles(int n_tok, int k, int n_exp, int bn = GROUP_BN);
 
-// ---- gemm_kq.hip (prefill, Q4_K × Q8_K on int8 MFMA; reached through gemm.hip) ----
-bool gemm_kq_supported(int ty, size_t K);
-// part (part_cap floats): partial sums of a K split (Q6_K, one ungrouped segment)
-bool launch_gemm_kq(const GemvSeg *segs, int nseg, const ActQ8 &act, int n_tok, int K, hipStream_t st, const GroupTiles *grp = nullptr,
-                    float *part = nullptr, size_t part_cap = 0);
+// Room for the partial sums of a GEMM launch's K splits: cap floats at part (under 4 GiB),
+// n_cnt zeroed ints at cnt (left zeroed), one per tile.  Empty: no split.
+struct GemmWs {
+    float *part = nullptr;
+    size_t cap = 0;
+    int *cnt = nullptr;
+    int n_cnt = 0;
+};
 // out[t·ld + r] += part[0][t·ld + r] + … + part[n_part−1][…] (planes stride floats
 // apart) for r < rows, t < n_tok, in split order
 void launch_gemm_add_parts(float *out, const float *part, size_t stride, int n_part, int rows, int ld, int n_tok, hipStream_t st);
+
+// ---- gemm_kq.hip (prefill, K-quants × Q8_K on int8 MFMA; reached through gemm.hip) ----
+bool gemm_kq_supported(int ty, size_t K);
+bool launch_gemm_kq(const GemvSeg *segs, int nseg, const ActQ8 &act, int n_tok, int K, hipStream_t st, const GroupTiles *grp = nullptr,
+                    const GemmWs &ws = {});
 bool launch_gemm_kq_glu(const DevWeight &gate, const DevWeight &up, const ActQ8 &act, int n_tok, int K, float *h, int ld, int gelu,
-                        hipStream_t st, const GroupTiles *grp = nullptr);
+                        hipStream_t st, const GroupTiles *grp = nullptr, const GemmWs &ws = {});
 
 // ---- gemm_float.hip (prefill, BF16 / F16 × f32 on 16-bit MFMA) ----
 bool gemm_float_supported(int ty, size_t K);
@@ -214,10 +222,9 @@ bool launch_gemm_float_glu(const DevWeight &gate, const DevWeight &up, const Act
 // ---- gemm.hip (prefill, int8 MFMA) ----
 bool gemm_supported(int ty, size_t K);
 // grp: one segment per expert group (the segment's rows are one expert's; see GroupTiles)
-// part (part_cap floats): room for the partial sums of a K split (see launch_t)
 bool launch_gemm(const GemvSeg *segs, int nseg, const ActQ8 &act, int n_tok, int K, hipStream_t st, const GroupTiles *grp = nullptr,
-                 float *part = nullptr, size_t part_cap = 0);
+                 const GemmWs &ws = {});
 bool launch_gemm_glu(const DevWeight &gate, const DevWeight &up, const ActQ8 &act, int n_tok, int K, float *h, int ld, int gelu,
-                     float *scratch, hipStream_t st, const GroupTiles *grp = nullptr);
+                     hipStream_t st, const GroupTiles *grp = nullptr, const GemmWs &ws = {});
 
 }  // namespace rie

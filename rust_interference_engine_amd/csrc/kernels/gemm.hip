@@ -23,6 +23,7 @@
 #include "../common.hpp"
 #include "../device.hpp"
 #include "../kernels.hpp"
+#include "../gemm_split.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -52,13 +53,9 @@ struct GemmP {
     int n_tok, K;
     int grouped;    // expert groups: one matrix per expert (grp), 64-token tiles from its table
     GroupTiles grp;
-    // K split (one segment, not gated or grouped): split 0 runs the segment's
-    // epilogue on its partial sum, split i > 0 stores its partial to part[i-1]
-    // ([n_tok][ld], stride part_stride floats), which a second launch adds to the
-    // output in split order
-    int ks;
-    float *part;
-    size_t part_stride;
+    int ks;  // K splits of a tile (not grouped), added up in ws by the last of them
+    GemmWs ws;
+    size_t plane;  // floats per plane of a split in planes (plane_count), 0: split_sum
 };
 
 // A workgroup's token rows: tokens [r0, r_end) of the batch, or gathered rows
@@ -394,12 +391,16 @@ __global__ __launch_bounds__(256, (!GLU && NT == 1) ? 3 : 2) void gemm_kernel(Ge
         body(s + 1, rb, ra);
     }
     // ---- epilogue: lane holds weight row row0 + wrow for tokens t0 + wc·64 + 32t + 16h + v ----
+    if (p.ks > 1 && !p.plane && !split_sum(reinterpret_cast<float(&)[NW * NT * 16]>(acc), p.ws.part, (uint32_t)(p.ws.cap * 4), p.ws.cnt,
+                               rg * p.n_tg + tg, ksi, p.ks))
+        return;
     const int rows = p.rows[sg];
     const int row = row0 + wrow;
     if (row >= rows) return;
     const int ld = p.ld[sg];
-    float *out = ksi ? p.part + (size_t)(ksi - 1) * p.part_stride : p.out[sg];
-    const int epi = ksi ? EPI_STORE : p.epi[sg];
+    const bool part = p.plane && ksi;
+    float *out = part ? p.ws.part + (size_t)(ksi - 1) * p.plane : p.out[sg];
+    const int epi = part ? EPI_STORE : p.epi[sg];
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
@@ -430,31 +431,38 @@ __global__ __launch_bounds__(256) void gemm_add_parts_kernel(float *__restrict__
     out[i] = v;
 }
 
-// 128-token tiles unless that leaves fewer than two workgroups per CU (256 CUs),
-// then 64-token tiles (one 32-token tile per wave); the gated pair always 64.
-// One segment with a long K (≥ 48 stages of 128) whose 128-token tiles number
-// under 512 keeps the 128-token tiles and splits K in 2 or 4 (each split ≥ 16
-// stages) while part holds the extra splits' partial sums (part_cap floats).
+void launch_gemm_add_parts(float *out, const float *part, size_t stride, int n_part, int rows, int ld, int n_tok, hipStream_t st) {
+    hipLaunchKernelGGL(gemm_add_parts_kernel, dim3((rows + 255) / 256, n_tok), dim3(256), 0, st, out, part, stride, n_part, rows, ld);
+}
+
+// 128-token tiles where that leaves two workgroups per CU (256 CUs), or where K is long
+// (≥ 48 stages of 128, one segment) and splits of ≥ 16 stages in planes leave one per CU;
+// otherwise 64-token tiles (one 32-token tile per wave), as always for the gated pair,
+// which split K as split_count allows while each split keeps 4 stages.
 template <int TY, bool GLU>
-static void launch_t(GemmP p, hipStream_t st, const GroupTiles *grp, float *part, size_t part_cap) {
+static void launch_t(GemmP p, hipStream_t st, const GroupTiles *grp, const GemmWs &ws) {
     const int tiles128 = p.n_rg * ((p.n_tok + 127) / 128);
     const int n_st = (p.K + 32 * G_KC - 1) / (32 * G_KC);
+    int nt = 1;
     p.ks = 1;
-    if (!GLU && !grp && p.nseg == 1 && part && n_st >= 48 && p.n_tok > 64) {
+    p.ws = ws;
+    if (!GLU && !grp && p.n_tok > 64) {  // GLU: two register sets of 128-token stages do not fit
         const size_t plane = (size_t)p.n_tok * p.ld[0];
-        while (p.ks < 4 && tiles128 * p.ks < 512 && n_st / (2 * p.ks) >= 16 && (size_t)(2 * p.ks - 1) * plane <= part_cap) p.ks *= 2;
-        p.part = part;
-        p.part_stride = plane;
+        const int ks = p.nseg == 1 && n_st >= 48 ? plane_count(tiles128, n_st, 16, plane, ws) : 1;
+        if (tiles128 >= 512 || (ks > 1 && tiles128 * ks >= 256)) {
+            nt = 2;
+            p.ks = ks;
+            p.plane = ks > 1 ? plane : 0;
+        }
     }
-    int nt = 2;
-    if (GLU || (p.ks == 1 && tiles128 < 512 && p.n_tok > 64)) nt = 1;  // GLU: two register sets of 128-token stages do not fit
     p.n_tg = (p.n_tok + 64 * nt - 1) / (64 * nt);
     if (grp) {  // 64-token tiles from the grouping's table
         static_assert(GROUP_BN == 64, "grouped tiles are one 32-token tile per wave");
-        nt = 1;
         p.grouped = 1;
         p.grp = *grp;
         p.n_tg = grp->max_tiles;
+    } else if (nt == 1) {
+        p.ks = split_count(p.n_rg * p.n_tg, n_st, 4, GLU ? 32 : 16, ws);
     }
     const dim3 grid(gemm_grid(p.n_rg, p.n_tg, p.ks, p.grouped));
     const bool tail = p.K % (32 * G_KC) != 0;
@@ -463,17 +471,11 @@ static void launch_t(GemmP p, hipStream_t st, const GroupTiles *grp, float *part
         else if (nt == 2) hipLaunchKernelGGL((gemm_kernel<TY, GLU, 2, false>), grid, dim3(256), 0, st, p);
         else if (tail) hipLaunchKernelGGL((gemm_kernel<TY, GLU, 1, true>), grid, dim3(256), 0, st, p);
         else hipLaunchKernelGGL((gemm_kernel<TY, GLU, 1, false>), grid, dim3(256), 0, st, p);
-        if (p.ks > 1)
-            hipLaunchKernelGGL(gemm_add_parts_kernel, dim3((p.rows[0] + 255) / 256, p.n_tok), dim3(256), 0, st, p.out[0], p.part,
-                               p.part_stride, p.ks - 1, p.rows[0], p.ld[0]);
+        if (p.plane) launch_gemm_add_parts(p.out[0], ws.part, p.plane, p.ks - 1, p.rows[0], p.ld[0], p.n_tok, st);
         return;
     }
     if (tail) hipLaunchKernelGGL((gemm_kernel<TY, GLU, 1, true>), grid, dim3(256), 0, st, p);
     else hipLaunchKernelGGL((gemm_kernel<TY, GLU, 1, false>), grid, dim3(256), 0, st, p);
-}
-
-void launch_gemm_add_parts(float *out, const float *part, size_t stride, int n_part, int rows, int ld, int n_tok, hipStream_t st) {
-    hipLaunchKernelGGL(gemm_add_parts_kernel, dim3((rows + 255) / 256, n_tok), dim3(256), 0, st, out, part, stride, n_part, rows, ld);
 }
 
 static bool operands_ok(const ActQ8 &act) { return act.qs && act.d; }
@@ -487,11 +489,11 @@ static void set_groups(GemmP &p, int nseg) {
     p.n_rg = acc;
 }
 
-bool launch_gemm(const GemvSeg *segs, int nseg, const ActQ8 &act, int n_tok, int K, hipStream_t st, const GroupTiles *grp, float *part,
-                 size_t part_cap) {
+bool launch_gemm(const GemvSeg *segs, int nseg, const ActQ8 &act, int n_tok, int K, hipStream_t st, const GroupTiles *grp,
+                 const GemmWs &ws) {
     if (nseg < 1 || nseg > 3 || n_tok < 1 || !operands_ok(act) || (grp && (nseg != 1 || grp->max_tiles < 1))) return false;
     const int ty = segs[0].w.ty;
-    if (gemm_kq_supported(ty, K)) return launch_gemm_kq(segs, nseg, act, n_tok, K, st, grp, part, part_cap);
+    if (gemm_kq_supported(ty, K)) return launch_gemm_kq(segs, nseg, act, n_tok, K, st, grp, ws);
     if (grp && grp->bn != GROUP_BN) return false;  // this kernel's grouped tiles are 64 tokens
     GemmP p{};
     for (int i = 0; i < nseg; i++) {
@@ -511,17 +513,16 @@ bool launch_gemm(const GemvSeg *segs, int nseg, const ActQ8 &act, int n_tok, int
     p.d = act.d;
     p.n_tok = n_tok;
     p.K = K;
-    if (ty == T_Q4_0) launch_t<T_Q4_0, false>(p, st, grp, part, part_cap);
-    else if (ty == T_Q5_0) launch_t<T_Q5_0, false>(p, st, grp, part, part_cap);
-    else launch_t<T_Q8_0, false>(p, st, grp, part, part_cap);
+    if (ty == T_Q4_0) launch_t<T_Q4_0, false>(p, st, grp, ws);
+    else if (ty == T_Q5_0) launch_t<T_Q5_0, false>(p, st, grp, ws);
+    else launch_t<T_Q8_0, false>(p, st, grp, ws);
     return true;
 }
 
 bool launch_gemm_glu(const DevWeight &gate, const DevWeight &up, const ActQ8 &act, int n_tok, int K, float *h, int ld, int gelu,
-                     float *scratch, hipStream_t st, const GroupTiles *grp) {
-    (void)scratch;
+                     hipStream_t st, const GroupTiles *grp, const GemmWs &ws) {
     if (grp && grp->max_tiles < 1) return false;
-    if (gemm_kq_supported(gate.ty, K)) return launch_gemm_kq_glu(gate, up, act, n_tok, K, h, ld, gelu, st, grp);
+    if (gemm_kq_supported(gate.ty, K)) return launch_gemm_kq_glu(gate, up, act, n_tok, K, h, ld, gelu, st, grp, ws);
     if (grp && grp->bn != GROUP_BN) return false;  // this kernel's grouped tiles are 64 tokens
     if (n_tok < 1 || !operands_ok(act) || gate.ty != up.ty || !gemm_supported(gate.ty, K) || gate.cols != (size_t)K ||
         up.cols != (size_t)K || gate.rows != up.rows || !gate.data || !up.data || !h)
@@ -542,9 +543,9 @@ bool launch_gemm_glu(const DevWeight &gate, const DevWeight &up, const ActQ8 &ac
     p.d = act.d;
     p.n_tok = n_tok;
     p.K = K;
-    if (gate.ty == T_Q4_0) launch_t<T_Q4_0, true>(p, st, grp, nullptr, 0);
-    else if (gate.ty == T_Q5_0) launch_t<T_Q5_0, true>(p, st, grp, nullptr, 0);
-    else launch_t<T_Q8_0, true>(p, st, grp, nullptr, 0);
+    if (gate.ty == T_Q4_0) launch_t<T_Q4_0, true>(p, st, grp, ws);
+    else if (gate.ty == T_Q5_0) launch_t<T_Q5_0, true>(p, st, grp, ws);
+    else launch_t<T_Q8_0, true>(p, st, grp, ws);
     return true;
 }
 

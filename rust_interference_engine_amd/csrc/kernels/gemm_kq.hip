@@ -45,6 +45,7 @@
 #include "../device.hpp"
 #include "../kernels.hpp"
 #include "../gemv_units.hpp"
+#include "../gemm_split.hpp"
 
 #include <type_traits>
 
@@ -75,13 +76,9 @@ struct KqP {
     int n_tok, K;
     int grouped;     // expert groups: one matrix per expert (grp), token tiles from its table
     GroupTiles grp;
-    // K split (Q6_K, one segment, not grouped): split i takes superblocks
-    // [i·nsb/ks, (i+1)·nsb/ks); split 0 runs the segment's epilogue on its partial
-    // sum, split i > 0 stores its partial to part[i-1] ([n_tok][ld], stride
-    // part_stride floats), which a second launch adds to the output in split order
-    int ks;
-    float *part;
-    size_t part_stride;
+    int ks;  // K splits of a tile (64-token tiles, not grouped), in whole superblocks
+    GemmWs ws;
+    size_t plane;  // floats per plane of a split in planes (plane_count), 0: split_sum
 };
 
 constexpr int KQ_BM = 64, KQ_BN = 64;
@@ -296,7 +293,7 @@ __global__ __launch_bounds__(256) void gemm_q45k_kernel(KqP p) {
     __shared__ KqEnd<GLU, BN> en;
     const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
     const int wr = wv / WC, wc = wv % WC;
-    constexpr bool KSPLIT = !GLU && BN == 64;
+    constexpr bool KSPLIT = BN == 64;
     const GemmTile gt = gemm_tile(blockIdx.x, p.n_rg, p.n_tg, KSPLIT ? p.ks : 1, p.grouped);
     const int rg = gt.rg, tg = gt.tg, ksi = gt.ks;
     if (rg < 0) return;  // whole workgroup: uniform
@@ -394,12 +391,18 @@ __global__ __launch_bounds__(256) void gemm_q45k_kernel(KqP p) {
         half(sb, std::integral_constant<int, 1>{});
     }
     // ---- epilogue: lane holds weight row row0 + wrow for tokens t0 + wc·32 + 16h + v ----
+    if constexpr (KSPLIT) {
+        if (p.ks > 1 && !p.plane && !split_sum(reinterpret_cast<float(&)[NW * 16]>(acc), p.ws.part, (uint32_t)(p.ws.cap * 4), p.ws.cnt,
+                                   rg * p.n_tg + tg, ksi, p.ks))
+            return;
+    }
     const int rows = p.rows[sg];
     const int row = row0 + wrow;
     if (row >= rows) return;
-    float *out = (KSPLIT && ksi) ? p.part + (size_t)(ksi - 1) * p.part_stride : p.out[sg];
+    const bool part = p.plane && ksi;
+    float *out = part ? p.ws.part + (size_t)(ksi - 1) * p.plane : p.out[sg];
     const int ld = p.ld[sg];
-    const int epi = (KSPLIT && ksi) ? EPI_STORE : p.epi[sg];
+    const int epi = part ? EPI_STORE : p.epi[sg];
 #pragma unroll
     for (int v = 0; v < 16; v++) {
         const int r = tr.r0 + wc * 32 + 16 * h + v;
@@ -591,12 +594,16 @@ __global__ __launch_bounds__(256) void gemm_q6k_kernel(KqP p) {
         half(sb, std::integral_constant<int, 0>{});
         half(sb, std::integral_constant<int, 1>{});
     }
+    if (p.ks > 1 && !p.plane && !split_sum(reinterpret_cast<float(&)[NW * 16]>(acc), p.ws.part, (uint32_t)(p.ws.cap * 4), p.ws.cnt,
+                               rg * p.n_tg + tg, ksi, p.ks))
+        return;
     const int rows = p.rows[sg];
     const int row = row0 + wrow;
     if (row >= rows) return;
-    float *out = ksi ? p.part + (size_t)(ksi - 1) * p.part_stride : p.out[sg];
+    const bool part = p.plane && ksi;
+    float *out = part ? p.ws.part + (size_t)(ksi - 1) * p.plane : p.out[sg];
     const int ld = p.ld[sg];
-    const int epi = ksi ? EPI_STORE : p.epi[sg];
+    const int epi = part ? EPI_STORE : p.epi[sg];
 #pragma unroll
     for (int v = 0; v < 16; v++) {
         const int r = tr.r0 + wc * 32 + 16 * h + v;
@@ -625,44 +632,29 @@ void kq_groups(KqP &p, int nseg, const GroupTiles *grp, int bm = KQ_BM) {
     }
 }
 
-// The non-gated 64-token form splits K as k6_launch does (below).
+// Launches of few tiles split K into parts of at least two superblocks, added up in the
+// launch; one ungated segment of under 512 tiles into parts of at least four, in planes.
 template <int TY, bool GLU, int BN = KQ_BN>
-void kq_launch(KqP p, hipStream_t st, float *part = nullptr, size_t part_cap = 0) {
-    const int tiles = p.n_rg * p.n_tg, nsb = p.K >> 8;
-    p.ks = 1;
-    if (!GLU && BN == 64 && !p.grouped && p.nseg == 1 && part && p.n_tok > 64) {
+void kq_launch(KqP p, hipStream_t st, const GemmWs &ws = {}) {
+    p.ks = p.grouped || BN != 64 ? 1 : split_count(p.n_rg * p.n_tg, p.K >> 8, 2, GLU ? 32 : 16, ws);
+    p.ws = ws;
+    if (p.ks == 1 && !GLU && BN == 64 && !p.grouped && p.nseg == 1 && p.n_tok > 64) {
         const size_t plane = (size_t)p.n_tok * p.ld[0];
-        while (p.ks < 4 && tiles * p.ks < 512 && nsb / (2 * p.ks) >= 4 && (size_t)(2 * p.ks - 1) * plane <= part_cap) p.ks *= 2;
-        p.part = part;
-        p.part_stride = plane;
+        p.ks = plane_count(p.n_rg * p.n_tg, p.K >> 8, 4, plane, ws);
+        p.plane = p.ks > 1 ? plane : 0;
     }
-    hipLaunchKernelGGL((gemm_q45k_kernel<TY, GLU, BN>), dim3(gemm_grid(p.n_rg, p.n_tg, p.ks, p.grouped)), dim3(256), 0, st, p);
-    if (p.ks > 1) launch_gemm_add_parts(p.out[0], p.part, p.part_stride, p.ks - 1, p.rows[0], p.ld[0], p.n_tok, st);
-}
-
-// A single ungrouped segment whose tiles number under 512 splits K in 2 or 4
-// (each split ≥ 4 superblocks) while part holds the extra splits' partial sums
-// (part_cap floats); the partials are added by a second launch.
-template <bool GLU>
-void k6_launch(KqP p, hipStream_t st, float *part = nullptr, size_t part_cap = 0) {
-    const int tiles = p.n_rg * p.n_tg, nsb = p.K >> 8;
-    p.ks = 1;
-    if (!GLU && !p.grouped && p.nseg == 1 && part && p.n_tok > 64) {
-        const size_t plane = (size_t)p.n_tok * p.ld[0];
-        while (p.ks < 4 && tiles * p.ks < 512 && nsb / (2 * p.ks) >= 4 && (size_t)(2 * p.ks - 1) * plane <= part_cap) p.ks *= 2;
-        p.part = part;
-        p.part_stride = plane;
-    }
-    hipLaunchKernelGGL((gemm_q6k_kernel<GLU>), dim3(gemm_grid(p.n_rg, p.n_tg, p.ks, p.grouped)), dim3(256), 0, st, p);
-    if (p.ks > 1) launch_gemm_add_parts(p.out[0], p.part, p.part_stride, p.ks - 1, p.rows[0], p.ld[0], p.n_tok, st);
+    const dim3 grid(gemm_grid(p.n_rg, p.n_tg, p.ks, p.grouped));
+    if constexpr (TY == T_Q6_K) hipLaunchKernelGGL((gemm_q6k_kernel<GLU>), grid, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((gemm_q45k_kernel<TY, GLU, BN>), grid, dim3(256), 0, st, p);
+    if (p.plane) launch_gemm_add_parts(p.out[0], ws.part, p.plane, p.ks - 1, p.rows[0], p.ld[0], p.n_tok, st);
 }
 
 }  // namespace
 
 bool gemm_kq_supported(int ty, size_t K) { return (ty == T_Q4_K || ty == T_Q5_K || ty == T_Q6_K) && K % 256 == 0 && K > 0; }
 
-bool launch_gemm_kq(const GemvSeg *segs, int nseg, const ActQ8 &act, int n_tok, int K, hipStream_t st, const GroupTiles *grp, float *part,
-                    size_t part_cap) {
+bool launch_gemm_kq(const GemvSeg *segs, int nseg, const ActQ8 &act, int n_tok, int K, hipStream_t st, const GroupTiles *grp,
+                    const GemmWs &ws) {
     if (nseg < 1 || nseg > 3 || n_tok < 1 || !act.qs || !act.d || (grp && (nseg != 1 || grp->max_tiles < 1))) return false;
     const int ty = segs[0].w.ty;
     if (ty != T_Q6_K && !act.bsums) return false;
@@ -686,15 +678,15 @@ bool launch_gemm_kq(const GemvSeg *segs, int nseg, const ActQ8 &act, int n_tok, 
     if (grp && grp->bn != KQ_BN && (grp->bn != 32 || ty != T_Q4_K)) return false;
     const bool t32 = grp && grp->bn == 32;  // 32-token tiles of a Q4_K expert grouping
     kq_groups(p, nseg, grp, t32 ? kq_bm<32>() : KQ_BM);
-    if (ty == T_Q6_K) k6_launch<false>(p, st, part, part_cap);
-    else if (ty == T_Q5_K) kq_launch<T_Q5_K, false>(p, st, part, part_cap);
+    if (ty == T_Q6_K) kq_launch<T_Q6_K, false>(p, st, ws);
+    else if (ty == T_Q5_K) kq_launch<T_Q5_K, false>(p, st, ws);
     else if (t32) kq_launch<T_Q4_K, false, 32>(p, st);
-    else kq_launch<T_Q4_K, false>(p, st, part, part_cap);
+    else kq_launch<T_Q4_K, false>(p, st, ws);
     return true;
 }
 
 bool launch_gemm_kq_glu(const DevWeight &gate, const DevWeight &up, const ActQ8 &act, int n_tok, int K, float *h, int ld, int gelu,
-                        hipStream_t st, const GroupTiles *grp) {
+                        hipStream_t st, const GroupTiles *grp, const GemmWs &ws) {
     if (grp && grp->max_tiles < 1) return false;
     if (n_tok < 1 || !act.qs || !act.d || (gate.ty != T_Q6_K && !act.bsums) || gate.ty != up.ty || !gemm_kq_supported(gate.ty, K) ||
         gate.cols != (size_t)K || up.cols != (size_t)K || gate.rows != up.rows || !gate.data || !up.data || !h)
@@ -718,10 +710,10 @@ bool launch_gemm_kq_glu(const DevWeight &gate, const DevWeight &up, const ActQ8 
     if (grp && grp->bn != KQ_BN && (grp->bn != 32 || gate.ty != T_Q4_K)) return false;
     const bool t32 = grp && grp->bn == 32;  // 32-token tiles of a Q4_K expert grouping
     kq_groups(p, 1, grp, t32 ? kq_bm<32>() : KQ_BM);
-    if (gate.ty == T_Q6_K) k6_launch<true>(p, st);
-    else if (gate.ty == T_Q5_K) kq_launch<T_Q5_K, true>(p, st);
+    if (gate.ty == T_Q6_K) kq_launch<T_Q6_K, true>(p, st, ws);
+    else if (gate.ty == T_Q5_K) kq_launch<T_Q5_K, true>(p, st, ws);
     else if (t32) kq_launch<T_Q4_K, true, 32>(p, st);
-    else kq_launch<T_Q4_K, true>(p, st);
+    else kq_launch<T_Q4_K, true>(p, st, ws);
     return true;
 }
 

@@ -52,3 +52,18 @@ def test_gated_and_grouped_k_quant_prompts_match_oracle(oracle, cuda, arch, ty):
     for t in range(70):
         err = max_rel_err(lg[t * nv:(t + 1) * nv], lo[t * nv:(t + 1) * nv])
         assert err < 0.03, f"{arch} {ty}: token {t}: {err}"
+
+
+# hidden 1024 (8 stages of 128, 4 superblocks): every launch of these prompts splits K and
+# adds its partial sums up in the launch, layer after layer on the same counters
+@pytest.mark.parametrize("arch,ty", [("llama", Q4_0), ("gemma2", Q8_0), ("qwen3", Q5_0), ("llama", Q5_K), ("gemma2", Q6_K)])
+def test_prompts_with_k_splits_match_oracle(oracle, cuda, arch, ty):
+    from naive_model import max_rel_err
+    spec, g, o = _pair(oracle, arch, ty, 0, n_ctx=96, max_batch=40, mutate=lambda s: [setattr(s, "n_embd", 1024), setattr(s, "n_ff", 2048)])
+    nv = spec.n_vocab
+    toks = [(i * 29 + 3) % nv for i in range(60)]
+    for pos, end in ((0, 20), (20, 60)):
+        lg, lo = g.forward(toks[pos:end], pos, True), o.forward(toks[pos:end], pos, True)
+        for t in range(end - pos):
+            err = max_rel_err(lg[t * nv:(t + 1) * nv], lo[t * nv:(t + 1) * nv])
+            assert err < 0.03, f"{arch} {ty}: token {pos + t}: {err}"
