@@ -122,15 +122,21 @@ constexpr int prompt_lds_bytes() {
 
 // NW groups of 4 waves: group q handles the tiles q, q + NW, …, and the groups'
 // online-softmax states are merged through LDS at the end.
-template <int HD, int NW, int KVT>
+// DS = 2 (head dim 2·HD): the two groups take the same tiles, group q the dims HD·q ..
+// HD·q + HD − 1 of queries, keys, values and outputs, since the fragments of 256 dims do
+// not fit a wave's registers.  Each forms its half of the scores, the halves are added
+// through LDS, and both run the same softmax.
+template <int HD, int NW, int KVT, int DS = 1>
 __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
+    static_assert(DS == 1 || (DS == 2 && NW == 2 && KVT != 2), "one group per half of the dims");
+    constexpr int FHD = HD * DS, NT = DS == 2 ? 1 : NW;  // head dim; groups that share out the tiles
     static_assert(KVT != 2 || HD == 128, "Turbo4 tiles: one 128-dim rotation block per row");
     constexpr int KS = HD / 16;          // 16-dim k-steps of the score product
     constexpr int DT = HD / 32;          // 32-dim output tiles
     constexpr int KROW = (KVT == 1 ? HD : HD * 2) + 16;  // bytes per K row in LDS (padded)
     constexpr int NCH = (PT * HD / (KVT == 1 ? 16 : 8) + 255) / 256;  // 16-byte K chunks per thread per tile
     constexpr int NV = (2 * HD + 255) / 256;             // V pieces (two positions × 8 dims) per thread per tile
-    constexpr int RB = KVT == 1 ? HD / 32 * 34 : KVT == 2 ? HD / 2 : HD * 2;  // cache row bytes
+    constexpr int RB = KVT == 1 ? FHD / 32 * 34 : KVT == 2 ? FHD / 2 : FHD * 2;  // cache row bytes
     extern __shared__ __align__(16) uint8_t lds[];
     constexpr int TB = tile_bytes<HD, KVT>();
     const int grp = threadIdx.x >> 8;
@@ -147,7 +153,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     const int tb = tr * tbw + wv / wpt;   // this wave's 32-token block
     const bool wave_on = wv < wpt * tbw && j < G && tb * 32 < a.n_tok;
     const int pos0 = a.pos0;
-    const int hd = HD, qd = a.n_head * HD;
+    const int hd = FHD, qd = a.n_head * FHD, dim0 = DS == 2 ? HD * grp : 0;
     const int head = g * G + j;
 
     // token of this lane and its visible positions [start_t, pos_t]
@@ -179,7 +185,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     i32x4 q8[KVT == 1 ? DT : 1];  // Q8_0: codes 16h .. +16 of each block, and the blocks' scales in log2 units
     float dq[KVT == 1 ? DT : 1];
     if constexpr (KVT == 1) {
-        const float *qrow = a.q + (size_t)(tok_ok ? t : a.n_tok - 1) * qd + (size_t)(wave_on ? head : 0) * hd + 16 * h;
+        const float *qrow = a.q + (size_t)(tok_ok ? t : a.n_tok - 1) * qd + (size_t)(wave_on ? head : 0) * hd + dim0 + 16 * h;
 #pragma unroll
         for (int b = 0; b < DT; b++) {
             float x[16], amax = 0.0f;
@@ -208,7 +214,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
         }
     } else {
         const int tq = tok_ok ? t : (a.n_tok - 1);
-        const float *qrow = a.q + (size_t)tq * qd + (size_t)(wave_on ? head : 0) * hd;
+        const float *qrow = a.q + (size_t)tq * qd + (size_t)(wave_on ? head : 0) * hd + dim0;
 #pragma unroll
         for (int s = 0; s < KS; s++) {
             const f32x4 x0 = *(const f32x4 *)(qrow + 16 * s + 8 * h);
@@ -218,8 +224,9 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
         }
     }
 
-    const uint8_t *kc = a.k_cache + (size_t)g * a.slots * RB;
-    const uint8_t *vc = a.v_cache + (size_t)g * a.slots * RB;
+    const int row0 = KVT == 1 ? dim0 / 32 * 34 : dim0 * 2;  // this group's dims in a row
+    const uint8_t *kc = a.k_cache + (size_t)g * a.slots * RB + (DS == 2 ? row0 : 0);
+    const uint8_t *vc = a.v_cache + (size_t)g * a.slots * RB + (DS == 2 ? row0 : 0);
     const uint16_t *ksc = KVT == 2 ? a.k_scale + (size_t)g * a.slots : nullptr;
     const uint16_t *vsc = KVT == 2 ? a.v_scale + (size_t)g * a.slots : nullptr;
     // one tile in flight in registers: f16 K as 16-byte row chunks and V as two
@@ -287,7 +294,8 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     };
     // Q8_0: blocks of 32 dims with values past the f16 range, found by the first run over
     // the tiles; their values are then staged ×2^-8 and their outputs multiplied by 2^8
-    __shared__ int vbig[KVT == 1 ? DT : 1];
+    __shared__ int vbig[KVT == 1 ? DT * DS : 1];
+    const int vb0 = DS == 2 ? DT * grp : 0;  // this group's first block
     uint32_t vsmall = 0;  // bit b: block b is staged ×2^-8
     auto stage = [&](const Regs &r, int buf) {
         uint8_t *kb = tiles + buf * TB, *vb = kb + PT * KROW;
@@ -342,7 +350,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
                 const int b = vi >> 6;
                 const float f = (vsmall >> b & 1) ? 1.0f / 256.0f : 1.0f;
                 const float d0 = h2f(r.vsc[c][0]), d1 = h2f(r.vsc[c][1]);
-                if (fmaxf(fabsf(d0), fabsf(d1)) > 512.0f) vbig[b] = 1;
+                if (fmaxf(fabsf(d0), fabsf(d1)) > 512.0f) vbig[vb0 + b] = 1;
                 uint8_t *dst = vb + 8 * (vi >> 4) * VROW + 4 * (vi & 15);
 #pragma unroll
                 for (int i = 0; i < 8; i++) {  // one dword = the two positions of one dim
@@ -378,23 +386,24 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     float m, l_half;
     f32x16 o[DT];
 
-    // group tile i is T(i) = t_lo + grp + i·NW; buffer i & 1 holds T(i) during iteration
+    const int tg0 = DS == 2 ? 0 : grp;
+    // group tile i is T(i) = t_lo + grp + i·NW (t_lo + i with DS = 2); buffer i & 1 holds T(i) during iteration
     // i, and the register sets hold T(i+1) and T(i+2) (issued two iterations before
     // their use)
-    const int n_iter = (t_hi - t_lo + NW - 1) / NW;
+    const int n_iter = (t_hi - t_lo + NT - 1) / NT;
     const int last = max(n_tiles - 1, 0);
     auto body = [&](int it, Regs &x) {
-        const int tile = t_lo + grp + it * NW;
+        const int tile = t_lo + tg0 + it * NT;
         stage(x, (it + 1) & 1);
-        fetch(min(tile + 3 * NW, last), x);
+        fetch(min(tile + 3 * NT, last), x);
         k_s = tiles + (it & 1) * TB;
         v_s = k_s + PT * KROW;
         const float *fk = (const float *)(v_s + HD * VROW), *fv = fk + PT;  // Turbo4 row factors
         const int P0 = k0 + tile * PT;
         const bool work = tile < n_tiles && wave_on && P0 <= w_pmax && P0 + PT - 1 >= w_smin;
+        f32x16 s = {}, s2 = {};
         if (work) {
             // Sᵀ[pos][tok] = Σ_d K[pos][d]·q[tok][d]; the hi and lo halves of q in two chains
-            f32x16 s = {}, s2 = {};
             if constexpr (KVT == 1) {
                 const float *dk = (const float *)(v_s + 2 * HD * VROW) + 4 * h;
 #pragma unroll
@@ -424,6 +433,26 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
                 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qh[ks], s, 0, 0, 0);
                 s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, ql[ks], s2, 0, 0, 0);
             }
+        }
+        if constexpr (DS == 2) {  // the other half of the dims: wave wv of the other group, the same token and positions
+            f32x4 *ex = (f32x4 *)(lds + 2 * NW * TB);
+            if (work) {
+                s += s2;
+                s2 = f32x16{};
+#pragma unroll
+                for (int q4 = 0; q4 < 4; q4++) ex[(grp * 4 + q4) * 256 + tid] = f32x4{s[4 * q4], s[4 * q4 + 1], s[4 * q4 + 2], s[4 * q4 + 3]};
+            }
+            lds_barrier();
+            if (work) {
+#pragma unroll
+                for (int q4 = 0; q4 < 4; q4++) {
+                    const f32x4 y = ex[((grp ^ 1) * 4 + q4) * 256 + tid];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) s[4 * q4 + e] += y[e];
+                }
+            }
+        }
+        if (work) {
             if constexpr (KVT == 2) {
 #pragma unroll
                 for (int v = 0; v < 16; v++) s[v] = (s[v] + s2[v]) * fk[8 * (v >> 2) + 4 * h + (v & 3)];
@@ -521,10 +550,10 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
         // tile; an empty split loads tile 0) so that every wait for a register set is an
         // exact count of the loads issued after it.
         Regs ra, rb;
-        fetch(min(t_lo + grp, last), ra);
+        fetch(min(t_lo + tg0, last), ra);
         stage(ra, 0);
-        fetch(min(t_lo + grp + NW, last), rb);
-        fetch(min(t_lo + grp + 2 * NW, last), ra);
+        fetch(min(t_lo + tg0 + NT, last), rb);
+        fetch(min(t_lo + tg0 + 2 * NT, last), ra);
         __syncthreads();
         // an even number of steps (the last one may be idle), so that the loop has one
         // entry path per register set and every wait count is exact
@@ -534,14 +563,17 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
         }
     };
     if constexpr (KVT == 1) {
-        if (threadIdx.x < DT) vbig[threadIdx.x] = 0;
+        if (threadIdx.x < DT * DS) vbig[threadIdx.x] = 0;
         __syncthreads();
         for (int again = 0;; again = 1) {
             run();  // ends with a barrier after the last staging, or stages tile 0 ahead of its only one
             if (again) break;
 #pragma unroll
-            for (int b = 0; b < DT; b++) vsmall |= (uint32_t)(vbig[b] != 0) << b;
-            if (!vsmall) break;
+            for (int b = 0; b < DT; b++) vsmall |= (uint32_t)(vbig[vb0 + b] != 0) << b;
+            int any = 0;
+#pragma unroll
+            for (int b = 0; b < DT * DS; b++) any |= vbig[b];
+            if (!any) break;  // the same for the whole workgroup
             __syncthreads();  // every flag is read before the second run's staging
         }
 #pragma unroll
@@ -550,7 +582,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     } else {
         run();
     }
-    if constexpr (NW > 1) {  // merge the groups' states into group 0 (the tile buffers are free now)
+    if constexpr (NT > 1) {  // merge the groups' states into group 0 (the tile buffers are free now)
         float *ms = (float *)lds, *ls = ms + NW * 256, *os = ls + NW * 256;
         ms[grp * 256 + tid] = m;
         ls[grp * 256 + tid] = l_half;
@@ -601,9 +633,9 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
                     f32x4 w4;
 #pragma unroll
                     for (int e = 0; e < 4; e++) w4[e] = o[d][4 * q4 + e] * osc;
-                    *(f32x4 *)(pp + 32 * d + 8 * q4 + 4 * h) = w4;
+                    *(f32x4 *)(pp + dim0 + 32 * d + 8 * q4 + 4 * h) = w4;
                 }
-            if (h == 0) {
+            if (h == 0 && (DS == 1 || grp == 0)) {
                 pp[hd] = m == -INFINITY ? -INFINITY : m * LN2_F;
                 pp[hd + 1] = l_tot;
             }
@@ -674,7 +706,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
 #pragma unroll
         for (int v = 0; v < 16; v++) y[v] = KVT == 2 ? o[d][v] : o[d][v] * inv;
         if (tok_ok) {
-            float *dst = a.att + (size_t)t * qd + (size_t)head * hd + 32 * d + 4 * h;
+            float *dst = a.att + (size_t)t * qd + (size_t)head * hd + dim0 + 32 * d + 4 * h;
 #pragma unroll
             for (int q4 = 0; q4 < 4; q4++) {
                 f32x4 w4;
@@ -708,7 +740,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
             su += xor_i<32>(su);
             scl += xor_i<32>(scl);
             if (tok_ok) {
-                const size_t e0 = (size_t)t * qd + (size_t)head * hd + 32 * d;
+                const size_t e0 = (size_t)t * qd + (size_t)head * hd + dim0 + 32 * d;
 #pragma unroll
                 for (int q4 = 0; q4 < 4; q4++) *(uint32_t *)(a.att_q.qs + e0 + 8 * q4 + 4 * h) = packed[q4];
                 if (h == 0) {
@@ -722,13 +754,14 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     }
 }
 
-template <int HD, int NW, int KVT>
+template <int HD, int NW, int KVT, int DS = 1>
 void launch_nw(const AttnArgs &a, dim3 grid, hipStream_t st) {
-    constexpr int lds = prompt_lds_bytes<HD, NW, KVT>();
-    static const bool attr = hipFuncSetAttribute((const void *)attn_prompt_f16_kernel<HD, NW, KVT>,
+    // DS = 2: the two groups' scores behind the tiles
+    constexpr int lds = DS == 2 ? 2 * NW * tile_bytes<HD, KVT>() + 2 * 256 * 64 : prompt_lds_bytes<HD, NW, KVT>();
+    static const bool attr = hipFuncSetAttribute((const void *)attn_prompt_f16_kernel<HD, NW, KVT, DS>,
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
     (void)attr;
-    hipLaunchKernelGGL((attn_prompt_f16_kernel<HD, NW, KVT>), grid, dim3(256 * NW), lds, st, a);
+    hipLaunchKernelGGL((attn_prompt_f16_kernel<HD, NW, KVT, DS>), grid, dim3(256 * NW), lds, st, a);
 }
 
 // Turbo4 query of one (token, head) per wave (turbo.rs:103-112, then the x86
@@ -778,21 +811,22 @@ __global__ __launch_bounds__(64) void turbo_query_kernel(const float *__restrict
 bool attention_prompt_mfma_ok(const AttnArgs &a) {
     const int G = a.n_kv > 0 ? a.n_head / a.n_kv : 0;
     const bool cache_ok = a.kv_type == 0 || a.kv_type == 1 || (a.kv_type == 2 && a.hd == 128 && a.turbo_signs && a.k_scale && a.v_scale && a.part);
-    return cache_ok && a.n_tok > 1 && !a.d_pos0 && a.slots >= 32 && (a.hd == 32 || a.hd == 64 || a.hd == 96 || a.hd == 128 || (a.hd == 256 && a.kv_type == 1)) && G >= 1 &&
+    return cache_ok && a.n_tok > 1 && !a.d_pos0 && a.slots >= 32 && (a.hd == 32 || a.hd == 64 || a.hd == 96 || a.hd == 128 || (a.hd == 256 && a.kv_type != 2)) && G >= 1 &&
            G <= 8 && a.n_head == G * a.n_kv && (a.att_fmt != ACT_Q8_0 || (a.att_q.qs && a.att_q.d));
 }
 
 // KV splits of a launch, merged by a second kernel: at least 16 tiles of 32 positions
-// each, up to about two workgroups per CU, at most 16.  Rows under 1024 positions keep
-// one pass where the grid has 64 workgroups or more: at a 512-token prompt from position
-// 0, two splits (8 tiles each) and the merge launch measured 29.3 k tok/s against 31.1 k
-// (128 workgroups), 80 against 84 k (64).  Smaller grids (a few drafted tokens, one KV
-// head) take splits of at least 4 tiles: 5 tokens at 900, 8 workgroups, 39 us in one pass.
+// each, up to about two workgroups per CU, at most 16.  Grids under 64 workgroups take
+// splits of at least 2 tiles, up to one workgroup per CU (650 tokens of gemma-3-1b, 21
+// workgroups, six layers: 1579 us in one pass with the per-token kernel, 1369 us in splits
+// of 4 tiles, 1323 us in splits of 2).  From 64 on, splits of fewer than 16 tiles measured
+// no better than one pass (512 tokens at 0, 128 workgroups: 1149 against 1142 us).
 static int prompt_kv_splits(const AttnArgs &a, const dim3 &grid, int tokens_per_wg) {
     int longest = (a.pos0 + a.n_tok - 1) / PT + 1;  // tiles of the last query row
     if (a.window > 0) longest = std::min(longest, (a.window + tokens_per_wg - 2) / PT + 2);
     const int wgs = (int)(grid.x * grid.y);
-    return std::max({1, std::min({16, longest / 16, 512 / wgs}), std::min({16, longest / 4, 64 / wgs})});
+    const int by_work = wgs < 64 ? longest / 2 : longest / 16, by_grid = wgs < 64 ? 256 / wgs : 512 / wgs;
+    return std::max(1, std::min({16, by_work, by_grid}));
 }
 
 bool launch_attention_prompt_mfma(const AttnArgs &a, hipStream_t st) {
@@ -817,14 +851,15 @@ bool launch_attention_prompt_mfma(const AttnArgs &a, hipStream_t st) {
         case 64: launch_nw<64, 2, 1>(b, grid, st); break;
         case 96: launch_nw<96, 2, 1>(b, grid, st); break;
         case 128: launch_nw<128, 2, 1>(b, grid, st); break;
-        default: launch_nw<256, 1, 1>(b, grid, st); break;
+        default: launch_nw<128, 2, 1, 2>(b, grid, st); break;
         }
     } else {
         switch (a.hd) {
         case 32: launch_nw<32, 2, 0>(b, grid, st); break;
         case 64: launch_nw<64, 2, 0>(b, grid, st); break;
         case 96: launch_nw<96, 2, 0>(b, grid, st); break;
-        default: launch_nw<128, 2, 0>(b, grid, st); break;
+        case 128: launch_nw<128, 2, 0>(b, grid, st); break;
+        default: launch_nw<128, 2, 0, 2>(b, grid, st); break;
         }
     }
     if (S > 1) launch_attention_combine(b, st);
