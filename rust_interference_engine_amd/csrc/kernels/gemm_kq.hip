@@ -380,7 +380,7 @@ __global__ __launch_bounds__(256) void gemm_q45k_kernel(KqP p) {
                 // block 1: lanes 32-63, dmin)
                 const v32f pp = __builtin_amdgcn_mfma_f32_32x32x1f32(en.da[arow], h == 0 ? en.wd[a][wrow] : en.wdm[a][wrow], zf32, 0, 0, 0);
 #pragma unroll
-                for (int v = 0; v < 16; v++) acc[a][v] = fmaf(pp[v], (float)s1[a][v], fmaf(-pp[16 + v], s2[v], acc[a][v]));
+                for (int v = 0; v < 16; v++) acc[a][v] += pp[v] * (float)s1[a][v] - pp[16 + v] * s2[v];
             }
         }
         if (more) kq_store<TY, GLU, BN, 1 - hs>(st[1 - hs], en, tid, R);
