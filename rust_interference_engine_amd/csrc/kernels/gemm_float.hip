@@ -22,10 +22,10 @@
 // against 0.95 / 1.01 / 1.23 in the batched GEMV.
 //
 // Bound: three MFMAs per product, ~830 TFLOP/s of useful rate, or the weight bytes for
-// short prompts; measured 190 TFLOP/s (203 tokens, gate/up 2 × 9728 × 2560: 110 us),
+// short prompts; measured 180 TFLOP/s (203 tokens, gate/up 2 × 9728 × 2560: 110 us),
 // held by LDS operand reads and by the waits between a stage's reads and its MFMAs.  The
 // prompt through two layers of hidden 2560: 6.20 ms in the batched GEMV, which reads the
-// weights once per 4 tokens, 0.77 ms here.
+// weights once per 4 tokens, 0.76 ms here.
 #include "../common.hpp"
 #include "../device.hpp"
 #include "../kernels.hpp"

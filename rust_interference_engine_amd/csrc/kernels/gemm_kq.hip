@@ -31,7 +31,7 @@
 // multiply loop reads its B operand without the nibble shifts of Q4_K, for 64 more LDS
 // bytes per row.  Bound like Q4_K by the int32 scale multiply-adds between the MFMAs.
 // A 421-token prompt through two layers of hidden 3072 (Q5_K, V and one down
-// projection Q6_K) takes 768 µs, against 7439 µs with its Q5_K weights in the batched
+// projection Q6_K) takes 778 µs, against 7439 µs with its Q5_K weights in the batched
 // GEMV, which reads and unpacks every weight once per 4 tokens.
 //
 // Q6_K weights × Q8_K activations (kernels/avx2.rs dot_q6_k 109-151): per
@@ -380,7 +380,13 @@ __global__ __launch_bounds__(256) void gemm_q45k_kernel(KqP p) {
                 // block 1: lanes 32-63, dmin)
                 const v32f pp = __builtin_amdgcn_mfma_f32_32x32x1f32(en.da[arow], h == 0 ? en.wd[a][wrow] : en.wdm[a][wrow], zf32, 0, 0, 0);
 #pragma unroll
-                for (int v = 0; v < 16; v++) acc[a][v] += pp[v] * (float)s1[a][v] - pp[16 + v] * s2[v];
+                for (int v = 0; v < 16; v++) {
+                    // Q5_K: two rounding steps less (gate/up 2 × 8192 × 3072, 421 tokens: 91
+                    // against 95 µs); Q4_K keeps the roundings its prompts always had, since
+                    // others move near-tied expert choices
+                    if constexpr (TY == T_Q5_K) acc[a][v] = fmaf(pp[v], (float)s1[a][v], fmaf(-pp[16 + v], s2[v], acc[a][v]));
+                    else acc[a][v] += pp[v] * (float)s1[a][v] - pp[16 + v] * s2[v];
+                }
             }
         }
         if (more) kq_store<TY, GLU, BN, 1 - hs>(st[1 - hs], en, tid, R);
