@@ -105,8 +105,8 @@ void launch_attention(const AttnArgs &a, hipStream_t st);
 bool attention_fused_ok(const AttnArgs &a);
 bool launch_attention_fused(const AttnArgs &a, const HeadPrepArgs &hp, hipStream_t st);
 // ---- attn_prompt.hip ----
-// Prompt batches over an f16 cache on f16 matrix cores (one launch, no range
-// partials); false when the shape or cache type is not covered.
+// Prompt batches on the matrix cores, over f16 and Q8_0 caches (head sizes 32, 64, 96,
+// 128, 256) and Turbo4 ones (128); false when the shape or cache type is not covered.
 bool attention_prompt_mfma_ok(const AttnArgs &a);
 bool launch_attention_prompt_mfma(const AttnArgs &a, hipStream_t st);
 // Merge of a.n_split range partials per (token, head) [t][head][split][hd + 2]

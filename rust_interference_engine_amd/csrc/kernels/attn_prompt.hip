@@ -1,6 +1,6 @@
-// attn_prompt.hip — causal grouped-query attention of a prompt batch over an f16
-// KV cache on CDNA4 f16 matrix cores (flash-attention form, one pass, no range
-// partials).  Reference semantics: crates/rie-core/src/model/cpu.rs:550-634
+// attn_prompt.hip — causal grouped-query attention of a prompt batch over an f16,
+// Q8_0 or Turbo4 KV cache on CDNA4 matrix cores (flash-attention form; long rows and
+// small grids in splits that a second kernel merges).  Reference semantics: crates/rie-core/src/model/cpu.rs:550-634
 // (scores q·k in f32 over positions start..=pos, optional softcap, softmax,
 // out = Σ p·v), with the KV rows at slot pos % slots (cpu.rs:304, 577).
 //
