@@ -24,10 +24,14 @@
 // v_mfma_i32_32x32x32_i8, and a score is Σ_b (d_k·isum)·d_q over its blocks.  A value
 // row's d·code has at most 18 significant bits, so it is staged as two f16 halves
 // without rounding and P·V takes the four products of its halves and the probability's.
-// A block of 32 dims whose values leave the f16 range (|d| > 512 somewhere) is found
-// at its staging; the workgroup then runs its tiles once more with that block's values
-// times 2^-8.  (512 tokens at 7680, 32 heads of 128: 2360 us per layer in
-// attn_split_kernel, a workgroup per token and KV head on the vector units.)
+// (512 tokens at 7680, 32 heads of 128: 2360 us per layer in attn_split_kernel, a
+// workgroup per token and KV head on the vector units.)
+//
+// Values that the matrix product may not see (Q8_0 caches, and f16 ones at head size
+// 256): an infinity or NaN, which would reach the tokens that do not see its position
+// (probability 0 times infinity), and Q8_0 blocks that leave the f16 range (|d| > 512).
+// Staging finds them; the workgroup then runs its tiles once more with zeros in their
+// place and adds their products on the vector units, for the tokens that see them.
 //
 // Work split: a workgroup (4 waves) owns one KV head and a block of query rows;
 // each wave owns 32 tokens of one query head.  Scores are computed transposed,
@@ -104,6 +108,7 @@ struct __attribute__((packed, aligned(2))) Codes16 {
 struct __attribute__((packed, aligned(2))) Codes8 {
     uint32_t w[2];
 };
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float code_f(uint32_t w, int e) { return (float)(int)(int8_t)((w >> (8 * e)) & 0xff); }
 
 // LDS bytes of one wave group's K and transposed V tile (+ the rows' score and
@@ -292,12 +297,15 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
             }
         }
     };
-    // Q8_0: blocks of 32 dims with values past the f16 range, found by the first run over
-    // the tiles; their values are then staged ×2^-8 and their outputs multiplied by 2^8
-    __shared__ int vbig[KVT == 1 ? DT * DS : 1];
-    const int vb0 = DS == 2 ? DT * grp : 0;  // this group's first block
-    uint32_t vsmall = 0;  // bit b: block b is staged ×2^-8
-    auto stage = [&](const Regs &r, int buf) {
+    // CHECK: look for values that the matrix product may not see (see the top).  The
+    // first run over the tiles (APART false) reports them in odd_seen; in the second they
+    // are staged as zeros and their products added apart.
+    constexpr bool CHECK = KVT == 1 || DS == 2;
+    __shared__ int odd_seen;
+    auto odd_scale = [](float d) { return !(fabsf(d) <= 512.0f); };        // of a Q8_0 block
+    auto odd_half = [](uint32_t b) { return (b & 0x7C00u) == 0x7C00u; };   // an infinite or NaN f16
+    auto stage = [&](const Regs &r, int buf, auto apart) {
+        constexpr bool APART = decltype(apart)::value;
         uint8_t *kb = tiles + buf * TB, *vb = kb + PT * KROW;
         if constexpr (KVT == 2) {
             // K row tid/8: code bytes 8c..8c+8 (c = tid%8) of chunk c/2 hold dims
@@ -347,14 +355,17 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
             for (int c = 0; c < NV; c++) {
                 const int vi = tid + 256 * c;
                 if (vi >= 2 * HD) continue;
-                const int b = vi >> 6;
-                const float f = (vsmall >> b & 1) ? 1.0f / 256.0f : 1.0f;
-                const float d0 = h2f(r.vsc[c][0]), d1 = h2f(r.vsc[c][1]);
-                if (fmaxf(fabsf(d0), fabsf(d1)) > 512.0f) vbig[vb0 + b] = 1;
+                float d0 = h2f(r.vsc[c][0]), d1 = h2f(r.vsc[c][1]);
+                if constexpr (APART) {
+                    d0 = odd_scale(d0) ? 0.0f : d0;
+                    d1 = odd_scale(d1) ? 0.0f : d1;
+                } else if (odd_scale(d0) || odd_scale(d1)) {
+                    odd_seen = 1;
+                }
                 uint8_t *dst = vb + 8 * (vi >> 4) * VROW + 4 * (vi & 15);
 #pragma unroll
                 for (int i = 0; i < 8; i++) {  // one dword = the two positions of one dim
-                    const float x0 = code_f(r.v[c][0][i >> 2], i & 3) * (d0 * f), x1 = code_f(r.v[c][1][i >> 2], i & 3) * (d1 * f);
+                    const float x0 = code_f(r.v[c][0][i >> 2], i & 3) * d0, x1 = code_f(r.v[c][1][i >> 2], i & 3) * d1;
                     const auto hi = __builtin_amdgcn_cvt_pkrtz(x0, x1);  // cut off: the rest fits 11 bits
                     const auto lo = __builtin_amdgcn_cvt_pkrtz(x0 - (float)hi[0], x1 - (float)hi[1]);
                     *(uint32_t *)(dst + i * VROW) = __builtin_bit_cast(uint32_t, hi);
@@ -373,10 +384,18 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
             const int vi = tid + 256 * c;
             if (vi >= 2 * HD) continue;
             uint8_t *dst = vb + 8 * (vi >> 4) * VROW + 4 * (vi & 15);
+            if constexpr (CHECK && !APART) {  // the largest magnitudes' bits, two halves at a time
+                u16x2 big = {0, 0};
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+                    big = __builtin_elementwise_max(big, __builtin_bit_cast(u16x2, r.v[c][i >> 2][i & 3] & 0x7FFF7FFFu));
+                if (big[0] >= 0x7C00 || big[1] >= 0x7C00) odd_seen = 1;
+            }
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 const uint32_t w0 = r.v[c][0][i >> 1], w1 = r.v[c][1][i >> 1];
-                const uint32_t pair = (i & 1) ? ((w0 >> 16) | (w1 & 0xFFFF0000u)) : ((w0 & 0xFFFFu) | (w1 << 16));
+                uint32_t pair = (i & 1) ? ((w0 >> 16) | (w1 & 0xFFFF0000u)) : ((w0 & 0xFFFFu) | (w1 << 16));
+                if constexpr (CHECK && APART) pair &= (odd_half(pair) ? 0u : 0xFFFFu) | (odd_half(pair >> 16) ? 0u : 0xFFFF0000u);
                 *(uint32_t *)(dst + i * VROW) = pair;
             }
         }
@@ -386,15 +405,59 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     float m, l_half;
     f32x16 o[DT];
 
+    // o += p·v over the values of the tile at position P0 that are staged as zeros; pv:
+    // this lane's probabilities of positions P0 + 8(v/4) + 4h + v%4
+    auto add_apart = [&](int P0, f32x16 pv) {
+        const int span = p_hi - P0;
+        auto vrow = [&](int off) { return vc + (size_t)((P0 + min(off, span)) % a.slots) * RB; };
+        bool odd = false;  // position lane % 32, half h of the dims (blocks h, h + 2, … of Q8_0)
+        if constexpr (KVT == 1) {
+            for (int b = h; b < DT; b += 2) odd |= odd_scale(h2f(*(const uint16_t *)(vrow(col) + b * 34)));
+        } else {
+            for (int i = h; i < HD / 4; i += 2) {
+                const uint2 x = ((const uint2 *)vrow(col))[i];
+                odd |= odd_half(x.x) || odd_half(x.x >> 16) || odd_half(x.y) || odd_half(x.y >> 16);
+            }
+        }
+        const uint64_t both = __builtin_amdgcn_ballot_w64(odd);
+        for (uint32_t left = (uint32_t)both | (uint32_t)(both >> 32); left; left &= left - 1) {
+            const int j = __builtin_ctz(left);  // wave-uniform
+            const float mine = pv[4 * (j >> 3) + (j & 3)], other = xor_f<32>(mine);
+            const float p = (j >> 2 & 1) == h ? mine : other;
+            if (!(tok_ok && P0 + j >= start_t && P0 + j <= pos_t)) continue;
+            const uint8_t *r = vrow(j);
+#pragma unroll
+            for (int d = 0; d < DT; d++)
+#pragma unroll
+                for (int q4 = 0; q4 < 4; q4++) {
+                    if constexpr (KVT == 1) {
+                        const float sc = h2f(*(const uint16_t *)(r + 34 * d));
+                        const uint16_t *c = (const uint16_t *)(r + 34 * d + 2 + 8 * q4 + 4 * h);
+                        const uint32_t w = c[0] | (uint32_t)c[1] << 16;
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            if (odd_scale(sc)) o[d][4 * q4 + e] = fmaf(p, code_f(w, e) * sc, o[d][4 * q4 + e]);
+                    } else {
+                        const uint2 x = *(const uint2 *)(r + (32 * d + 8 * q4 + 4 * h) * 2);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            const uint32_t b = ((e < 2 ? x.x : x.y) >> (16 * (e & 1))) & 0xFFFFu;
+                            if (odd_half(b)) o[d][4 * q4 + e] = fmaf(p, h2f(b), o[d][4 * q4 + e]);
+                        }
+                    }
+                }
+        }
+    };
+
     const int tg0 = DS == 2 ? 0 : grp;
     // group tile i is T(i) = t_lo + grp + i·NW (t_lo + i with DS = 2); buffer i & 1 holds T(i) during iteration
     // i, and the register sets hold T(i+1) and T(i+2) (issued two iterations before
     // their use)
     const int n_iter = (t_hi - t_lo + NT - 1) / NT;
     const int last = max(n_tiles - 1, 0);
-    auto body = [&](int it, Regs &x) {
+    auto body = [&](int it, Regs &x, auto apart) {
         const int tile = t_lo + tg0 + it * NT;
-        stage(x, (it + 1) & 1);
+        stage(x, (it + 1) & 1, apart);
         fetch(min(tile + 3 * NT, last), x);
         k_s = tiles + (it & 1) * TB;
         v_s = k_s + PT * KROW;
@@ -538,10 +601,16 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
                     }
                 }
             }
+            if constexpr (decltype(apart)::value) {
+                f32x16 pw;
+#pragma unroll
+                for (int v = 0; v < 16; v++) pw[v] = pv[v];
+                add_apart(P0, pw);
+            }
         }
         __syncthreads();
     };
-    auto run = [&]() {
+    auto run = [&](auto apart) {
         m = -INFINITY;
         l_half = 0.0f;
 #pragma unroll
@@ -551,36 +620,24 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
         // exact count of the loads issued after it.
         Regs ra, rb;
         fetch(min(t_lo + tg0, last), ra);
-        stage(ra, 0);
+        stage(ra, 0, apart);
         fetch(min(t_lo + tg0 + NT, last), rb);
         fetch(min(t_lo + tg0 + 2 * NT, last), ra);
         __syncthreads();
         // an even number of steps (the last one may be idle), so that the loop has one
         // entry path per register set and every wait count is exact
         for (int it = 0; it < n_iter; it += 2) {
-            body(it, rb);
-            body(it + 1, ra);
+            body(it, rb, apart);
+            body(it + 1, ra, apart);
         }
     };
-    if constexpr (KVT == 1) {
-        if (threadIdx.x < DT * DS) vbig[threadIdx.x] = 0;
+    if constexpr (CHECK) {
+        if (threadIdx.x == 0) odd_seen = 0;
         __syncthreads();
-        for (int again = 0;; again = 1) {
-            run();  // ends with a barrier after the last staging, or stages tile 0 ahead of its only one
-            if (again) break;
-#pragma unroll
-            for (int b = 0; b < DT; b++) vsmall |= (uint32_t)(vbig[vb0 + b] != 0) << b;
-            int any = 0;
-#pragma unroll
-            for (int b = 0; b < DT * DS; b++) any |= vbig[b];
-            if (!any) break;  // the same for the whole workgroup
-            __syncthreads();  // every flag is read before the second run's staging
-        }
-#pragma unroll
-        for (int d = 0; d < DT; d++)
-            if (vsmall >> d & 1) o[d] *= 256.0f;
+        run(std::false_type{});  // its last barrier follows every staging
+        if (odd_seen) run(std::true_type{});  // the same for the whole workgroup
     } else {
-        run();
+        run(std::false_type{});
     }
     if constexpr (NT > 1) {  // merge the groups' states into group 0 (the tile buffers are free now)
         float *ms = (float *)lds, *ls = ms + NW * 256, *os = ls + NW * 256;
