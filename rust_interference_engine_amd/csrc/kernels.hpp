@@ -97,6 +97,7 @@ struct AttnArgs {
     const int *d_pos0;
     const float *turbo_signs;
     int *counters;               // fused single-token path: [n_head · ATT_CNT_STRIDE] zeroed ints, left zeroed
+    int part_log2 = 0;           // the range maxima in part are in log2 units, not natural ones
 };
 constexpr int ATT_CNT_STRIDE = 32;  // ints between the arrival counters of the head slices
 void launch_attention(const AttnArgs &a, hipStream_t st);
@@ -110,7 +111,7 @@ bool launch_attention_fused(const AttnArgs &a, const HeadPrepArgs &hp, hipStream
 bool attention_prompt_mfma_ok(const AttnArgs &a);
 bool launch_attention_prompt_mfma(const AttnArgs &a, hipStream_t st);
 // Merge of a.n_split range partials per (token, head) [t][head][split][hd + 2]
-// (maximum in natural-log units), the inverse Turbo4 rotation, f32 att and Q8_0.
+// (maximum in natural-log units, or log2 units with part_log2), the inverse Turbo4 rotation, f32 att and Q8_0.
 void launch_attention_combine(const AttnArgs &a, hipStream_t st);
 // number of context ranges (n_split) for a launch whose longest query sees max_len
 // positions; fused: a single token on the one-launch path (attention_fused_ok), which

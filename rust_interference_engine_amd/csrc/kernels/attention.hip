@@ -1553,7 +1553,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a) {
         float L = 0.0f;
         for (int s = tid; s < a.n_split; s += 64) {
             const float ms = part[(size_t)s * (hd + 2) + hd], ls = part[(size_t)s * (hd + 2) + hd + 1];
-            const float w = ls > 0.0f ? expf(ms - m) : 0.0f;
+            const float w = ls > 0.0f ? (a.part_log2 ? exp2_hw(ms - m) : expf(ms - m)) : 0.0f;
             wts[s] = w;
             L += ls * w;
         }
@@ -1643,7 +1643,7 @@ __global__ __launch_bounds__(256) void attn_combine_rows_kernel(AttnArgs a) {
         l = part[(size_t)lane * (HD + 2) + HD + 1];
     }
     const float M = xmax_f<64>(m);
-    const float w = l > 0.0f ? expf(m - M) : 0.0f;
+    const float w = l > 0.0f ? (a.part_log2 ? exp2_hw(m - M) : expf(m - M)) : 0.0f;
     const float inv = 1.0f / xsum_f<64>(l * w);
     float o[V] = {};
 #pragma unroll 4

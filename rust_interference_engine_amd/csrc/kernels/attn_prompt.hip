@@ -33,6 +33,22 @@
 // Staging finds them; the workgroup then runs its tiles once more with zeros in their
 // place and adds their products on the vector units, for the tokens that see them.
 //
+// Rounding (CARE: the same two, whose prompts ran in f32 on the vector units before these
+// kernels).  The sums are held to that f32 path's error against float64 by: probabilities
+// times 2^7 and queries of 256 times a power of two per token, so that their low halves
+// are no subnormal f16 values; scores left in their own unit, log2 e entering in the fma
+// of the exponent's argument; score sums in chains of two k-steps and outputs in one
+// chain per tile, small products first, since the matrix core rounds every step of a
+// chain, and down: every other chain and odd tiles run on negated queries and
+// probabilities and are subtracted; probability sums as trees; range maxima merged in log2 units.  Relative error of a layer's outputs
+// (2-norm, 1e-7; f32 path / here / none of this), two seeds each: gemma-3-1b, f16 cache,
+// 650 tokens 0.87 / 0.88 / 2.04 (window layer) and 0.72 / 0.74 / 0.92 (global), 200 at
+// 6000 1.34 / 1.34 / 3.04 and 0.84 / 0.86 / 1.17; Q8_0 cache, 200 at 6000 1.29 / 1.26 /
+// 1.62 and 0.87 / 0.86 / 1.16; 32 heads of 128, Q8_0 cache, 512 at 7680 2.94 / 1.50 /
+// 2.68, 100 at 0 1.23 / 1.25 / 1.51; heads of 64, 64 at 300 0.96 / 0.97 / 1.15.  It costs
+// 1 % of the 512-token call at 7680 (1635 to 1660 us) and 4 % of the gemma-3-1b prompt
+// (1335 to 1390 us, where some registers spill).
+//
 // Work split: a workgroup (4 waves) owns one KV head and a block of query rows;
 // each wave owns 32 tokens of one query head.  Scores are computed transposed,
 // Sᵀ = K·Qᵀ (v_mfma_f32_32x32x16_f16: lane l holds token l mod 32 and 16 cache
@@ -88,12 +104,16 @@ typedef float f32x8 __attribute__((ext_vector_type(8)));
 // (v_cvt_f16_f32 for lo, v_cvt_pk_f16_f32 for the packed hi), and values just
 // above a rounding midpoint have come out of the two on opposite sides, an error
 // of one f16 ulp of x.
+// E, NEG: the halves of ±2^E·x instead (finite x ≥ 0), so that the low half of a small x
+// is no subnormal f16; a NaN stays in lo.
+template <int E = 0, bool NEG = false>
 __device__ __forceinline__ half8 split_hi(const float (&x)[8], half8 &lo) {
     f32x8 hi, r;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        hi[i] = __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, x[i]) + 0x1000u) & 0xFFFFE000u);
-        r[i] = x[i] - hi[i];
+        const uint32_t b = (__builtin_bit_cast(uint32_t, x[i]) + (0x1000u + ((uint32_t)E << 23))) & 0xFFFFE000u;
+        hi[i] = __builtin_bit_cast(float, b | (NEG ? 0x80000000u : 0u));
+        r[i] = E ? fmaf(x[i], (float)(NEG ? -(1 << E) : 1 << E), -hi[i]) : x[i] - hi[i];
     }
     lo = __builtin_convertvector(r, half8);
     return __builtin_convertvector(hi, half8);
@@ -186,8 +206,10 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     const bool w_full = wave_on && tb * 32 + 31 < a.n_tok;                        // all 32 tokens exist
 
     // query fragments: token col of the block, dims 16s + 8h .. +8 (f32 → hi + lo)
+    constexpr bool CARE = KVT == 1 || DS == 2;  // see "Rounding" at the top
     half8 qh[KVT == 1 ? 1 : KS], ql[KVT == 1 ? 1 : KS];
-    i32x4 q8[KVT == 1 ? DT : 1];  // Q8_0: codes 16h .. +16 of each block, and the blocks' scales in log2 units
+    float s_unit = 1.0f;  // CARE: the unit of this token's scores, a power of two
+    i32x4 q8[KVT == 1 ? DT : 1];  // Q8_0: codes 16h .. +16 of each block, and the blocks' scales
     float dq[KVT == 1 ? DT : 1];
     if constexpr (KVT == 1) {
         const float *qrow = a.q + (size_t)(tok_ok ? t : a.n_tok - 1) * qd + (size_t)(wave_on ? head : 0) * hd + dim0 + 16 * h;
@@ -205,7 +227,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
             }
             amax = fmaxf(amax, xor_f<32>(amax));
             const float d = amax / 127.0f, id = d != 0.0f ? 1.0f / d : 0.0f;
-            dq[b] = d * LOG2E_F;
+            dq[b] = d;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 uint32_t w = 0;
@@ -220,10 +242,28 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     } else {
         const int tq = tok_ok ? t : (a.n_tok - 1);
         const float *qrow = a.q + (size_t)tq * qd + (size_t)(wave_on ? head : 0) * hd + dim0;
+        float qs = 1.0f;
+        if constexpr (DS == 2) {  // its largest value (of both groups' dims) to [2^14, 2^15)
+            float amax = 0.0f;
+#pragma unroll
+            for (int s = 0; s < 2 * KS; s++) {
+                const f32x4 x = *(const f32x4 *)(qrow + 16 * (s >> 1) + 8 * h + 4 * (s & 1));
+#pragma unroll
+                for (int e = 0; e < 4; e++) amax = fmaxf(amax, fabsf(x[e]));
+            }
+            amax = fmaxf(amax, xor_f<32>(amax));
+            float *ax = (float *)lds;  // the tile buffers: free until the barrier in front of the first staging
+            ax[threadIdx.x] = amax;
+            __syncthreads();
+            amax = fmaxf(amax, ax[threadIdx.x ^ 256]);
+            if (amax > 0.0f) qs = ldexpf(1.0f, min(max(14 - ilogbf(amax), -100), 100));
+            s_unit = 1.0f / qs;
+        }
 #pragma unroll
         for (int s = 0; s < KS; s++) {
-            const f32x4 x0 = *(const f32x4 *)(qrow + 16 * s + 8 * h);
-            const f32x4 x1 = *(const f32x4 *)(qrow + 16 * s + 8 * h + 4);
+            const float f = DS == 2 && (s & 2) ? -qs : qs;  // every other chain below on negated queries
+            const f32x4 x0 = *(const f32x4 *)(qrow + 16 * s + 8 * h) * f;
+            const f32x4 x1 = *(const f32x4 *)(qrow + 16 * s + 8 * h + 4) * f;
             float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
             qh[s] = split_hi(x, ql[s]);
         }
@@ -247,7 +287,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     };
     // Every lane issues the same loads (indices past the tile's data repeat valid
     // ones, and ring slots wrap without a branch: slots ≥ 32 = the tile length).
-    auto fetch = [&](int tile, Regs &r) {
+    auto fetch = [&](int tile, Regs &r) __attribute__((always_inline)) {
         const int P0 = k0 + tile * PT;
         const int slot0 = P0 % a.slots;
         const int span = p_hi - P0;  // positions past p_hi repeat row p_hi
@@ -297,14 +337,13 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
             }
         }
     };
-    // CHECK: look for values that the matrix product may not see (see the top).  The
+    // CARE: look for values that the matrix product may not see (see the top).  The
     // first run over the tiles (APART false) reports them in odd_seen; in the second they
     // are staged as zeros and their products added apart.
-    constexpr bool CHECK = KVT == 1 || DS == 2;
     __shared__ int odd_seen;
     auto odd_scale = [](float d) { return !(fabsf(d) <= 512.0f); };        // of a Q8_0 block
     auto odd_half = [](uint32_t b) { return (b & 0x7C00u) == 0x7C00u; };   // an infinite or NaN f16
-    auto stage = [&](const Regs &r, int buf, auto apart) {
+    auto stage = [&](const Regs &r, int buf, auto apart) __attribute__((always_inline)) {
         constexpr bool APART = decltype(apart)::value;
         uint8_t *kb = tiles + buf * TB, *vb = kb + PT * KROW;
         if constexpr (KVT == 2) {
@@ -384,7 +423,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
             const int vi = tid + 256 * c;
             if (vi >= 2 * HD) continue;
             uint8_t *dst = vb + 8 * (vi >> 4) * VROW + 4 * (vi & 15);
-            if constexpr (CHECK && !APART) {  // the largest magnitudes' bits, two halves at a time
+            if constexpr (CARE && !APART) {  // the largest magnitudes' bits, two halves at a time
                 u16x2 big = {0, 0};
 #pragma unroll
                 for (int i = 0; i < 8; i++)
@@ -395,7 +434,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
             for (int i = 0; i < 8; i++) {
                 const uint32_t w0 = r.v[c][0][i >> 1], w1 = r.v[c][1][i >> 1];
                 uint32_t pair = (i & 1) ? ((w0 >> 16) | (w1 & 0xFFFF0000u)) : ((w0 & 0xFFFFu) | (w1 << 16));
-                if constexpr (CHECK && APART) pair &= (odd_half(pair) ? 0u : 0xFFFFu) | (odd_half(pair >> 16) ? 0u : 0xFFFF0000u);
+                if constexpr (CARE && APART) pair &= (odd_half(pair) ? 0u : 0xFFFFu) | (odd_half(pair >> 16) ? 0u : 0xFFFF0000u);
                 *(uint32_t *)(dst + i * VROW) = pair;
             }
         }
@@ -405,9 +444,11 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     float m, l_half;
     f32x16 o[DT];
 
+    constexpr int PX = CARE ? 7 : 0;  // o is times 2^PX
+    constexpr float PS = (float)(1 << PX);
     // o += p·v over the values of the tile at position P0 that are staged as zeros; pv:
     // this lane's probabilities of positions P0 + 8(v/4) + 4h + v%4
-    auto add_apart = [&](int P0, f32x16 pv) {
+    auto add_apart = [&](int P0, f32x16 pv) __attribute__((always_inline)) {
         const int span = p_hi - P0;
         auto vrow = [&](int off) { return vc + (size_t)((P0 + min(off, span)) % a.slots) * RB; };
         bool odd = false;  // position lane % 32, half h of the dims (blocks h, h + 2, … of Q8_0)
@@ -436,13 +477,13 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
                         const uint32_t w = c[0] | (uint32_t)c[1] << 16;
 #pragma unroll
                         for (int e = 0; e < 4; e++)
-                            if (odd_scale(sc)) o[d][4 * q4 + e] = fmaf(p, code_f(w, e) * sc, o[d][4 * q4 + e]);
+                            if (odd_scale(sc)) o[d][4 * q4 + e] = fmaf(p * PS, code_f(w, e) * sc, o[d][4 * q4 + e]);
                     } else {
                         const uint2 x = *(const uint2 *)(r + (32 * d + 8 * q4 + 4 * h) * 2);
 #pragma unroll
                         for (int e = 0; e < 4; e++) {
                             const uint32_t b = ((e < 2 ? x.x : x.y) >> (16 * (e & 1))) & 0xFFFFu;
-                            if (odd_half(b)) o[d][4 * q4 + e] = fmaf(p, h2f(b), o[d][4 * q4 + e]);
+                            if (odd_half(b)) o[d][4 * q4 + e] = fmaf(p * PS, h2f(b), o[d][4 * q4 + e]);
                         }
                     }
                 }
@@ -455,7 +496,9 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     // their use)
     const int n_iter = (t_hi - t_lo + NT - 1) / NT;
     const int last = max(n_tiles - 1, 0);
-    auto body = [&](int it, Regs &x, auto apart) {
+    // (without always_inline some of these lambdas stay functions, and o in memory)
+    auto body = [&](int it, Regs &x, auto apart, auto odd_it) __attribute__((always_inline)) {
+        constexpr bool NEG = CARE && decltype(odd_it)::value;  // subtract the sums of -p·v
         const int tile = t_lo + tg0 + it * NT;
         stage(x, (it + 1) & 1, apart);
         fetch(min(tile + 3 * NT, last), x);
@@ -491,7 +534,24 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
                 }
             }
 #pragma unroll
-            for (int ks = 0; ks < (KVT == 1 ? 0 : KS); ks++) {
+            for (int k0 = 0; k0 < (KVT == 1 || !CARE ? 0 : KS); k0 += 4) {  // chains of two k-steps, the small products first
+                f32x16 c[2] = {};
+#pragma unroll
+                for (int g = 0; g < 2; g++) {
+                    const int k1 = k0 + 2 * g;
+                    half8 kf[2];
+#pragma unroll
+                    for (int i = 0; i < 2; i++) kf[i] = as_half8(*(const u32x4 *)(k_s + col * KROW + (16 * (k1 + i) + 8 * h) * 2));
+#pragma unroll
+                    for (int i = 0; i < 2; i++) c[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[i], ql[k1 + i], c[g], 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 2; i++) c[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[i], qh[k1 + i], c[g], 0, 0, 0);
+                }
+                c[0] -= c[1];
+                s = k0 ? s + c[0] : c[0];
+            }
+#pragma unroll
+            for (int ks = 0; ks < (KVT == 1 || CARE ? 0 : KS); ks++) {
                 const half8 kf = as_half8(*(const u32x4 *)(k_s + col * KROW + (16 * ks + 8 * h) * 2));
                 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qh[ks], s, 0, 0, 0);
                 s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, ql[ks], s2, 0, 0, 0);
@@ -500,8 +560,6 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
         if constexpr (DS == 2) {  // the other half of the dims: wave wv of the other group, the same token and positions
             f32x4 *ex = (f32x4 *)(lds + 2 * NW * TB);
             if (work) {
-                s += s2;
-                s2 = f32x16{};
 #pragma unroll
                 for (int q4 = 0; q4 < 4; q4++) ex[(grp * 4 + q4) * 256 + tid] = f32x4{s[4 * q4], s[4 * q4 + 1], s[4 * q4 + 2], s[4 * q4 + 3]};
             }
@@ -519,13 +577,15 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
             if constexpr (KVT == 2) {
 #pragma unroll
                 for (int v = 0; v < 16; v++) s[v] = (s[v] + s2[v]) * fk[8 * (v >> 2) + 4 * h + (v & 3)];
-            } else if constexpr (KVT == 0) {
+            } else if constexpr (!CARE) {
 #pragma unroll
                 for (int v = 0; v < 16; v++) s[v] = (s[v] + s2[v]) * LOG2E_F;
             }
-            // lane: token col, positions P0 + 8(v/4) + 4h + v%4; scores in log2 units (q carries log2 e)
+            // lane: token col, positions P0 + 8(v/4) + 4h + v%4; scores in log2 units (CARE: of
+            // s_unit, and lu is one of them in log2 units)
+            const float lu = LOG2E_F * s_unit;
             if (a.softcap > 0.0f) {
-                const float cl = a.softcap * LOG2E_F;  // the cap in the same units
+                const float cl = CARE ? a.softcap / s_unit : a.softcap * LOG2E_F;  // the cap in the same units
 #pragma unroll
                 for (int v = 0; v < 16; v++) s[v] = cl * tanhf(s[v] / cl);
             }
@@ -540,6 +600,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
 #pragma unroll
             for (int v = 1; v < 16; v++) mx = fmaxf(mx, s[v]);
             mx = fmaxf(mx, xor_f<32>(mx));
+            if constexpr (CARE) mx *= lu;  // m is in log2 units
             // The reference maximum m moves only when a score exceeds it by more than
             // 2^8, so probabilities stay ≤ 256 and the accumulators are rescaled rarely
             // (exact either way: m cancels in O / l).
@@ -560,8 +621,18 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
             float pv[16];
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                pv[v] = exp2_hw(s[v] - mref);
-                l_half += pv[v];
+                pv[v] = CARE ? exp2_hw(fmaf(s[v], lu, -mref)) : exp2_hw(s[v] - mref);
+                if constexpr (!CARE) l_half += pv[v];
+            }
+            if constexpr (CARE) {  // the tile's sum as a tree
+                float x[8];
+#pragma unroll
+                for (int v = 0; v < 8; v++) x[v] = pv[v] + pv[v + 8];
+#pragma unroll
+                for (int w = 4; w; w /= 2)
+#pragma unroll
+                    for (int v = 0; v < w; v++) x[v] += x[v + w];
+                l_half += x[0];
             }
             if constexpr (KVT == 2) {  // the value rows' scale/46 (l keeps the plain probabilities)
 #pragma unroll
@@ -573,31 +644,41 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
                 float x[8];
 #pragma unroll
                 for (int i = 0; i < 8; i++) x[i] = pv[8 * u + i];
-                ph[u] = split_hi(x, pl[u]);
+                ph[u] = split_hi<PX, NEG>(x, pl[u]);
             }
             // Oᵀ[dim][tok] = alpha·Oᵀ + Σ_pos Vᵀ[dim][pos]·P[tok][pos]; k-slot 8h + i of step u
             // is position 16u + 4h + i (i < 4) or 16u + 8 + 4h + (i − 4)
 #pragma unroll
             for (int d = 0; d < DT; d++) {
                 const uint8_t *vrow = v_s + (32 * d + col) * VROW;
-#pragma unroll
-                for (int u = 0; u < 2; u++) {
+                auto frag = [&](int u) {
                     const uint2 lo4 = *(const uint2 *)(vrow + (16 * u + 4 * h) * 2);
                     const uint2 hi4 = *(const uint2 *)(vrow + (16 * u + 8 + 4 * h) * 2);
-                    u32x4 vv;
-                    vv[0] = lo4.x;
-                    vv[1] = lo4.y;
-                    vv[2] = hi4.x;
-                    vv[3] = hi4.y;
-                    const half8 vf = as_half8(vv);
-                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, ph[u], o[d], 0, 0, 0);
-                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pl[u], o[d], 0, 0, 0);
+                    return as_half8(u32x4{lo4.x, lo4.y, hi4.x, hi4.y});
+                };
+                const half8 vf[2] = {frag(0), frag(1)};
+                if constexpr (CARE) {
+                    f32x16 t = {};
+#pragma unroll
+                    for (int u = 0; u < 2; u++) t = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[u], pl[u], t, 0, 0, 0);
                     if constexpr (KVT == 1) {  // the values' low halves
-                        const uint2 lo4l = *(const uint2 *)(vrow + HD * VROW + (16 * u + 4 * h) * 2);
-                        const uint2 hi4l = *(const uint2 *)(vrow + HD * VROW + (16 * u + 8 + 4 * h) * 2);
-                        const half8 vfl = as_half8(u32x4{lo4l.x, lo4l.y, hi4l.x, hi4l.y});
-                        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vfl, ph[u], o[d], 0, 0, 0);
-                        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vfl, pl[u], o[d], 0, 0, 0);
+#pragma unroll
+                        for (int u = 0; u < 2; u++) {
+                            const uint2 lo4l = *(const uint2 *)(vrow + HD * VROW + (16 * u + 4 * h) * 2);
+                            const uint2 hi4l = *(const uint2 *)(vrow + HD * VROW + (16 * u + 8 + 4 * h) * 2);
+                            const half8 vfl = as_half8(u32x4{lo4l.x, lo4l.y, hi4l.x, hi4l.y});
+                            t = __builtin_amdgcn_mfma_f32_32x32x16_f16(vfl, pl[u], t, 0, 0, 0);
+                            t = __builtin_amdgcn_mfma_f32_32x32x16_f16(vfl, ph[u], t, 0, 0, 0);
+                        }
+                    }
+#pragma unroll
+                    for (int u = 0; u < 2; u++) t = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[u], ph[u], t, 0, 0, 0);
+                    o[d] = NEG ? o[d] - t : o[d] + t;
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 2; u++) {
+                        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[u], ph[u], o[d], 0, 0, 0);
+                        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[u], pl[u], o[d], 0, 0, 0);
                     }
                 }
             }
@@ -610,7 +691,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
         }
         __syncthreads();
     };
-    auto run = [&](auto apart) {
+    auto run = [&](auto apart) __attribute__((always_inline)) {
         m = -INFINITY;
         l_half = 0.0f;
 #pragma unroll
@@ -627,11 +708,11 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
         // an even number of steps (the last one may be idle), so that the loop has one
         // entry path per register set and every wait count is exact
         for (int it = 0; it < n_iter; it += 2) {
-            body(it, rb, apart);
-            body(it + 1, ra, apart);
+            body(it, rb, apart, std::false_type{});
+            body(it + 1, ra, apart, std::true_type{});
         }
     };
-    if constexpr (CHECK) {
+    if constexpr (CARE) {
         if (threadIdx.x == 0) odd_seen = 0;
         __syncthreads();
         run(std::false_type{});  // its last barrier follows every staging
@@ -678,11 +759,11 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     if (!wave_on) return;
     const float l_tot = l_half + xor_f<32>(l_half);
     if (gridDim.z > 1) {
-        // KV split: this range's partial (unnormalized output, maximum in natural-log
+        // KV split: this range's partial (unnormalized output, maximum in natural-log or (CARE) log2
         // units, sum) in the layout attn_combine_kernel merges: [t][head][split][hd + 2]
         if (tok_ok) {
             float *pp = a.part + (((size_t)t * a.n_head + head) * gridDim.z + blockIdx.z) * (hd + 2);
-            const float osc = KVT == 2 ? 1.0f / 256.0f : 1.0f;
+            const float osc = KVT == 2 ? 1.0f / 256.0f : 1.0f / PS;
 #pragma unroll
             for (int d = 0; d < DT; d++)
 #pragma unroll
@@ -693,13 +774,13 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
                     *(f32x4 *)(pp + dim0 + 32 * d + 8 * q4 + 4 * h) = w4;
                 }
             if (h == 0 && (DS == 1 || grp == 0)) {
-                pp[hd] = m == -INFINITY ? -INFINITY : m * LN2_F;
+                pp[hd] = CARE || m == -INFINITY ? m : m * LN2_F;
                 pp[hd + 1] = l_tot;
             }
         }
         return;
     }
-    const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+    const float inv = l_tot > 0.0f ? 1.0f / (l_tot * PS) : 0.0f;
     // lane: token col, dims 32d + 8(v/4) + 4h + v%4
     if constexpr (KVT == 2) {
         // Rᵀ o (turbo.rs:113-117): the normalized FWHT of the rotated output (stages of
@@ -895,6 +976,7 @@ bool launch_attention_prompt_mfma(const AttnArgs &a, hipStream_t st) {
     grid.z = S;
     AttnArgs b = a;
     b.n_split = S;
+    b.part_log2 = a.kv_type == 1 || a.hd == 256;
     // partials [t][head][split][hd + 2] at the start of the range-partial buffer; the
     // Turbo4 path's rotated, quantized queries after them
     float *qhat = a.part + (S > 1 ? (size_t)a.n_tok * a.n_head * S * (a.hd + 2) : 0);
