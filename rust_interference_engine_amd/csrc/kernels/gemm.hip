@@ -158,8 +158,9 @@ struct StageRegs {
 // tokA: the activation row of the thread's token (tid / (256/BN)); tokD: of token tid
 // (tid < BN); woff: the expert's byte offset in a grouped launch
 // TAIL: K is an odd multiple of 64, so the last stage holds two blocks.  Its other two
-// repeat the row's last ones (in bounds) with activation scales of 0.  (As a run-time
-// check in every launch this took a 512-token Q8_0 prompt from 1353 to 1478 us.)
+// repeat the row's last ones (in bounds) with both scales 0 (the weights' at the store: an
+// infinite one would make the row NaN).  (As a run-time check in every launch this took a
+// 512-token Q8_0 prompt from 1353 to 1478 us.)
 template <int TY, bool GLU, int BN, bool TAIL>
 __device__ __forceinline__ void stage_load(const GemmP &p, int sg, int row0, int tokA, int tokD, size_t woff, int b0, int tid,
                                            StageRegs<TY, GLU, BN> &R) {
@@ -235,8 +236,9 @@ __device__ __forceinline__ void put_block(const uint32_t (&q)[block_dwords<TY>()
     }
 }
 
-template <int TY, bool GLU, int BN>
-__device__ __forceinline__ void stage_store(GemmStage<TY, GLU, BN> &S, int tid, const StageRegs<TY, GLU, BN> &R) {
+// tail: R holds a last stage of two blocks
+template <int TY, bool GLU, int BN, bool TAIL>
+__device__ __forceinline__ void stage_store(GemmStage<TY, GLU, BN> &S, int tid, const StageRegs<TY, GLU, BN> &R, bool tail) {
     {
         constexpr int TPT = 256 / BN, NV = 128 / TPT / 16;
         v4i *dst = (v4i *)(S.a + (tid / TPT) * G_AST + 16 * NV * (tid % TPT));
@@ -249,7 +251,7 @@ __device__ __forceinline__ void stage_store(GemmStage<TY, GLU, BN> &S, int tid, 
     if constexpr (by_units<TY, GLU, BN>()) {
         if (!GLU && tid >= 128) return;
         const int nw = GLU ? (tid >> 7) : 0, row = (tid & 127) >> 1, u = tid & 1;
-        const uint32_t *w = R.w.w;
+        const uint32_t *w = R.w.w, keep = TAIL && tail && u ? 0u : ~0u;
         constexpr int C0 = TY == T_Q5_0 ? 1 : 0;  // the dword whose upper half starts block 0's codes
 #pragma unroll
         for (int b = 0; b < 2; b++) {
@@ -257,12 +259,12 @@ __device__ __forceinline__ void stage_store(GemmStage<TY, GLU, BN> &S, int tid, 
 #pragma unroll
             for (int i = 0; i < ND; i++) q[i] = b ? w[unit_dwords<TY>() - ND + i] : __builtin_amdgcn_alignbyte(w[C0 + i + 1], w[C0 + i], 2);
             const uint32_t qh = TY == T_Q5_0 ? (b ? w[6] : __builtin_amdgcn_alignbyte(w[1], w[0], 2)) : 0u;
-            put_block<TY>(q, qh, b ? w[C0 + ND] >> 16 : w[0] & 0xffff, S.wq[nw] + row * WST + (2 * u + b) * QB, S.dw[nw] + row * G_KC + 2 * u + b);
+            put_block<TY>(q, qh, (b ? w[C0 + ND] >> 16 : w[0] & 0xffff) & keep, S.wq[nw] + row * WST + (2 * u + b) * QB, S.dw[nw] + row * G_KC + 2 * u + b);
         }
     } else {
 #pragma unroll
         for (int i = 0; i < ND; i++) q[i] = R.w.q[i / 4].w[i % 4];
-        put_block<TY>(q, R.w.qh, R.w.d, S.wq[0] + (tid >> 2) * WST + (tid & 3) * QB, S.dw[0] + (tid >> 2) * G_KC + (tid & 3));
+        put_block<TY>(q, R.w.qh, TAIL && tail && (tid & 2) ? 0u : R.w.d, S.wq[0] + (tid >> 2) * WST + (tid & 3) * QB, S.dw[0] + (tid >> 2) * G_KC + (tid & 3));
     }
 }
 
@@ -314,7 +316,8 @@ __global__ __launch_bounds__(256, (!GLU && NT == 1) ? 3 : 2) void gemm_kernel(Ge
     const int last_stage = n_stages - 1;
     StageRegs<TY, GLU, BN> ra, rb;
     stage_load<TY, GLU, BN, TAIL>(p, sg, row0, tokA, tokD, woff, k0 * G_KC, tid, ra);
-    stage_store<TY, GLU, BN>(st[0], tid, ra);
+    auto tail_at = [&](int s) { return TAIL && 32 * G_KC * (k0 + s + 1) > p.K; };
+    stage_store<TY, GLU, BN, TAIL>(st[0], tid, ra, tail_at(0));
     stage_load<TY, GLU, BN, TAIL>(p, sg, row0, tokA, tokD, woff, (k0 + min(1, last_stage)) * G_KC, tid, rb);
     __syncthreads();
     // Per stage: all operands of the stage's KC blocks from LDS, then the
@@ -383,7 +386,7 @@ __global__ __launch_bounds__(256, (!GLU && NT == 1) ? 3 : 2) void gemm_kernel(Ge
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (s + 1 < n_stages) stage_store<TY, GLU, BN>(st[(s + 1) & 1], tid, rs);
+        if (s + 1 < n_stages) stage_store<TY, GLU, BN, TAIL>(st[(s + 1) & 1], tid, rs, tail_at(s + 1));
         __syncthreads();
     };
     for (int s = 0; s < n_stages; s += 2) {
