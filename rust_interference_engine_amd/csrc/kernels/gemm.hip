@@ -268,8 +268,19 @@ __device__ __forceinline__ void stage_store(GemmStage<TY, GLU, BN> &S, int tid, 
     }
 }
 
+// Sums in three levels: a stage's four blocks, 8 stages, all of them.  For the launches
+// that ran in the batched GEMV before, whose sums are trees: one chain over the K / 32
+// blocks has up to 3 times its error against float64 (Q5_0, K 896 / 4096 / 14336, in 1e-7:
+// GEMV 0.67 / 0.78 / 0.87, one chain 1.00 / 2.05 / 2.71, three levels 0.72 / 0.84 / 0.95).
+// Two waves per SIMD (three spill: 68 against 50 us for 512 tokens, 4096 x 4096); the
+// gated and 128-token forms hold one register set of loads (two spill: gate/up 2 x 14336 x
+// 4096 321 against 253 us, down 186 against 135 us; in one chain 239 and 127 us).
+template <int TY, bool TAIL>
+constexpr bool fine_sums() { return TY == T_Q5_0 || TAIL; }
+
 template <int TY, bool GLU, int NT, bool TAIL>
-__global__ __launch_bounds__(256, (!GLU && NT == 1) ? 3 : 2) void gemm_kernel(GemmP p) {  // one-tile non-gated: three waves per SIMD
+__global__ __launch_bounds__(256, (!GLU && NT == 1 && !fine_sums<TY, TAIL>()) ? 3 : 2) void gemm_kernel(GemmP p) {  // one-tile non-gated: three waves per SIMD
+    constexpr bool FINE = fine_sums<TY, TAIL>(), ONE = FINE && (GLU || NT == 2);
     constexpr int NW = GLU ? 2 : 1;
     constexpr int BN = 64 * NT;  // tokens per workgroup tile: NT 32-token tiles per wave, 2 waves along tokens
     constexpr int QB = GemmLds<TY>::QB, WST = GemmLds<TY>::WST;
@@ -301,6 +312,7 @@ __global__ __launch_bounds__(256, (!GLU && NT == 1) ? 3 : 2) void gemm_kernel(Ge
         for (int t = 0; t < NT; t++)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[a][t][v] = 0.0f;
+    float tot[FINE ? NW : 1][NT][16] = {}, part4[16];  // FINE: sums of 8 stages' acc, of one stage
     const v16i zi = {0};
     const v32f zf32 = {0};
 
@@ -324,8 +336,10 @@ __global__ __launch_bounds__(256, (!GLU && NT == 1) ? 3 : 2) void gemm_kernel(Ge
     // P = KC·NT·NW tile products in a software pipeline: the MFMAs of product
     // q+1 are issued before the VALU epilogue of product q.
     constexpr int P = G_KC * NT * NW;
-    // rl: receives stage s + 2; rs: holds stage s + 1, stored to LDS after stage s
+    // rl: receives stage s + 2; rs: holds stage s + 1, stored to LDS after stage s (ONE: one
+    // register set, which is stored and then loaded again before stage s)
     auto body = [&](int s, StageRegs<TY, GLU, BN> &rl, const StageRegs<TY, GLU, BN> &rs) {
+        if (ONE && s + 1 < n_stages) stage_store<TY, GLU, BN, TAIL>(st[(s + 1) & 1], tid, rs, tail_at(s + 1));
         stage_load<TY, GLU, BN, TAIL>(p, sg, row0, tokA, tokD, woff, (k0 + min(s + 2, last_stage)) * G_KC, tid, rl);
         if (s < n_stages) {  // workgroup-uniform; the idle step of an odd stage count skips it
             const GemmStage<TY, GLU, BN> &S = st[s & 1];
@@ -344,11 +358,15 @@ __global__ __launch_bounds__(256, (!GLU && NT == 1) ? 3 : 2) void gemm_kernel(Ge
             // product 2i + h's, for the two-block outer product v_mfma_f32_32x32x1f32
             // (block h's 32×32 result in registers 16h..16h+15, laid out as a single
             // block's); one such MFMA per two products halves the scale-MFMA cycles
+            // product q: block j of tile (t, a); FINE: a tile's blocks one after the other
+            auto blk = [](int q) { return FINE ? q % G_KC : q / (NT * NW); };
+            auto tok = [](int q) { return FINE ? q / G_KC / NW : (q / NW) % NT; };
+            auto mat = [](int q) { return FINE ? q / G_KC % NW : q % NW; };
             float sa[P / 2], sb[P / 2];
 #pragma unroll
             for (int i = 0; i < P / 2; i++) {
                 const int qh = 2 * i + h;
-                const int jh = qh / (NT * NW), th = (qh / NW) % NT, ah = qh % NW;
+                const int jh = blk(qh), th = tok(qh), ah = mat(qh);
                 const int arh = wc * 32 * NT + 32 * th + tok_m;
                 sa[i] = S.da[arh * G_KC + jh];
                 sb[i] = S.dw[ah][wrow * G_KC + jh];
@@ -359,11 +377,10 @@ __global__ __launch_bounds__(256, (!GLU && NT == 1) ? 3 : 2) void gemm_kernel(Ge
             // accumulators of product q-2: at most two result pairs are live, and the
             // MFMAs of q overlap the VALU epilogue of q-1.
             auto issue = [&](int q) {
-                const int j = q / (NT * NW), t = (q / NW) % NT, a = q % NW;
+                const int j = blk(q), t = tok(q), a = mat(q);
                 v4i aop = av[j][t];
                 if (q >= 2) {
-                    const int t2 = ((q - 2) / NW) % NT, a2 = (q - 2) % NW;
-                    const float *d = acc[a2][t2];
+                    const float *d = FINE && blk(q - 2) != G_KC - 1 ? part4 : acc[mat(q - 2)][tok(q - 2)];
                     asm volatile("" : "+v"(aop) : "v"(d[0]), "v"(d[1]), "v"(d[2]), "v"(d[3]), "v"(d[4]), "v"(d[5]), "v"(d[6]), "v"(d[7]),
                                  "v"(d[8]), "v"(d[9]), "v"(d[10]), "v"(d[11]), "v"(d[12]), "v"(d[13]), "v"(d[14]), "v"(d[15]));
                 }
@@ -379,19 +396,39 @@ __global__ __launch_bounds__(256, (!GLU && NT == 1) ? 3 : 2) void gemm_kernel(Ge
                 // itself the scheduler moves each epilogue right behind its own MFMAs and
                 // fills the latency with s_nop)
                 __builtin_amdgcn_sched_barrier(0);
-                const int t = (q / NW) % NT, a = q % NW;
+                const int t = tok(q), a = mat(q);
 #pragma unroll
-                for (int v = 0; v < 16; v++)
-                    acc[a][t][v] = fmaf((float)Iq[q & 1][v], Sp[(q >> 1) & 1][16 * (q & 1) + v], acc[a][t][v]);
+                for (int v = 0; v < 16; v++) {
+                    const float I = (float)Iq[q & 1][v], S = Sp[(q >> 1) & 1][16 * (q & 1) + v];
+                    if constexpr (!FINE) acc[a][t][v] = fmaf(I, S, acc[a][t][v]);
+                    else part4[v] = blk(q) == 0 ? I * S : fmaf(I, S, part4[v]);
+                    if (FINE && blk(q) == G_KC - 1) acc[a][t][v] += part4[v];
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (s + 1 < n_stages) stage_store<TY, GLU, BN, TAIL>(st[(s + 1) & 1], tid, rs, tail_at(s + 1));
+        if (!ONE && s + 1 < n_stages) stage_store<TY, GLU, BN, TAIL>(st[(s + 1) & 1], tid, rs, tail_at(s + 1));
         __syncthreads();
     };
     for (int s = 0; s < n_stages; s += 2) {
-        body(s, ra, rb);
-        body(s + 1, rb, ra);
+        if constexpr (ONE) {
+            body(s, rb, rb);
+            body(s + 1, rb, rb);
+        } else {
+            body(s, ra, rb);
+            body(s + 1, rb, ra);
+        }
+        if (FINE && ((s & 6) == 6 || s + 2 >= n_stages)) {
+#pragma unroll
+            for (int a = 0; a < NW; a++)
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) {
+                        tot[FINE ? a : 0][t][v] += acc[a][t][v];
+                        acc[a][t][v] = s + 2 >= n_stages ? tot[FINE ? a : 0][t][v] : 0.0f;
+                    }
+        }
     }
     // ---- epilogue: lane holds weight row row0 + wrow for tokens t0 + wc·64 + 32t + 16h + v ----
     if (p.ks > 1 && !p.plane && !split_sum(reinterpret_cast<float(&)[NW * NT * 16]>(acc), p.ws.part, (uint32_t)(p.ws.cap * 4), p.ws.cnt,
