@@ -287,7 +287,8 @@ __device__ __forceinline__ void pin16(int (&s)[16]) {
 }
 
 template <int TY, bool GLU, int BN = KQ_BN>
-__global__ __launch_bounds__(256) void gemm_q45k_kernel(KqP p) {
+__global__ __launch_bounds__(256, TY == T_Q5_K && !GLU ? 3 : 1) void gemm_q45k_kernel(KqP p) {
+    constexpr bool FINE = TY == T_Q5_K && !GLU;
     constexpr int NW = GLU ? 2 : 1, BM = kq_bm<BN>(), WC = BN / 32;  // waves along the tokens
     __shared__ KqStage<TY, GLU, BN> st[2];
     __shared__ KqEnd<GLU, BN> en;
@@ -318,6 +319,7 @@ __global__ __launch_bounds__(256) void gemm_q45k_kernel(KqP p) {
     for (int a = 0; a < NW; a++)
 #pragma unroll
         for (int v = 0; v < 16; v++) acc[a][v] = 0.0f;
+    float tot[FINE ? 16 : 1] = {};
     // this workgroup's superblocks [sb0, sb1) (its K split)
     const int nsb = p.K >> 8;
     const int sb0 = KSPLIT ? ksi * nsb / p.ks : 0, sb1 = KSPLIT ? (ksi + 1) * nsb / p.ks : nsb;
@@ -395,6 +397,15 @@ __global__ __launch_bounds__(256) void gemm_q45k_kernel(KqP p) {
     for (int sb = sb0; sb < sb1; sb++) {
         half(sb, std::integral_constant<int, 0>{});
         half(sb, std::integral_constant<int, 1>{});
+        // Q5_K down projections: sums of 8 superblocks, then of those (K 14336 in one chain
+        // has 1.3 to 2.1 times the error against float64 of the batched GEMV, which ran them before)
+        if (FINE && ((sb - sb0) % 8 == 7 || sb + 1 == sb1)) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                tot[FINE ? v : 0] += acc[0][v];
+                acc[0][v] = sb + 1 == sb1 ? tot[FINE ? v : 0] : 0.0f;
+            }
+        }
     }
     // ---- epilogue: lane holds weight row row0 + wrow for tokens t0 + wc·32 + 16h + v ----
     if constexpr (KSPLIT) {
