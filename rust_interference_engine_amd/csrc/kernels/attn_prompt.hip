@@ -46,8 +46,8 @@
 // 6000 1.34 / 1.34 / 3.04 and 0.84 / 0.86 / 1.17; Q8_0 cache, 200 at 6000 1.29 / 1.26 /
 // 1.62 and 0.87 / 0.86 / 1.16; 32 heads of 128, Q8_0 cache, 512 at 7680 2.94 / 1.50 /
 // 2.68, 100 at 0 1.23 / 1.25 / 1.51; heads of 64, 64 at 300 0.96 / 0.97 / 1.15.  It costs
-// 1 % of the 512-token call at 7680 (1635 to 1660 us) and 4 % of the gemma-3-1b prompt
-// (1335 to 1390 us, where some registers spill).
+// 1 % of the 512-token call at 7680 (1635 to 1660 us) and 2 % of the gemma-3-1b prompt
+// (1335 to 1358 us).
 //
 // Work split: a workgroup (4 waves) owns one KV head and a block of query rows;
 // each wave owns 32 tokens of one query head.  Scores are computed transposed,
@@ -60,6 +60,7 @@
 #include "../common.hpp"
 #include "../device.hpp"
 #include "../kernels.hpp"
+#include "../attn_splits.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -496,12 +497,14 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
     // their use)
     const int n_iter = (t_hi - t_lo + NT - 1) / NT;
     const int last = max(n_tiles - 1, 0);
+    // DS = 2: one register set, loaded one iteration ahead (the second one spilled: gemma-3-1b,
+    // 650 tokens 1390 against 1358 us, 200 at 6000 982 against 952 us)
     // (without always_inline some of these lambdas stay functions, and o in memory)
     auto body = [&](int it, Regs &x, auto apart, auto odd_it) __attribute__((always_inline)) {
         constexpr bool NEG = CARE && decltype(odd_it)::value;  // subtract the sums of -p·v
         const int tile = t_lo + tg0 + it * NT;
         stage(x, (it + 1) & 1, apart);
-        fetch(min(tile + 3 * NT, last), x);
+        fetch(min(tile + (DS == 2 ? 2 : 3) * NT, last), x);
         k_s = tiles + (it & 1) * TB;
         v_s = k_s + PT * KROW;
         const float *fk = (const float *)(v_s + HD * VROW), *fv = fk + PT;  // Turbo4 row factors
@@ -703,13 +706,13 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
         fetch(min(t_lo + tg0, last), ra);
         stage(ra, 0, apart);
         fetch(min(t_lo + tg0 + NT, last), rb);
-        fetch(min(t_lo + tg0 + 2 * NT, last), ra);
+        if constexpr (DS == 1) fetch(min(t_lo + tg0 + 2 * NT, last), ra);
         __syncthreads();
         // an even number of steps (the last one may be idle), so that the loop has one
         // entry path per register set and every wait count is exact
         for (int it = 0; it < n_iter; it += 2) {
             body(it, rb, apart, std::false_type{});
-            body(it + 1, ra, apart, std::true_type{});
+            body(it + 1, DS == 2 ? rb : ra, apart, std::true_type{});
         }
     };
     if constexpr (CARE) {
@@ -949,22 +952,12 @@ __global__ __launch_bounds__(64) void turbo_query_kernel(const float *__restrict
 bool attention_prompt_mfma_ok(const AttnArgs &a) {
     const int G = a.n_kv > 0 ? a.n_head / a.n_kv : 0;
     const bool cache_ok = a.kv_type == 0 || a.kv_type == 1 || (a.kv_type == 2 && a.hd == 128 && a.turbo_signs && a.k_scale && a.v_scale && a.part);
+    // heads of 256 over f16 caches: up to 8 tokens in the per-token kernel (gemma-3-1b, 2 / 8
+    // tokens at 12000, six layers: 473 / 610 us there, 534 / 660 us here; 12 tokens 1067
+    // against 767 us)
+    if (a.hd == 256 && a.kv_type == 0 && a.n_tok <= 8) return false;
     return cache_ok && a.n_tok > 1 && !a.d_pos0 && a.slots >= 32 && (a.hd == 32 || a.hd == 64 || a.hd == 96 || a.hd == 128 || (a.hd == 256 && a.kv_type != 2)) && G >= 1 &&
            G <= 8 && a.n_head == G * a.n_kv && (a.att_fmt != ACT_Q8_0 || (a.att_q.qs && a.att_q.d));
-}
-
-// KV splits of a launch, merged by a second kernel: at least 16 tiles of 32 positions
-// each, up to about two workgroups per CU, at most 16.  Grids under 64 workgroups take
-// splits of at least 2 tiles, up to one workgroup per CU (650 tokens of gemma-3-1b, 21
-// workgroups, six layers: 1579 us in one pass with the per-token kernel, 1369 us in splits
-// of 4 tiles, 1323 us in splits of 2).  From 64 on, splits of fewer than 16 tiles measured
-// no better than one pass (512 tokens at 0, 128 workgroups: 1149 against 1142 us).
-static int prompt_kv_splits(const AttnArgs &a, const dim3 &grid, int tokens_per_wg) {
-    int longest = (a.pos0 + a.n_tok - 1) / PT + 1;  // tiles of the last query row
-    if (a.window > 0) longest = std::min(longest, (a.window + tokens_per_wg - 2) / PT + 2);
-    const int wgs = (int)(grid.x * grid.y);
-    const int by_work = wgs < 64 ? longest / 2 : longest / 16, by_grid = wgs < 64 ? 256 / wgs : 512 / wgs;
-    return std::max(1, std::min({16, by_work, by_grid}));
 }
 
 bool launch_attention_prompt_mfma(const AttnArgs &a, hipStream_t st) {
@@ -972,7 +965,9 @@ bool launch_attention_prompt_mfma(const AttnArgs &a, hipStream_t st) {
     const int G = a.n_head / a.n_kv;
     const int wpt = G < 4 ? G : 4, tbw = 4 / wpt, hgroups = (G + 3) / 4;
     dim3 grid((a.n_tok + 32 * tbw - 1) / (32 * tbw), a.n_kv * hgroups);
-    const int S = prompt_kv_splits(a, grid, 32 * tbw);
+    int tiles = (a.pos0 + a.n_tok - 1) / PT + 1;  // of the last query row
+    if (a.window > 0) tiles = std::min(tiles, (a.window + 32 * tbw - 2) / PT + 2);
+    const int S = prompt_kv_splits((int)(grid.x * grid.y), tiles, a.kv_type == 1);
     grid.z = S;
     AttnArgs b = a;
     b.n_split = S;
