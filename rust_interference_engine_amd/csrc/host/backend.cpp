@@ -210,6 +210,12 @@ HipBackend::HipBackend(const uint8_t *gguf, size_t len, const BackendConfig &cfg
     for (auto &L : layers_)
         for (const DevWeight *w : {&L.wq, &L.wk, &L.wv, &L.wo, &L.gate, &L.up, &L.down, &L.router, &L.sh_gate, &L.sh_up, &L.sh_down})
             halves = halves || w->ty == T_BF16 || w->ty == T_F16;
+    // Few tokens of a narrow model stay in the batched GEMV: a pass over its weights per 4
+    // tokens takes less than the GEMM's launches of few workgroups, whose time hardly
+    // depends on the tokens (two layers, GEMV / GEMM: hidden 960, 24 tokens 235 / 281 us, 48
+    // tokens 303 / 300; 1024, 13 tokens 217 / 245; 1536, 9 tokens 263 / 298; 2048, 9 tokens
+    // 294 / 301, 13 tokens 366 / 310)
+    float_min_n_ = E < 1024 ? 33 : std::max<int>(9, (int)((20480 + E - 1) / E));
     if (halves && mb > 8) {
         for (auto &p : split_.p) p = dalloc<uint16_t>(allocs_, mb * kmax_);
         split_.scale = dalloc<float>(allocs_, mb);
@@ -344,7 +350,7 @@ void HipBackend::prepare(const float *x, const float *norm, int n, int K, const 
 }
 
 void HipBackend::float_rows(const float *x, const float *norm, int n, int K, int ty, bool ref_order) {
-    if (n > 8 && split_.p[0] && gemm_float_supported(ty, K)) {
+    if (n >= float_min_n_ && split_.p[0] && gemm_float_supported(ty, K)) {
         launch_split_rows(x, K, norm, m_.cfg.rms_eps, n, K, d_xn_, ty, split_, st_, ref_order);
         split_ty_ = ty;
         return;
@@ -372,7 +378,7 @@ void HipBackend::matmul(const GemvSeg *segs, int nseg, int n, int K, const ActQ8
             if (!launch_gemm(&segs[s], e - s, a, n, K, st_, nullptr, gemm_ws_)) break;
             s = e;
         }
-        while (n > 8 && s < j && split_.p[0] && gemm_float_supported(segs[s].w.ty, K)) {
+        while (n >= float_min_n_ && s < j && split_.p[0] && gemm_float_supported(segs[s].w.ty, K)) {
             int e = s + 1;
             while (e < j && e - s < 3 && segs[e].w.ty == segs[s].w.ty) e++;
             if (split_ty_ != segs[s].w.ty) {
@@ -403,7 +409,7 @@ void HipBackend::ffn_dense(const DevLayer &L, int n, float *out, int epi) {
     const ActQ8 &a = act_format(L.gate.ty) == ACT_Q8K ? actk_ : act0_;
     bool done = false;
     if (n > 8 && gemm_supported(L.gate.ty, E)) done = launch_gemm_glu(L.gate, L.up, a, n, E, d_h_, ff, c.gelu, st_, nullptr, gemm_ws_);
-    if (n > 8 && L.gate.ty == split_ty_) done = launch_gemm_float_glu(L.gate, L.up, split_, n, E, d_h_, ff, c.gelu, st_);
+    if (L.gate.ty == split_ty_) done = launch_gemm_float_glu(L.gate, L.up, split_, n, E, d_h_, ff, c.gelu, st_);
     const int fmt = act_format(L.down.ty);
     // single-token Q8_0 down projection: the gate/up kernel quantizes h itself
     bool h_quantized = false;
@@ -646,7 +652,7 @@ void HipBackend::expert_ffn(const DevWeight &g, const DevWeight &u, const DevWei
     const ActQ8 &a = act_format(g.ty) == ACT_Q8K ? actk_ : act0_;
     bool done = false;
     if (m > 8 && gemm_supported(g.ty, E)) done = launch_gemm_glu(g, u, a, m, E, d_h_, ff, c.gelu, st_, nullptr, gemm_ws_);
-    if (m > 8 && g.ty == split_ty_) done = launch_gemm_float_glu(g, u, split_, m, E, d_h_, ff, c.gelu, st_);
+    if (g.ty == split_ty_) done = launch_gemm_float_glu(g, u, split_, m, E, d_h_, ff, c.gelu, st_);
     if (!done && !launch_gemv_glu(g, u, a, d_xn_, m, E, d_h_, ff, c.gelu, nullptr, st_))
         throw Error{E_UNSUPPORTED, "unsupported: expert FFN weights"};
     const int fmt = act_format(dn.ty);

@@ -141,6 +141,7 @@ class HipBackend {
     ActQ8 act0_, actk_;  // Q8_0 and Q8_K batches
     ActQ8 act_h_;        // Q8_0 of the single-token FFN hidden
     ActSplit split_;     // 16-bit parts of d_xn_'s rows (models with BF16 / F16 matrices)
+    int float_min_n_ = 9;  // the fewest tokens that BF16 / F16 matrices multiply in the GEMM
     int split_ty_ = -1;  // the weight type split_ was made for, -1: not d_xn_'s present rows
     // d_xn_ = RMSNorm(x)·norm (x itself without norm) in f32, with its parts where n rows go to the GEMM of ty
     void float_rows(const float *x, const float *norm, int n, int K, int ty, bool ref_order = false);
