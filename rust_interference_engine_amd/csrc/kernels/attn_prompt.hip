@@ -126,6 +126,9 @@ __device__ __forceinline__ half8 as_half8(u32x4 v) { return __builtin_bit_cast(h
 struct __attribute__((packed, aligned(2))) Codes16 {
     uint32_t w[4];
 };
+struct __attribute__((packed, aligned(8))) Part4 {  // of a range partial: rows are hd + 2 floats apart
+    f32x4 v;
+};
 struct __attribute__((packed, aligned(2))) Codes8 {
     uint32_t w[2];
 };
@@ -774,7 +777,7 @@ __global__ __launch_bounds__(256 * NW) void attn_prompt_f16_kernel(AttnArgs a) {
                     f32x4 w4;
 #pragma unroll
                     for (int e = 0; e < 4; e++) w4[e] = o[d][4 * q4 + e] * osc;
-                    *(f32x4 *)(pp + dim0 + 32 * d + 8 * q4 + 4 * h) = w4;
+                    *(Part4 *)(pp + dim0 + 32 * d + 8 * q4 + 4 * h) = Part4{w4};
                 }
             if (h == 0 && (DS == 1 || grp == 0)) {
                 pp[hd] = CARE || m == -INFINITY ? m : m * LN2_F;
