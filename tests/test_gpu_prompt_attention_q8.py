@@ -79,3 +79,27 @@ def test_q8_0_values_past_the_half_range(oracle, cuda):
         v = _rows(g.kv_layer(0, 1, nkv, 96)[0].reshape(nkv, 96, -1), hd)[0]
         assert v[0, pos0:end, 1].max() > 516 and v[0, pos0:end, 0].max() < 1
         _check(oracle, g, spec, hd, nh, nkv, 96, pos0, end - pos0)
+
+
+# heads of 128 and, in two groups, of 256; later batches split their positions over workgroups
+@pytest.mark.parametrize("hd", [128, 256])
+def test_q8_0_values_past_the_half_range_in_splits(oracle, cuda, hd):
+    from gguf_np import GGUF
+    nh, nkv = 4, 2
+    spec = synth.tiny("llama", Q8_0)
+    spec.head_dim, spec.n_head, spec.n_head_kv, spec.rope_dim = hd, nh, nkv, hd
+    img = bytearray(synth.build(spec))
+    for name, start, size in GGUF(bytes(img)).tensor_order:
+        if name == "blk.0.attn_v.weight":
+            rows = np.frombuffer(img, np.uint8, size, start).reshape(nkv * hd, spec.n_embd // 32, 34)
+            d = rows[hd - 64:hd - 32, :, :2].copy().view(np.float16)
+            rows[hd - 64:hd - 32, :, :2] = np.full_like(d, 800).view(np.uint8)
+    g = R.HipBackend(bytes(img), n_ctx=160, max_batch=64, kv_type=R.KvType.Q8_0)
+    g.set_capture(True)
+    toks = [(i * 53 + 11) % spec.n_vocab for i in range(155)]
+    spec.n_layer = 1  # the others see this layer's output through their norms
+    for pos0, end in ((0, 64), (64, 128), (128, 150), (150, 155)):
+        g.forward(toks[pos0:end], pos0)
+        _check(oracle, g, spec, hd, nh, nkv, 160, pos0, end - pos0)
+    v = _rows(g.kv_layer(0, 1, nkv, 160)[0].reshape(nkv, 160, -1), hd)[0]
+    assert v[0, :155, hd // 32 - 2].max() > 516 and v[0, :155, 0].max() < 1

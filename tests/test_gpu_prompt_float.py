@@ -21,7 +21,7 @@ def _compare(g, o, nv, n, tol):
         assert err < tol, f"token {t} of {n}: {err}"
 
 
-# one stage of K, 64- and 128-token tiles with remainders, K splits (ff 2080: uneven stages), GELU
+# three stages of K and more, one to four 64-token tiles with remainders, K splits (ff 2080: uneven stages), GELU
 @pytest.mark.parametrize("arch,ty,ff,n", [("llama", BF16, 96, 9), ("llama", F16, 160, 64), ("qwen3", BF16, 2080, 70),
                                           ("gemma2", BF16, 288, 65), ("gemma2", F16, 2080, 130), ("qwen2", F16, 1056, 200)])
 def test_float_prompts_match_oracle(oracle, cuda, arch, ty, ff, n):

@@ -7,7 +7,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
-from test_gpu_parity import Q4_0, Q5_0, Q5_K, Q6_K, Q8_0, _gemv, _pair, _quant_on_gpu, act_fmt, cuda  # noqa: E402,F401
+from test_gpu_parity import Q4_0, Q4_K, Q5_0, Q5_K, Q6_K, Q8_0, _gemv, _pair, _quant_on_gpu, act_fmt, cuda  # noqa: E402,F401
 
 
 def _check_rows(oracle, cuda, ty, k, rows, n_tok):
@@ -32,12 +32,26 @@ def test_q5_k_gemm_matches_oracle_rows(oracle, cuda, k, rows, n_tok):
     _check_rows(oracle, cuda, Q5_K, k, rows, n_tok)
 
 
-# K of one whole stage, of one and a half, of half a stage, 128-token tiles over an odd
-# number of stages, a K split in uneven parts with half a stage at the end (49 stages)
+# K of one whole stage, of one and a half, of half a stage, 330 tiles' worth of rows and
+# tokens in 64-token tiles over an odd number of half stages, a K split in uneven parts with
+# half a stage at the end (49 stages)
 @pytest.mark.parametrize("ty", [Q4_0, Q5_0, Q8_0])
 @pytest.mark.parametrize("k,rows,n_tok", [(128, 40, 9), (192, 70, 33), (64, 64, 65), (960, 4200, 520), (6208, 96, 70)])
 def test_32_block_gemm_matches_oracle_rows(oracle, cuda, ty, k, rows, n_tok):
     _check_rows(oracle, cuda, ty, k, rows, n_tok)
+
+
+# 128-token tiles with half a stage at the end (520 of them), and in four splits in planes (65 stages)
+@pytest.mark.parametrize("ty", [Q4_0, Q5_0, Q8_0])
+@pytest.mark.parametrize("k,rows,n_tok", [(960, 6600, 520), (8256, 4096, 130)])
+def test_128_token_tiles_match_oracle_rows(oracle, cuda, ty, k, rows, n_tok):
+    _check_rows(oracle, cuda, ty, k, rows, n_tok)
+
+
+# 256 tiles: too many to add their splits up in the launch, so two planes of four superblocks
+@pytest.mark.parametrize("ty", [Q4_K, Q5_K, Q6_K])
+def test_k_quant_splits_in_planes_match_oracle_rows(oracle, cuda, ty):
+    _check_rows(oracle, cuda, ty, 2048, 4096, 200)
 
 
 @pytest.mark.parametrize("arch,ty", [("llama", Q5_K), ("gemma2", Q5_K), ("gemma2", Q6_K), ("qwen3moe", Q5_K), ("qwen3moe", Q6_K),
@@ -54,8 +68,9 @@ def test_gated_and_grouped_k_quant_prompts_match_oracle(oracle, cuda, arch, ty):
         assert err < 0.03, f"{arch} {ty}: token {t}: {err}"
 
 
-# hidden 1024 (8 stages of 128, 4 superblocks): every launch of these prompts splits K and
-# adds its partial sums up in the launch, layer after layer on the same counters
+# hidden 1024 (8 stages of 128, 4 superblocks): every launch of these prompts but the attention
+# output's (K 256) splits K and adds its partial sums up in the launch, layer after layer on
+# the same counters
 @pytest.mark.parametrize("arch,ty", [("llama", Q4_0), ("gemma2", Q8_0), ("qwen3", Q5_0), ("llama", Q5_K), ("gemma2", Q6_K)])
 def test_prompts_with_k_splits_match_oracle(oracle, cuda, arch, ty):
     from naive_model import max_rel_err
