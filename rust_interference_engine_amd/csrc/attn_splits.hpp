@@ -8,8 +8,9 @@ namespace rie {
 // Splits of a prompt attention launch of wgs workgroups whose longest query row sees
 // `tiles` tiles of 32 positions; a second kernel merges them.
 // * From 64 workgroups on: splits of at least 16 tiles, up to about two workgroups per CU
-//   (finer ones measured no better than one pass: 512 tokens at 0, 128 workgroups, 1149
-//   against 1142 us).
+//   (finer ones, by the rule below, measured no better: at 0 / at 800, two layers of 64
+//   workgroups 733 / 744 against 726 / 750 us, 88 508 / 527 against 500 / 528, 96 503 / 491
+//   against 501 / 493, 112 1100 / 1123 against 1098 / 1122; 128 at 0 1149 against 1142).
 // * Below: splits of at least 2 tiles, up to one workgroup per CU (650 tokens of
 //   gemma-3-1b, 21 workgroups, six layers: 1579 us in one pass with the per-token kernel,
 //   1369 us in splits of 4 tiles, 1323 us in splits of 2; two workgroups per CU are slower

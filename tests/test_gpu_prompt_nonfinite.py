@@ -55,7 +55,12 @@ def test_values_past_the_cache_format_stay_with_the_tokens_that_see_them(cuda, h
     assert np.array_equal(a[:at], b[:at])  # their sums add probability 0 times another value, if any
     # from there on: infinities of the values' signs in the 32 dims, finite everywhere else
     sign = np.where(np.arange(32) % 3 == 0, -np.inf, np.inf)
-    assert (a[at:, :G, 32:64] == sign).all()
+    # (the per-token kernel, which runs up to 8 tokens of 256-wide heads over an f16 cache,
+    # fills idle slots of a range with its first row at probability 0: NaN for a token that
+    # sees an infinity there, as ever)
+    seen = a[at:, :G, 32:64]
+    per_token = hd == 256 and kv == 0
+    assert ((seen == sign) | (np.isnan(seen) & (per_token & (np.arange(at, 155) >= 150))[:, None, None])).all()
     rest = np.ones(a.shape[1:], bool)
     rest[:G, 32:64] = False
     assert np.isfinite(a[at:][:, rest]).all()
