@@ -955,10 +955,14 @@ __global__ __launch_bounds__(64) void turbo_query_kernel(const float *__restrict
 bool attention_prompt_mfma_ok(const AttnArgs &a) {
     const int G = a.n_kv > 0 ? a.n_head / a.n_kv : 0;
     const bool cache_ok = a.kv_type == 0 || a.kv_type == 1 || (a.kv_type == 2 && a.hd == 128 && a.turbo_signs && a.k_scale && a.v_scale && a.part);
-    // heads of 256 over f16 caches: up to 8 tokens in the per-token kernel (gemma-3-1b, 2 / 8
-    // tokens at 12000, six layers: 473 / 610 us there, 534 / 660 us here; 12 tokens 1067
-    // against 767 us)
-    if (a.hd == 256 && a.kv_type == 0 && a.n_tok <= 8) return false;
+    // Few rows past 96 positions (where this kernel takes splits) in the per-token kernel:
+    // heads of 256 over f16 caches up to 8 tokens (gemma-3-1b, per-token / here, 8 tokens at
+    // 30 559 / 544 us, at 200 560 / 582, at 3000 566 / 587, at 12000 592 / 660; 12 tokens at
+    // 12000 1067 / 767), and Q8_0 caches up to 4 rows per KV head (two layers of hidden 2048,
+    // 2 tokens, 2 heads per KV head, at 20 133 / 128 us, at 1000 134 / 141, at 12000 161 / 178;
+    // 8 rows at 12000 290 / 281)
+    const bool few = a.kv_type == 0 ? a.hd == 256 && a.n_tok <= 8 : a.kv_type == 1 && a.n_tok * G <= 4;
+    if (few && a.pos0 + a.n_tok > 96) return false;
     return cache_ok && a.n_tok > 1 && !a.d_pos0 && a.slots >= 32 && (a.hd == 32 || a.hd == 64 || a.hd == 96 || a.hd == 128 || (a.hd == 256 && a.kv_type != 2)) && G >= 1 &&
            G <= 8 && a.n_head == G * a.n_kv && (a.att_fmt != ACT_Q8_0 || (a.att_q.qs && a.att_q.d));
 }

@@ -52,3 +52,11 @@ def attention_error(oracle, hd, nh, nkv, kv, batches):
 def test_prompt_attention_error_is_that_of_f32(oracle, cuda, hd, nh, nkv, kv):
     err = attention_error(oracle, hd, nh, nkv, kv, [(0, 200), (200, 400), (400, 600), (600, 605)])
     assert err <= 1.5 * 2.0 ** -24, err
+
+
+# up to 8 tokens (f16, heads of 256) and 4 rows per KV head (Q8_0) run in the per-token kernel
+# from 97 positions on
+@pytest.mark.parametrize("hd,nh,nkv,kv", [(256, 4, 1, 0), (128, 4, 2, 1), (256, 2, 2, 1)])
+def test_few_rows_on_either_side_of_the_kernels_line(oracle, cuda, hd, nh, nkv, kv):
+    batches = [(0, 80), (80, 88), (88, 94), (94, 96), (96, 98), (98, 102), (102, 110), (110, 119)]
+    assert attention_error(oracle, hd, nh, nkv, kv, batches) <= 1.5 * 2.0 ** -24
